@@ -73,7 +73,7 @@ def listed():
         dict(_case("gradient", "100vertebrates", regions=60, lo=100, hi=1500, gap=0.15, rho=True),
              name="branch_gradients_fp64m"),
         # the omega (dN/dS) test of a gene family's regions
-        dict(_case("score", "58mammals", regions=60, lo=50, hi=500, strategy="omega"), name="omega_fp64m"),
+        dict(_case("score", "58mammals", regions=40, lo=150, hi=600, strategy="omega"), name="omega_fp64m"),
         # one E-step of an ECM re-estimation
         dict(_case("counts", "58mammals", regions=120, lo=50, hi=2000), name="estep_codons"),
         # a nucleotide model through PhyloLik (the library's other alphabet), every alignment column
@@ -104,8 +104,8 @@ def draw(rng: random.Random):
         return _case("score", rng.choice(trees), regions=_log_int(rng, 1, 100), lo=lo, hi=hi, gap=gap,
                      strategy="mle_grad", precision=FP16S, rho=rng.random() < 0.5)
     if kind == "omega":
-        return _case("score", rng.choice(["12flies", "29mammals", "58mammals"]), regions=_log_int(rng, 1, 50),
-                     lo=50, hi=50 + _log_int(rng, 1, 450), strategy="omega", gap=gap)
+        return _case("score", rng.choice(["12flies", "29mammals", "58mammals"]), regions=_log_int(rng, 1, 40),
+                     lo=150, hi=150 + _log_int(rng, 1, 450), strategy="omega", gap=gap)
     if kind == "forward":
         return _case("forward", rng.choice(trees), regions=_log_int(rng, 1, 1500), lo=lo, hi=hi, gap=gap,
                      precision=rng.choice([FP32, FP16S, FP16S, FP64M]))
