@@ -364,7 +364,6 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
       any = any || act[k];
     }
     if (!any) continue;
-    RegionChunk ch;
     ch.r0 = r0;
     ch.nreg = nr;
     ch.block0 = b->al.block0[r0];
@@ -385,9 +384,14 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
         b->setqs_cap = 0;
         b->eig_ref_ok.clear();
         HIP_TRY(c, dalloc(&b->d_setqs, (size_t)b->rs.cap * 12));
+    RegionChunk ch;
         HIP_TRY(c, dalloc(&b->d_eigmode, (size_t)b->rs.cap));
         HIP_TRY(c, dalloc(&b->d_eigref, (size_t)b->rs.cap * 4096));
         b->setqs_cap = (size_t)b->rs.cap * 12;
+      if (act[k]) {
+        const size_t r = r0 + k / nm;
+        ch.work += (b->offsets[r + 1] - b->offsets[r] + kAlignCols - 1) / kAlignCols;
+      }
       }
       // per set: keep (inactive, or settings as last built), warm (the
       // reference basis has the same pi: only kappa / omega differ), or cold

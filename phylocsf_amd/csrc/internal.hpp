@@ -196,6 +196,8 @@ struct RegionChunk {
   const PSets* sets = nullptr;      // set (r - r0) * nm + q; set q when `sets` is the
                                     // model's own (fixed) sets, shared by every region
 };
+  int64_t work = 0;                 // 64-column blocks of active sets (0: every block of
+                                    // every model)
 
 // ---- kernel launchers (kernels/*.hip) --------------------------------------
 // bad (may be null) gets a nonzero value if a code is neither a codon index
@@ -211,9 +213,10 @@ constexpr unsigned kBuildP64 = 1, kBuildMfma = 2, kBuildTangent = 4, kBuildP64M 
 // Doubles per branch of PSets::d_P64F.  Internal branch: P[a][b] at
 // ((a / 16) * 16 + b / 4) * 64 + a % 16 + 16 (b % 4) (the A-fragment order of
 // fp64_tiles.hpp).  Leaf branch: 65 messages of 64 entries, message c < 64
-// the column P[.][c] and message 64 all ones (`Marginalize), each stored so
-// that lane group g's 16 rows are contiguous: row 16 mo + 4 v + g at
-// c * 64 + 16 g + 4 mo + v.
+// the column P[.][c] and message 64 all ones (`Marginalize), row 16 mo + 4 v +
+// g at c * 64 + 16 mo + 4 g + v: the four lane groups' rows of one 16-row
+// block share a 128-byte line, so a wave's load of 16 columns looks up 16
+// lines (64 with each group's 16 rows contiguous).
 constexpr int kTile64 = 65 * 64;
 hipError_t launch_pbuild(const pcsf_model* m, const PSets& sets, int nsets, int fmt,
                          unsigned outputs, hipStream_t s);

@@ -35,16 +35,16 @@ using namespace fp64t;
 
 // the message of leaf branch `br` for `code`: column `code` of P, or ones
 // for `Marginalize (message 64), from the branch's leaf messages in P64F
-// (row 16 mo + 4 v + g at code * 64 + 16 g + 4 mo + v)
+// (row 16 mo + 4 v + g at code * 64 + 16 mo + 4 g + v)
 __device__ __forceinline__ Tile leaf_message(const double* __restrict__ PF, int code, int grp) {
   const int c = (code == PCSF_MARGINALIZE) ? 64 : code;
-  const double2* src = reinterpret_cast<const double2*>(PF + c * 64 + 16 * grp);
+  const double2* src = reinterpret_cast<const double2*>(PF + c * 64 + 4 * grp);
   Tile t;
 #pragma unroll
   for (int mo = 0; mo < 4; ++mo)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const double2 d = src[2 * mo + h];
+      const double2 d = src[8 * mo + h];
       t.r[mo][2 * h] = d.x;
       t.r[mo][2 * h + 1] = d.y;
     }

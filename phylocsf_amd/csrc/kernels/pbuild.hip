@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256, WITH_D ? 2 : 3) void pbuild_kernel(
         for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            out[(16 * w + 4 * r + lk) * 64 + 16 * (lr & 3) + 4 * ct + (lr >> 2)] = acc[ct][r];
+            out[(16 * w + 4 * r + lk) * 64 + 16 * ct + 4 * (lr & 3) + (lr >> 2)] = acc[ct][r];
         if (tid < 64) out[4096 + tid] = 1.0;
       } else {
 #pragma unroll

@@ -1,9 +1,8 @@
-// prune_fp64m.hip -- launcher of the FP64 forward on matrix cores
-// (prune_fp64m.hpp): the tree's generated program when it has one, the
-// op-program interpreter otherwise.
+// prune_fp64m.hip -- launcher of the FP64 forward on matrix cores: the
+// tree's generated program (prune_fp64m.hpp) where it has one and the columns
+// fill the device, the row-split kernel (prune_fp64r.hip) otherwise.
 #include "prune_tree.hpp"
 
-using pcsf_mfma::Interp;
 using pcsf_mfma::MfmaParams;
 
 hipError_t launch_forward_fp64m(const pcsf_model* m, const pcsf_batch* b, const RegionChunk& ch,
@@ -29,20 +28,18 @@ hipError_t launch_forward_fp64m(const pcsf_model* m, const pcsf_batch* b, const 
   prm.r0 = ch.r0;
   prm.shared_sets = ch.sets == &m->fixed ? 1 : 0;
   prm.P64F = ch.sets->d_P64F;
+  prm.astart = b->al.d_astart;
+  prm.off = b->d_offsets;
   if (prm.ngroups == 0) return hipSuccess;
   const int cus = m->ctx->num_cus;
-  if (m->specialized && m->tree_p) {
+  // 64-column blocks of work.  Up to four per CU the row-split kernel is the
+  // faster one (58mammals: 251 against 285 us at 366 blocks, 529 against 556
+  // at 772), above it the generated program, which reads P once per 64
+  // columns (898 against 850 us at 1520 blocks, 3619 against 3207 at 6214).
+  const int64_t blocks = ch.work > 0 ? ch.work : ch.nblocks * m->nm;
+  if (m->specialized && m->tree_p && blocks > 4 * (int64_t)cus) {
     const auto* t = static_cast<const pcsf_mfma::TreeProgram*>(m->tree_p);
     if (t->fp64m) return t->fp64m(prm, 0, 0, cus, s);
   }
-  using pcsf_mfma::f64m::launch_ns;
-  switch (m->slots) {
-    case 1:
-    case 2: return launch_ns<2, Interp<2>>(prm, cus, s);
-    case 3: return launch_ns<3, Interp<3>>(prm, cus, s);
-    case 4: return launch_ns<4, Interp<4>, 1>(prm, cus, s);
-    case 5: return launch_ns<5, Interp<5>, 1>(prm, cus, s);
-    case 6: return launch_ns<6, Interp<6>, 1>(prm, cus, s);
-    default: return hipErrorInvalidValue;
-  }
+  return launch_fp64_rows(prm, blocks, m->slots, (int)(m->prog.size() / kOpWords / 2), cus, s);
 }

@@ -1,6 +1,6 @@
 // prune_fp64m.hpp -- the FP64 forward on matrix cores (precision
-// PCSF_FP64M), driven by an op program: the interpreter (prune_fp64m.hip) or
-// a tree's straight-line program (generated per shipped tree).
+// PCSF_FP64M), driven by a tree's straight-line op program (generated per
+// shipped tree); prune_fp64r.hip takes the other trees and the small calls.
 //
 // Same result as PhyloLik.ensure_alpha and the root posterior
 // (lib/CamlPaml/PhyloLik.ml:73-93,127-138), per column ln z and the root's
@@ -16,8 +16,8 @@
 // tile's loads straight from memory into the idle buffer (the sets' P64F
 // holds P in the MFMA's A-fragment order, so the copy is a plain one), and
 // the barrier opening the next product is the only wait.  Leaf messages are
-// the columns of P (the leaf-branch layout of P64F keeps each lane group's
-// 16 rows of a column contiguous), all ones for `Marginalize.  Paths are
+// the columns of P (in the leaf-branch layout of P64F the four lanes of a
+// column read one 128-byte line per 16 rows), all ones for `Marginalize.  Paths are
 // relative to the mlin/PhyloCSF tree.
 #pragma once
 #include "fp64_tiles.hpp"
@@ -63,13 +63,13 @@ struct Walk64 {
     constexpr uint32_t kBranchBytes = kTile64 * 8;
     const Rsrc r = make_rsrc(p.P64F + (size_t)oset() * p.nbr * kTile64,
                                         p.nbr * kBranchBytes);
-    const uint32_t off = c * 512u + (uint32_t)grp * 128u;
+    const uint32_t off = c * 512u + (uint32_t)grp * 32u;
     Tile64 t;
 #pragma unroll
     for (int mo = 0; mo < 4; ++mo)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, off + 32u * mo + 16u * h,
+        const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, off + 128u * mo + 16u * h,
                                                              leaf * kBranchBytes, 0);
         const double2 d = __builtin_bit_cast(double2, x);
         t.r[mo][2 * h] = d.x;
@@ -147,11 +147,10 @@ struct Walk64 {
   }
 };
 
-// MINB workgroups per CU: two (a generated program keeps only its live
-// tiles in registers), one for the interpreter above three live tiles (it
-// keeps every slot live through its dispatch; at two per CU it spills)
-template <int NS, class PROG, int MINB>
-__global__ __launch_bounds__(kNT, MINB) void prune_fp64m_kernel(MfmaParams p) {
+// two workgroups per CU: a generated program keeps only its live tiles in
+// registers
+template <int NS, class PROG>
+__global__ __launch_bounds__(kNT, 2) void prune_fp64m_kernel(MfmaParams p) {
   __shared__ __attribute__((aligned(16))) double Pbuf[2][4096];
   extern __shared__ __attribute__((aligned(16))) uint8_t codes_s[];  // nl x kGC
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -203,9 +202,9 @@ __global__ __launch_bounds__(kNT, MINB) void prune_fp64m_kernel(MfmaParams p) {
   }
 }
 
-template <int NS, class PROG, int MINB = 2>
+template <int NS, class PROG>
 hipError_t launch_ns(const MfmaParams& prm, int cus, hipStream_t s) {
-  auto kern = prune_fp64m_kernel<NS, PROG, MINB>;
+  auto kern = prune_fp64m_kernel<NS, PROG>;
   const size_t dyn = ((size_t)prm.nl * kGC + 15) / 16 * 16;
   int per_cu = 0;
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kNT, dyn);

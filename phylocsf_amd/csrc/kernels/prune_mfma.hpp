@@ -107,8 +107,21 @@ struct MfmaParams {
   // the FP64 matrix-core forward only: P of the sets (PSets::d_P64F)
   const double* P64F;
 };
+  const int64_t* astart;
+  const int64_t* off;
 
 struct Task {
+}  // namespace pcsf_mfma
+
+// The FP64 forward with rows split over waves (prune_fp64r.hip): p's groups
+// are 64-column blocks, `blocks` of them (over all models) have work; the
+// program has `nsteps` pairs of ops, each a node's last op and the product
+// above it.
+hipError_t launch_fp64_rows(const pcsf_mfma::MfmaParams& p, int64_t blocks, int slots, int nsteps,
+                            int cus, hipStream_t s);
+
+namespace pcsf_mfma {
+
   int q;       // model
   int set;     // transition-matrix set
   int64_t g;   // group within the launch
