@@ -60,6 +60,11 @@ bool known_precision(int p) { return p >= PCSF_FP64 && p <= PCSF_FP64M; }
 // FP64 arithmetic throughout (plain or on matrix cores)
 bool fp64_precision(int p) { return p == PCSF_FP64 || p == PCSF_FP64M; }
 
+// What a forward at `precision` reads of its transition sets.
+unsigned set_outputs(int precision) {
+  return precision == PCSF_FP64M ? kBuildP64M : precision == PCSF_FP64 ? kBuildP64 : kBuildMfma;
+}
+
 constexpr const char* kTreeOnly =
     "a tree-only model (made with n_models = 0) serves the omega test only";
 
@@ -199,24 +204,45 @@ int run_pbuild(pcsf_model* m, PSets& ps, int nsets, const double* rho_host, int 
   return PCSF_OK;
 }
 
-// Transition sets and cherry tables of the fixed scales rho[0 .. nm) (one
-// per model) with P tiles in format fmt; rebuilt only when either changes.
-// Allocates nothing: the sets are the model's own and cached_rho's capacity
-// is reserved when the model is made.
-int ensure_transitions(pcsf_model* m, const double* rho, int fmt, float* ms_out) {
+// Transition sets of the fixed scales rho[0 .. nm) (one per model) holding
+// `need` (kBuild* outputs), P tiles in format fmt, and the cherry tables where
+// the MFMA kernels will read them; what the model already holds at these
+// scales is kept, only what is missing is built (a maximiser at FP64M moves
+// its scales on every call and reads neither tiles nor tables).  Allocates
+// nothing: the sets are the model's own and cached_rho's capacity is reserved
+// when the model is made.
+int ensure_transitions(pcsf_model* m, const double* rho, int fmt, unsigned need, float* ms_out) {
   pcsf_ctx* c = m->ctx;
   if (ms_out) *ms_out = 0.f;
   const bool same_rho = (int)m->cached_rho.size() == m->nm &&
                         std::equal(rho, rho + m->nm, m->cached_rho.begin());
-  if (same_rho && m->fixed.fmt == fmt) return PCSF_OK;
-  m->cached_rho.clear();
-  HIP_TRY(c, hipMemcpyAsync(m->fixed.d_rho, rho, sizeof(double) * m->nm, hipMemcpyHostToDevice,
-                            c->stream));
-  HIP_TRY(c, hipMemsetAsync(m->fixed.d_active, 1, (size_t)m->nm, c->stream));
-  int rc = run_pbuild(m, m->fixed, m->nm, rho, fmt, ms_out);
-  if (rc) return rc;
-  if (!same_rho) HIP_TRY(c, launch_cherry_tables(m, m->fixed, m->nm, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (!same_rho) {
+    m->cached_rho.clear();
+    m->built = 0;
+    m->tables = false;
+    HIP_TRY(c, hipMemcpyAsync(m->fixed.d_rho, rho, sizeof(double) * m->nm,
+                              hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, hipMemsetAsync(m->fixed.d_active, 1, (size_t)m->nm, c->stream));
+  }
+  if ((m->built & kBuildMfma) && m->fixed.fmt != fmt) m->built &= ~kBuildMfma;
+  const bool tables = (need & kBuildMfma) && !m->cherries.empty() && !m->tables;
+  if (tables) need |= kBuildP64M;  // the tables are products of the FP64 matrices
+  const unsigned missing = need & ~m->built;
+  if (missing) {
+    const int had_fmt = (m->built & kBuildMfma) ? m->fixed.fmt : -1;
+    int rc = run_pbuild(m, m->fixed, m->nm, rho, fmt, ms_out, missing);
+    if (rc) {
+      m->cached_rho.clear();
+      m->built = 0;
+      return rc;
+    }
+    if (!(missing & kBuildMfma)) m->fixed.fmt = had_fmt;
+    m->built |= missing;
+  }
+  if (tables) {
+    HIP_TRY(c, launch_cherry_tables(m, m->fixed, m->nm, c->stream));
+    m->tables = true;
+  }
   m->cached_rho.assign(rho, rho + m->nm);
   return PCSF_OK;
 }
@@ -359,9 +385,14 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
     const int32_t nr = std::min<int32_t>(chunk_regions, b->nreg - r0);
     act.assign((size_t)nr * nm, 1);
     bool any = false;
+    RegionChunk ch;
     for (size_t k = 0; k < act.size(); ++k) {
       if (active) act[k] = active[(size_t)r0 * nm + k] ? 1 : 0;
       any = any || act[k];
+      if (act[k]) {
+        const size_t r = r0 + k / nm;
+        ch.work += (b->offsets[r + 1] - b->offsets[r] + kAlignCols - 1) / kAlignCols;
+      }
     }
     if (!any) continue;
     ch.r0 = r0;
@@ -384,14 +415,9 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
         b->setqs_cap = 0;
         b->eig_ref_ok.clear();
         HIP_TRY(c, dalloc(&b->d_setqs, (size_t)b->rs.cap * 12));
-    RegionChunk ch;
         HIP_TRY(c, dalloc(&b->d_eigmode, (size_t)b->rs.cap));
         HIP_TRY(c, dalloc(&b->d_eigref, (size_t)b->rs.cap * 4096));
         b->setqs_cap = (size_t)b->rs.cap * 12;
-      if (act[k]) {
-        const size_t r = r0 + k / nm;
-        ch.work += (b->offsets[r + 1] - b->offsets[r] + kAlignCols - 1) / kAlignCols;
-      }
       }
       // per set: keep (inactive, or settings as last built), warm (the
       // reference basis has the same pi: only kappa / omega differ), or cold
@@ -446,7 +472,7 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
     }
     float tp = 0.f;
     rc = run_pbuild(m, b->rs, nr * nm, rho + (size_t)r0 * nm, fmt, &tp,
-                    precision == PCSF_FP64M ? kBuildP64M : fp64 ? kBuildP64 : kBuildMfma);
+                    set_outputs(precision));
     if (rc) {
       char buf[64];
       std::snprintf(buf, sizeof buf, " (region block from %d)", r0);
@@ -936,7 +962,7 @@ int pcsf_model_transition(pcsf_model* m, int model, double rho, double* P_out) {
   if (!rho_valid(rho))
     return set_err(c, PCSF_EINVAL, "CamlPaml.P14n.instantiate_tree: domain violation on variable 0");
   std::vector<double> r(m->nm, rho);
-  int rc = ensure_transitions(m, r.data(), m->fixed.fmt < 0 ? kFragF32 : m->fixed.fmt, nullptr);
+  int rc = ensure_transitions(m, r.data(), kFragF32, kBuildP64, nullptr);
   if (rc) return rc;
   std::vector<double> T((size_t)m->nbr * 4096);
   HIP_TRY(c, hipMemcpy(T.data(), m->fixed.d_P64T + (size_t)model * m->nbr * 4096, T.size() * 8,
@@ -1151,9 +1177,7 @@ int pcsf_forward(pcsf_batch* b, const double* rho, int rho_per_region, int preci
                      "CamlPaml.P14n.instantiate_tree: domain violation on variable 0");
   HIP_TRY(c, hipSetDevice(c->device));
   float tp = 0.f;
-  const int fmt = fp64_precision(precision) ? (m->fixed.fmt < 0 ? kFragF32 : m->fixed.fmt)
-                                            : frag_format(precision);
-  int rc = ensure_transitions(m, r.data(), fmt, &tp);
+  int rc = ensure_transitions(m, r.data(), frag_format(precision), set_outputs(precision), &tp);
   if (rc) return rc;
   if (precision == PCSF_FP64M && b->nreg > 0) {
     // region-aligned columns, the model's sets for every region
@@ -1257,9 +1281,7 @@ int pcsf_forward_noalloc(pcsf_model* m, const uint8_t* d_codes, int64_t n_cols,
                    std::string("pcsf_forward_noalloc: scratch lookup failed: ") +
                        hipGetErrorString(se));
   // transition sets at these scales: the model's own (allocated when it was made)
-  const int fmt = precision == PCSF_FP64 ? (m->fixed.fmt < 0 ? kFragF32 : m->fixed.fmt)
-                                         : frag_format(precision);
-  int rc = ensure_transitions(m, rho, fmt, nullptr);
+  int rc = ensure_transitions(m, rho, frag_format(precision), set_outputs(precision), nullptr);
   if (rc) return rc;
   // a view of the scratch as a batch (owns nothing; its vectors stay empty)
   pcsf_batch v;
@@ -1315,7 +1337,7 @@ int pcsf_autotune(pcsf_batch* b, int precision, int reps, double* ms_out, int* c
   HIP_TRY(c, hipSetDevice(c->device));
   {
     std::vector<double> one(m->nm, 1.0);
-    int rc = ensure_transitions(m, one.data(), frag_format(precision), nullptr);
+    int rc = ensure_transitions(m, one.data(), frag_format(precision), kBuildMfma, nullptr);
     if (rc) return rc;
   }
   hipEvent_t e0, e1;

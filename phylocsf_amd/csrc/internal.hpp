@@ -133,7 +133,8 @@ struct pcsf_model {
   int n_lsl = 0, n_lsl_t = 0;
   // device: transition matrices at the cached tree scales (set q = model q)
   std::vector<double> cached_rho;
-  int cached_fmt = -1;
+  unsigned built = 0;   // kBuild* outputs `fixed` holds at cached_rho
+  bool tables = false;  // and whether its cherry tables do
   PSets fixed;
   // failure record of the P builder: the minimum packed (set, branch, row,
   // column, check) key over failing rows, all ones when none failed
@@ -195,9 +196,9 @@ struct RegionChunk {
   int64_t block0 = 0, nblocks = 0;  // aligned blocks covering them
   const PSets* sets = nullptr;      // set (r - r0) * nm + q; set q when `sets` is the
                                     // model's own (fixed) sets, shared by every region
-};
   int64_t work = 0;                 // 64-column blocks of active sets (0: every block of
                                     // every model)
+};
 
 // ---- kernel launchers (kernels/*.hip) --------------------------------------
 // bad (may be null) gets a nonzero value if a code is neither a codon index

@@ -37,7 +37,9 @@
 //   DT32, Dfrag  (tangent sets only) D = dP(rho b)/drho = b Q P in the layouts
 //         of PT32 (divided by P[c][c]; row 64 zero) and of the FP32 tile
 //         (dense), for leaf and internal branches respectively.
-#include "../internal.hpp"
+#include <algorithm>
+
+#include "fp64_tiles.hpp"
 
 namespace {
 
@@ -366,35 +368,65 @@ __global__ __launch_bounds__(256, WITH_D ? 2 : 3) void pbuild_kernel(
 // Cherry tables: for cherry c with leaves a, b (branches into them from c),
 // T[x][y] = P_c (P_a[:, x] o P_b[:, y]) for codons x, y or `Marginalize (64,
 // the all-ones leaf vector), in FP64, stored normalised to max 1 (FP32) with
-// its ln max (FP64).  One 64-thread workgroup per (x, y) and (set, table).
-__global__ __launch_bounds__(64) void cherry_table_kernel(const double* __restrict__ P64T,
-                                                         const int32_t* __restrict__ cher,
-                                                         int nctab, int nbr,
-                                                         float* __restrict__ ctab,
-                                                         double* __restrict__ clnt) {
-  __shared__ double al[64];
-  __shared__ double mx[64];
-  const int xy = blockIdx.x, x = xy / kTabCodes, y = xy % kTabCodes;
-  const int st = blockIdx.y, set = st / nctab, t = st % nctab, k = threadIdx.x;
+// its ln max (FP64).  The 65 x 65 pairs of a table are the columns of one
+// 64 x 64 by 64 x 4225 product on v_mfma_f64_16x16x4f64: a wave takes 16
+// pairs at a time as a tile of fp64_tiles.hpp (the two leaf messages
+// multiplied), P_c sits in LDS for the workgroup's four waves.
+constexpr int kPairTiles = (kTabCodes * kTabCodes + 15) / 16;  // tiles of 16 pairs per table
+
+__device__ __forceinline__ fp64t::Tile leaf_tile64(const double* __restrict__ PL, int c, int g) {
+  // row 16 mo + 4 v + g of message c at c * 64 + 16 mo + 4 g + v (kTile64)
+  const double2* src = reinterpret_cast<const double2*>(PL + c * 64 + 4 * g);
+  fp64t::Tile t;
+#pragma unroll
+  for (int mo = 0; mo < 4; ++mo)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const double2 d = src[8 * mo + h];
+      t.r[mo][2 * h] = d.x;
+      t.r[mo][2 * h + 1] = d.y;
+    }
+  return t;
+}
+
+__global__ __launch_bounds__(256, 2) void cherry_table_kernel(const double* __restrict__ P64F,
+                                                          const int32_t* __restrict__ cher,
+                                                          int nctab, int nbr,
+                                                          float* __restrict__ ctab,
+                                                          double* __restrict__ clnt) {
+  __shared__ __attribute__((aligned(16))) double Pc[4096];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int j = lane & 15, g = lane >> 4;
+  const int st = blockIdx.y, set = st / nctab, t = st % nctab;
   const int c = cher[3 * t], a = cher[3 * t + 1], b = cher[3 * t + 2];
-  const double* Pa = P64T + ((size_t)set * nbr + a) * 4096;  // Pa[col * 64 + row]
-  const double* Pb = P64T + ((size_t)set * nbr + b) * 4096;
-  const double* Pc = P64T + ((size_t)set * nbr + c) * 4096;
-  al[k] = (x == 64 ? 1.0 : Pa[x * 64 + k]) * (y == 64 ? 1.0 : Pb[y * 64 + k]);
+  const double* base = P64F + (size_t)set * nbr * kTile64;
+  fp64t::copy_tile((fp64t::L3*)&Pc[0], base + (size_t)c * kTile64, wave, tid);
   __syncthreads();
-  double m = 0.0;
-  for (int j = 0; j < 64; ++j) m = fma(Pc[j * 64 + k], al[j], m);  // row k of P_c al
-  mx[k] = m;
-  __syncthreads();
-  for (int w = 32; w > 0; w >>= 1) {
-    if (k < w) mx[k] = fmax(mx[k], mx[k + w]);
-    __syncthreads();
+  for (int u = blockIdx.x * 4 + wave; u < kPairTiles; u += gridDim.x * 4) {
+    const int pair = min(16 * u + j, kTabCodes * kTabCodes - 1);
+    const int x = pair / kTabCodes, y = pair - x * kTabCodes;
+    fp64t::Tile al = leaf_tile64(base + (size_t)a * kTile64, x, g);
+    const fp64t::Tile bl = leaf_tile64(base + (size_t)b * kTile64, y, g);
+#pragma unroll
+    for (int mo = 0; mo < 4; ++mo) al.r[mo] *= bl.r[mo];
+    const fp64t::Tile m = fp64t::gemm(Pc, al, lane);
+    double top = 0.0;
+#pragma unroll
+    for (int mo = 0; mo < 4; ++mo)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) top = fmax(top, m.r[mo][v]);
+    top = fmax(top, __shfl_xor(top, 16));
+    top = fmax(top, __shfl_xor(top, 32));
+    if (16 * u + j >= kTabCodes * kTabCodes) continue;
+    const size_t e = (size_t)st * kTabCodes * kTabCodes + pair;
+    const bool ones = (x == 64 && y == 64);  // P 1 = 1 exactly
+#pragma unroll
+    for (int mo = 0; mo < 4; ++mo)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        ctab[e * 64 + 16 * mo + 4 * v + g] = ones ? 1.0f : (float)(m.r[mo][v] / top);
+    if (g == 0) clnt[e] = ones ? 0.0 : log(top);
   }
-  const double top = mx[0];
-  const size_t base = ((size_t)st * kTabCodes * kTabCodes + xy);
-  const bool ones = (x == 64 && y == 64);  // P 1 = 1 exactly
-  ctab[base * 64 + k] = ones ? 1.0f : (float)(m / top);
-  if (k == 0) clnt[base] = ones ? 0.0 : log(top);
 }
 
 }  // namespace
@@ -403,8 +435,12 @@ hipError_t launch_cherry_tables(const pcsf_model* m, const PSets& sets, int nset
                                 hipStream_t s) {
   const int nct = (int)m->cherries.size() / 3;
   if (nct == 0 || nsets == 0) return hipSuccess;
-  dim3 grid(kTabCodes * kTabCodes, nsets * nct);
-  hipLaunchKernelGGL(cherry_table_kernel, grid, dim3(64), 0, s, sets.d_P64T, m->d_cherries, nct,
+  // four tiles per wave, so that P_c in LDS serves 16 of them, and fewer where
+  // a small tree's few tables would leave compute units idle
+  const int per_table = (kPairTiles + 3) / 4;
+  const int want = (4 * m->ctx->num_cus + nsets * nct - 1) / (nsets * nct);
+  dim3 grid(std::min(per_table, std::max(want, (per_table + 3) / 4)), nsets * nct);
+  hipLaunchKernelGGL(cherry_table_kernel, grid, dim3(256), 0, s, sets.d_P64F, m->d_cherries, nct,
                      m->nbr, sets.d_ctab, sets.d_clnt);
   return hipGetLastError();
 }
