@@ -104,13 +104,13 @@ struct MfmaParams {
   int prior_per_set;
   // region mode over the model's own sets (set q in every region)
   int shared_sets;
-  // the FP64 matrix-core forward only: P of the sets (PSets::d_P64F)
+  // the FP64 matrix-core forward only: P of the sets (PSets::d_P64F), and the
+  // regions' first aligned columns and packed offsets
   const double* P64F;
-};
   const int64_t* astart;
   const int64_t* off;
+};
 
-struct Task {
 }  // namespace pcsf_mfma
 
 // The FP64 forward with rows split over waves (prune_fp64r.hip): p's groups
@@ -122,6 +122,7 @@ hipError_t launch_fp64_rows(const pcsf_mfma::MfmaParams& p, int64_t blocks, int 
 
 namespace pcsf_mfma {
 
+struct Task {
   int q;       // model
   int set;     // transition-matrix set
   int64_t g;   // group within the launch
@@ -654,16 +655,18 @@ template <int NS>
 struct Interp {
   template <class W, class T, class M>
   __device__ __forceinline__ static void run(W& w, T (&S)[NS], M (&K)[NS]) {
-    const int32_t* prog = w.p.prog;
+    const int4* prog = reinterpret_cast<const int4*>(w.p.prog);
+    int4 next = prog[0];
     for (int pc = 0;; ++pc) {
-      const int w0 = __builtin_amdgcn_readfirstlane(prog[4 * pc]);
-      const int w1 = __builtin_amdgcn_readfirstlane(prog[4 * pc + 1]);
-      const int w2 = __builtin_amdgcn_readfirstlane(prog[4 * pc + 2]);
-      const uint32_t w3 = __builtin_amdgcn_readfirstlane(prog[4 * pc + 3]);
+      const int w0 = __builtin_amdgcn_readfirstlane(next.x);
+      const int w1 = __builtin_amdgcn_readfirstlane(next.y);
+      const int w2 = __builtin_amdgcn_readfirstlane(next.z);
+      const uint32_t w3 = __builtin_amdgcn_readfirstlane(next.w);
       const int op = w0 & 0xff, d = (w0 >> 8) & 0xff;
       const bool use_pf = (w0 >> 16) & 1;
       const int a0 = w1 & 0xffff, a1 = (w1 >> 16) & 0xffff;
       if (op == OP_END) break;
+      next = prog[pc + 1];  // in flight during this op: its latency would open every op
 #define PCSF_CASES(D)                                          \
   case OP_CHERRY * 8 + D:                                      \
     if constexpr (D < NS) w.cherry(S[D], K[D], a0, a1, use_pf); \
