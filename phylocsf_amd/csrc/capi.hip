@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <initializer_list>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -14,6 +15,7 @@
 #include "host/omega.hpp"
 #include "host/program.hpp"
 #include "host/text.hpp"
+#include "devpool.hpp"
 #include "internal.hpp"
 
 namespace {
@@ -40,18 +42,60 @@ bool alloc_over_limit(size_t bytes) {
   return bytes > std::strtoull(lim, nullptr, 10);
 }
 
+pcsf::DevPool& pool() {
+  static pcsf::DevPool* p = new pcsf::DevPool();  // outlives every context
+  return *p;
+}
+
+// Device memory of context c (kept by its pool once freed).
 template <typename T>
-hipError_t dalloc(T** p, size_t count) {
+hipError_t dalloc(pcsf_ctx* c, T** p, size_t count) {
   *p = nullptr;
   if (count == 0) return hipSuccess;
   if (alloc_over_limit(count * sizeof(T))) return hipErrorOutOfMemory;
-  return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
+  return pool().alloc(c ? c->pool_id : 0, count * sizeof(T), reinterpret_cast<void**>(p));
 }
 
 template <typename T>
 void dfree(T*& p) {
-  if (p) (void)hipFree(p);
+  if (p) pool().free(const_cast<void*>(static_cast<const void*>(p)));
   p = nullptr;
+}
+
+// Every wait for the context's stream: what its pinned ring holds has been
+// copied by then.
+hipError_t ctx_wait(pcsf_ctx* c) {
+  const hipError_t e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) c->pin_used = 0;
+  return e;
+}
+
+// `bytes` of the context's pinned ring (nullptr when it is smaller): filled
+// by the host for an upload, or by a copy from the device.
+uint8_t* pin_take(pcsf_ctx* c, size_t bytes, hipError_t* e) {
+  *e = hipSuccess;
+  bytes = (bytes + 63) / 64 * 64;
+  if (!c->pin || bytes > c->pin_cap) return nullptr;
+  if (c->pin_used + bytes > c->pin_cap) *e = ctx_wait(c);
+  if (*e != hipSuccess) return nullptr;
+  uint8_t* p = c->pin + c->pin_used;
+  c->pin_used += bytes;
+  return p;
+}
+
+// Copies host memory to the device on the context's stream; the host memory
+// may change as soon as this returns.  Small pieces go through the pinned ring
+// (no wait), large ones wait for the copy.
+hipError_t upload(pcsf_ctx* c, void* dst, const void* src, size_t bytes) {
+  if (!bytes) return hipSuccess;
+  hipError_t e;
+  if (uint8_t* p = pin_take(c, bytes, &e)) {
+    std::memcpy(p, src, bytes);
+    return hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, c->stream);
+  }
+  if (e != hipSuccess) return e;
+  e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream);
+  return e == hipSuccess ? ctx_wait(c) : e;
 }
 
 bool rho_valid(double r) { return r > 0.0 && std::isfinite(r); }
@@ -70,43 +114,55 @@ constexpr const char* kTreeOnly =
 
 void free_psets(PSets& ps);
 
-hipError_t alloc_psets(PSets& ps, int cap, int nbr, bool fp64, int nctab = 0,
-                       bool tangent = false, bool own_models = false) {
+// The arrays of the kBuild* outputs that the sets do not hold yet.
+hipError_t add_outputs(pcsf_ctx* c, PSets& ps, int nbr, unsigned outputs) {
   hipError_t e = hipSuccess;
   auto chk = [&](hipError_t x) {
     if (e == hipSuccess) e = x;
   };
-  const size_t n = (size_t)cap * nbr;
-  chk(dalloc(&ps.d_PT32, n * kLeafRows * 64));
-  chk(dalloc(&ps.d_Pfrag, n * kTileFloats));
-  chk(dalloc(&ps.d_lnPcc, n * kLeafRows));
-  chk(dalloc(&ps.d_rho, (size_t)cap));
-  chk(dalloc(&ps.d_active, (size_t)cap));
-  if (fp64) chk(dalloc(&ps.d_P64T, n * 4096));
-  if (fp64) chk(dalloc(&ps.d_P64F, n * kTile64));
-  if (fp64) chk(dalloc(&ps.d_P64FT, n * 4096));
-  if (tangent) {
-    chk(dalloc(&ps.d_DT32, n * kLeafRows * 64));
-    chk(dalloc(&ps.d_Dfrag, n * 4096));
+  const size_t n = (size_t)ps.cap * nbr;
+  const unsigned add = outputs & ~ps.outputs;
+  if (add & kBuildMfma) {
+    chk(dalloc(c, &ps.d_PT32, n * kLeafRows * 64));
+    chk(dalloc(c, &ps.d_Pfrag, n * kTileFloats));
+    chk(dalloc(c, &ps.d_lnPcc, n * kLeafRows));
   }
+  if (add & kBuildP64) chk(dalloc(c, &ps.d_P64T, n * 4096));
+  if (add & kBuildP64M) chk(dalloc(c, &ps.d_P64F, n * kTile64));
+  if (add & kBuildP64MT) chk(dalloc(c, &ps.d_P64FT, n * 4096));
+  if (add & kBuildTangent) {
+    chk(dalloc(c, &ps.d_DT32, n * kLeafRows * 64));
+    chk(dalloc(c, &ps.d_Dfrag, n * 4096));
+  }
+  if (e == hipSuccess) ps.outputs |= add;
+  else free_psets(ps);  // nothing half-allocated survives: cap is 0
+  return e;
+}
+
+hipError_t alloc_psets(pcsf_ctx* c, PSets& ps, int cap, int nbr, unsigned outputs, int nctab = 0,
+                       bool own_models = false) {
+  hipError_t e = hipSuccess;
+  auto chk = [&](hipError_t x) {
+    if (e == hipSuccess) e = x;
+  };
+  // the parameters of a pass: scales, settings, flags, modes (set_params)
+  chk(dalloc(c, &ps.d_params, (size_t)cap * (8 + 1 + (own_models ? 12 * 8 + 1 : 0))));
   if (nctab > 0) {
-    chk(dalloc(&ps.d_ctab, (size_t)cap * nctab * kTabCodes * kTabCodes * 64));
-    chk(dalloc(&ps.d_clnt, (size_t)cap * nctab * kTabCodes * kTabCodes));
+    chk(dalloc(c, &ps.d_ctab, (size_t)cap * nctab * kTabCodes * kTabCodes * 64));
+    chk(dalloc(c, &ps.d_clnt, (size_t)cap * nctab * kTabCodes * kTabCodes));
   }
   if (own_models) {
-    chk(dalloc(&ps.d_eVT, (size_t)cap * 4096));
-    chk(dalloc(&ps.d_eVinv, (size_t)cap * 4096));
-    chk(dalloc(&ps.d_elam, (size_t)cap * 64));
-    chk(dalloc(&ps.d_epi, (size_t)cap * 64));
-    chk(dalloc(&ps.d_elnpi, (size_t)cap * 64));
-  }
-  if (e != hipSuccess) {
-    free_psets(ps);  // nothing half-allocated survives: cap stays 0
-    return e;
+    chk(dalloc(c, &ps.d_eVT, (size_t)cap * 4096));
+    chk(dalloc(c, &ps.d_eVinv, (size_t)cap * 4096));
+    chk(dalloc(c, &ps.d_elam, (size_t)cap * 64));
+    chk(dalloc(c, &ps.d_epi, (size_t)cap * 64));
+    chk(dalloc(c, &ps.d_elnpi, (size_t)cap * 64));
+    chk(dalloc(c, &ps.d_eref, (size_t)cap * 4096));
   }
   ps.cap = cap;
-  ps.fp64 = fp64;
   ps.fmt = -1;
+  if (e == hipSuccess) e = add_outputs(c, ps, nbr, outputs);
+  else free_psets(ps);
   return e;
 }
 
@@ -117,8 +173,7 @@ void free_psets(PSets& ps) {
   dfree(ps.d_PT32);
   dfree(ps.d_Pfrag);
   dfree(ps.d_lnPcc);
-  dfree(ps.d_rho);
-  dfree(ps.d_active);
+  dfree(ps.d_params);
   dfree(ps.d_ctab);
   dfree(ps.d_clnt);
   dfree(ps.d_DT32);
@@ -128,9 +183,40 @@ void free_psets(PSets& ps) {
   dfree(ps.d_elam);
   dfree(ps.d_epi);
   dfree(ps.d_elnpi);
+  dfree(ps.d_eref);
+  ps.d_rho = ps.d_qs = nullptr;
+  ps.d_active = ps.d_mode = nullptr;
   ps.cap = 0;
-  ps.fp64 = false;
+  ps.outputs = 0;
   ps.fmt = -1;
+}
+
+// One upload of a pass's per-set parameters (n sets): tree scales, then the
+// omega settings and modes of sets with rate models of their own, and the
+// active flags.
+hipError_t set_params(pcsf_ctx* c, PSets& ps, size_t n, const double* rho, const uint8_t* active,
+                      const double* qs = nullptr, const uint8_t* mode = nullptr) {
+  const size_t nq = qs ? n * 12 * 8 : 0;
+  const size_t bytes = n * 8 + nq + n + (qs ? n : 0);
+  ps.d_rho = reinterpret_cast<double*>(ps.d_params);
+  ps.d_qs = qs ? reinterpret_cast<double*>(ps.d_params + n * 8) : nullptr;
+  ps.d_active = ps.d_params + n * 8 + nq;
+  ps.d_mode = qs ? ps.d_active + n : nullptr;
+  auto fill = [&](uint8_t* p) {
+    std::memcpy(p, rho, n * 8);
+    if (qs) std::memcpy(p + n * 8, qs, nq);
+    std::memcpy(p + n * 8 + nq, active, n);
+    if (qs) std::memcpy(p + n * 9 + nq, mode, n);
+  };
+  hipError_t e;
+  if (uint8_t* p = pin_take(c, bytes, &e)) {
+    fill(p);
+    return hipMemcpyAsync(ps.d_params, p, bytes, hipMemcpyHostToDevice, c->stream);
+  }
+  if (e != hipSuccess) return e;
+  std::vector<uint8_t> h(bytes);
+  fill(h.data());
+  return upload(c, ps.d_params, h.data(), bytes);
 }
 
 // The reference's message for a P(t) failure recorded by the P builder as
@@ -170,16 +256,24 @@ int pbuild_failure(pcsf_model* m, unsigned long long key, const double* rho_host
   return set_err(c, PCSF_EFAIL, buf);
 }
 
-// Runs the P builder over `nsets` sets whose rho/active are already on the
+// The failure record holds all ones unless a build failed since the last
+// reset; a failure reads it, resets it and makes the reference's message.
+int failed_build(pcsf_model* m, unsigned long long key, const double* rho_host,
+                 bool own_models) {
+  (void)hipMemsetAsync(m->d_perr, 0xff, sizeof(unsigned long long), m->ctx->stream);
+  return pbuild_failure(m, key, rho_host, own_models);
+}
+
+// Runs the P builder over `nsets` sets whose parameters are already on the
 // device.  A failure comes back as the key of the first failing (set,
 // branch, row) in the reference's order; its message is made on the host
-// from the same P(t) built in FP64 by Q.Diag.real_to_Pt's rules.
+// from the same P(t) built in FP64 by Q.Diag.real_to_Pt's rules.  With
+// `later` the record is not read here: the caller's results come with a copy
+// of it (the kernels in between run on whatever was built: no index depends
+// on it).
 int run_pbuild(pcsf_model* m, PSets& ps, int nsets, const double* rho_host, int fmt,
-               float* ms_out,
-               unsigned outputs = kBuildP64 | kBuildP64M | kBuildP64MT | kBuildMfma |
-                                  kBuildTangent) {
+               float* ms_out, unsigned outputs, bool later) {
   pcsf_ctx* c = m->ctx;
-  HIP_TRY(c, hipMemsetAsync(m->d_perr, 0xff, sizeof(unsigned long long), c->stream));
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (c->timing && ms_out) {
     HIP_TRY(c, hipEventCreate(&e0));
@@ -190,8 +284,10 @@ int run_pbuild(pcsf_model* m, PSets& ps, int nsets, const double* rho_host, int 
   HIP_TRY(c, launch_pbuild(m, ps, nsets, fmt, outputs, c->stream));
   if (e1) HIP_TRY(c, hipEventRecord(e1, c->stream));
   unsigned long long key = ~0ull;
-  HIP_TRY(c, hipMemcpyAsync(&key, m->d_perr, sizeof key, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (!later || e0) {
+    HIP_TRY(c, hipMemcpyAsync(&key, m->d_perr, sizeof key, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, ctx_wait(c));
+  }
   if (e0) {
     float ms = 0;
     (void)hipEventElapsedTime(&ms, e0, e1);
@@ -199,7 +295,7 @@ int run_pbuild(pcsf_model* m, PSets& ps, int nsets, const double* rho_host, int 
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
   }
-  if (key != ~0ull) return pbuild_failure(m, key, rho_host, ps.d_eVT != nullptr);
+  if (key != ~0ull) return failed_build(m, key, rho_host, ps.d_eVT != nullptr);
   ps.fmt = (outputs & kBuildMfma) ? fmt : -1;
   return PCSF_OK;
 }
@@ -211,7 +307,8 @@ int run_pbuild(pcsf_model* m, PSets& ps, int nsets, const double* rho_host, int 
 // its scales on every call and reads neither tiles nor tables).  Allocates
 // nothing: the sets are the model's own and cached_rho's capacity is reserved
 // when the model is made.
-int ensure_transitions(pcsf_model* m, const double* rho, int fmt, unsigned need, float* ms_out) {
+int ensure_transitions(pcsf_model* m, const double* rho, int fmt, unsigned need, float* ms_out,
+                       bool later = false) {
   pcsf_ctx* c = m->ctx;
   if (ms_out) *ms_out = 0.f;
   const bool same_rho = (int)m->cached_rho.size() == m->nm &&
@@ -220,9 +317,8 @@ int ensure_transitions(pcsf_model* m, const double* rho, int fmt, unsigned need,
     m->cached_rho.clear();
     m->built = 0;
     m->tables = false;
-    HIP_TRY(c, hipMemcpyAsync(m->fixed.d_rho, rho, sizeof(double) * m->nm,
-                              hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, hipMemsetAsync(m->fixed.d_active, 1, (size_t)m->nm, c->stream));
+    const uint8_t all[8] = {1, 1, 1, 1, 1, 1, 1, 1};  // nm <= 8
+    HIP_TRY(c, set_params(c, m->fixed, (size_t)m->nm, rho, all));
   }
   if ((m->built & kBuildMfma) && m->fixed.fmt != fmt) m->built &= ~kBuildMfma;
   const bool tables = (need & kBuildMfma) && !m->cherries.empty() && !m->tables;
@@ -230,7 +326,7 @@ int ensure_transitions(pcsf_model* m, const double* rho, int fmt, unsigned need,
   const unsigned missing = need & ~m->built;
   if (missing) {
     const int had_fmt = (m->built & kBuildMfma) ? m->fixed.fmt : -1;
-    int rc = run_pbuild(m, m->fixed, m->nm, rho, fmt, ms_out, missing);
+    int rc = run_pbuild(m, m->fixed, m->nm, rho, fmt, ms_out, missing, later);
     if (rc) {
       m->cached_rho.clear();
       m->built = 0;
@@ -272,17 +368,14 @@ int ensure_aligned(pcsf_batch* b) {
   auto chk = [&](hipError_t x) {
     if (e == hipSuccess) e = x;
   };
-  chk(dalloc(&al.d_codes, (size_t)m->nl * al.ld));
-  chk(dalloc(&al.d_block_region, br.size()));
-  chk(dalloc(&al.d_astart, al.astart.size()));
-  chk(dalloc(&b->d_alogz, (size_t)m->nm * al.ld));
-  chk(dalloc(&b->d_acolelpr, (size_t)m->nm * al.ld));
-  if (e == hipSuccess)
-    chk(hipMemcpy(al.d_block_region, br.data(), br.size() * 4, hipMemcpyHostToDevice));
-  if (e == hipSuccess)
-    chk(hipMemcpy(al.d_astart, al.astart.data(), al.astart.size() * 8, hipMemcpyHostToDevice));
+  chk(dalloc(c, &al.d_codes, (size_t)m->nl * al.ld));
+  chk(dalloc(c, &al.d_block_region, br.size()));
+  chk(dalloc(c, &al.d_astart, al.astart.size()));
+  chk(dalloc(c, &b->d_alogz, (size_t)m->nm * al.ld));
+  chk(dalloc(c, &b->d_acolelpr, (size_t)m->nm * al.ld));
+  if (e == hipSuccess) chk(upload(c, al.d_block_region, br.data(), br.size() * 4));
+  if (e == hipSuccess) chk(upload(c, al.d_astart, al.astart.data(), al.astart.size() * 8));
   if (e == hipSuccess) chk(launch_align_codes(b, c->stream));
-  if (e == hipSuccess) chk(hipStreamSynchronize(c->stream));
   if (e != hipSuccess) {
     // leave the batch as before the call: the next per-region call retries
     dfree(al.d_codes);
@@ -299,25 +392,98 @@ int ensure_aligned(pcsf_batch* b) {
 }
 
 // Device memory for the per-region transition sets of a batch: regions go
-// through in chunks of as many sets as fit, 24 GiB (a fraction of the 288 GB
-// of one MI355X, so that several large batches can live side by side) unless
-// PHYLOCSF_SET_BUDGET_MB says otherwise (read on every pass; small values
-// force many chunks, which the tests use).
+// through in chunks of as many sets as fit, 4 GiB per kind of pass (600 sets of
+// 100vertebrates: thousands of workgroups a chunk; all kinds together stay
+// within what the context's pool keeps) unless PHYLOCSF_SET_BUDGET_MB says
+// otherwise (read on every pass; small values force many chunks, which the
+// tests use).
 size_t set_budget() {
   const char* e = std::getenv("PHYLOCSF_SET_BUDGET_MB");
   if (e && *e) {
     const long long mb = std::atoll(e);
     if (mb > 0) return (size_t)mb << 20;
   }
-  return (size_t)24 << 30;
+  return (size_t)4 << 30;
 }
 
 // Bytes of one transition set on the device.
-size_t set_bytes(const pcsf_model* m, bool fp64, bool tangent = false, bool own_model = false) {
-  return (size_t)m->nbr * (kLeafRows * 64 * 4 + kTileFloats * 4 + kLeafRows * 8 +
-                           (fp64 ? (2 * 4096 + kTile64) * 8 : 0) +
-                           (tangent ? (kLeafRows + 64) * 64 * 4 : 0)) +
-         (own_model ? (2 * 4096 + 3 * 64) * 8 : 0);
+size_t set_bytes(const pcsf_model* m, unsigned outputs, bool own_model) {
+  const size_t branch = ((outputs & kBuildMfma) ? kLeafRows * 64 * 4 + kTileFloats * 4 + kLeafRows * 8 : 0) +
+                        ((outputs & kBuildP64) ? 4096 * 8 : 0) +
+                        ((outputs & kBuildP64M) ? kTile64 * 8 : 0) +
+                        ((outputs & kBuildP64MT) ? 4096 * 8 : 0) +
+                        ((outputs & kBuildTangent) ? (kLeafRows + 64) * 64 * 4 : 0);
+  return m->nbr * branch + (own_model ? (3 * 4096 + 3 * 64) * 8 : 0) + 128;
+}
+
+// The batch's transition sets hold `need` (with or without rate models of
+// their own) for all regions or as many as the budget lets through at a time.
+// A reallocated pool keeps what the old one served, so that maximisers
+// alternating passes do not rebuild it each time.
+int ensure_region_sets(pcsf_batch* b, unsigned need, bool own) {
+  pcsf_model* m = b->m;
+  pcsf_ctx* c = m->ctx;
+  PSets& rs = b->rs;
+  const bool keep = rs.cap > 0 && own == (rs.d_eVT != nullptr);
+  const unsigned all = need | (keep ? rs.outputs : 0);
+  int cap = (int)std::max<size_t>(m->nm, set_budget() / set_bytes(m, all, own) / m->nm * m->nm);
+  cap = std::min<int>(cap, std::max(m->nm, b->nreg * m->nm));
+  if (rs.cap >= cap && keep && !(need & ~rs.outputs)) return PCSF_OK;
+  b->eig_ok.clear();
+  b->eig_ref_ok.clear();
+  if (rs.cap >= cap && keep) {
+    HIP_TRY(c, add_outputs(c, rs, m->nbr, need));
+  } else {
+    free_psets(rs);
+    HIP_TRY(c, alloc_psets(c, rs, cap, m->nbr, all, 0, own));
+  }
+  return PCSF_OK;
+}
+
+// Results of a pass, `head` (the P builder's failure record) and then the
+// per-pair values, from the device to the host arrays in `out` (np values
+// each; null: not wanted), and the failure, if the pass left the check to here.
+int fetch_results(pcsf_batch* b, const double* d_res, size_t np,
+                  std::initializer_list<double*> out, bool check, const double* rho, bool own,
+                  const char* where) {
+  pcsf_model* m = b->m;
+  pcsf_ctx* c = m->ctx;
+  const size_t count = 1 + np * out.size();
+  hipError_t e;
+  std::vector<double> h;
+  double* p = reinterpret_cast<double*>(pin_take(c, count * 8, &e));
+  HIP_TRY(c, e);
+  if (!p) {
+    h.resize(count);
+    p = h.data();
+  }
+  HIP_TRY(c, hipMemcpyAsync(p, d_res, count * 8, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, ctx_wait(c));
+  if (check) {
+    unsigned long long key;
+    std::memcpy(&key, p, 8);
+    if (key != ~0ull) {
+      const int rc = failed_build(m, key, rho, own);
+      c->err += where;
+      return rc;
+    }
+  }
+  size_t k = 0;
+  for (double* o : out) {
+    if (o) std::memcpy(o, p + 1 + np * k, np * 8);
+    ++k;
+  }
+  return PCSF_OK;
+}
+
+// The batch's timing events (made when timing is first on).
+hipError_t ensure_events(pcsf_batch* b) {
+  for (auto& ev : b->ev)
+    if (!ev) {
+      const hipError_t e = hipEventCreate(&ev);
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
 }
 
 // Rate models of their own for every (region, model) pair k = r * nm + q:
@@ -336,7 +502,7 @@ int ensure_adj_scratch(pcsf_batch* b) {
   if (b->adj_scratch >= need) return PCSF_OK;
   dfree(b->d_adj_scratch);
   b->adj_scratch = 0;
-  HIP_TRY(c, dalloc(&b->d_adj_scratch, need));
+  HIP_TRY(c, dalloc(c, &b->d_adj_scratch, need));
   b->adj_scratch = need;
   return PCSF_OK;
 }
@@ -344,9 +510,10 @@ int ensure_adj_scratch(pcsf_batch* b) {
 // Forward with one tree scale per (region, model): rho[r*nm+q].  active
 // (optional, r*nm+q) restricts the work to the listed pairs; results of the
 // others are left as they were.  Regions go through in chunks whose
-// transition sets fit the memory budget.
+// transition sets fit the memory budget.  The results come to loglik and elpr
+// (host, may be null) as well.
 int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int precision,
-                    const SetModels* sm = nullptr) {
+                    double* loglik, double* elpr, const SetModels* sm = nullptr) {
   pcsf_model* m = b->m;
   pcsf_ctx* c = m->ctx;
   const int nm = m->nm;
@@ -355,24 +522,15 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
   const bool fp64 = fp64_precision(precision);
   const int fmt = fp64 ? kFragF32 : frag_format(precision);
   const bool own = sm != nullptr;
-  // a reallocated pool keeps what the old one served (FP64 and tangent
-  // data), so that maximisers alternating passes do not rebuild it each time
-  const bool keep = own == (b->rs.d_eVT != nullptr);
-  const bool want_fp64 = fp64 || (keep && b->rs.fp64);
-  const bool want_tangent = keep && b->rs.d_Dfrag != nullptr;
-  int cap = (int)std::max<size_t>(
-      nm, set_budget() / set_bytes(m, want_fp64, want_tangent, own) / nm * nm);
-  cap = std::min<int>(cap, std::max(nm, b->nreg * nm));
-  if (b->rs.cap < cap || (fp64 && !b->rs.fp64) || !keep) {
-    free_psets(b->rs);
-    b->eig_ok.clear();
-    b->eig_ref_ok.clear();
-    HIP_TRY(c, alloc_psets(b->rs, cap, m->nbr, want_fp64, 0, want_tangent, own));
-  }
+  if ((rc = ensure_region_sets(b, set_outputs(precision), own))) return rc;
+  if (c->timing) HIP_TRY(c, ensure_events(b));
   const int chunk_regions = b->rs.cap / nm;
   // one chunk: set k is pair k on every pass, so a set's eigensystem can
   // seed (or stand for) the next one's
   const bool one_chunk = chunk_regions >= b->nreg;
+  // one chunk: a failed P build is reported with the results
+  const bool later = one_chunk && !c->timing;
+  bool ran = false;
   if (!one_chunk) {
     b->eig_ok.clear();
     b->eig_ref_ok.clear();
@@ -402,23 +560,10 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
         (r0 + nr < b->nreg) ? b->al.block0[r0 + nr] : (b->al.ld / kAlignCols);
     ch.nblocks = end_block - ch.block0;
     ch.sets = &b->rs;
-    HIP_TRY(c, hipMemcpyAsync(b->rs.d_rho, rho + (size_t)r0 * nm, sizeof(double) * nr * nm,
-                              hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(b->rs.d_active, act.data(), act.size(), hipMemcpyHostToDevice,
-                              c->stream));
+    ran = true;
+    if (!own) HIP_TRY(c, set_params(c, b->rs, (size_t)nr * nm, rho + (size_t)r0 * nm, act.data()));
     if (own) {  // the chunk's rate models, built from their settings
       const size_t k0 = (size_t)r0 * nm, nk = (size_t)nr * nm;
-      if (b->setqs_cap < (size_t)b->rs.cap * 12) {
-        dfree(b->d_setqs);
-        dfree(b->d_eigmode);
-        dfree(b->d_eigref);
-        b->setqs_cap = 0;
-        b->eig_ref_ok.clear();
-        HIP_TRY(c, dalloc(&b->d_setqs, (size_t)b->rs.cap * 12));
-        HIP_TRY(c, dalloc(&b->d_eigmode, (size_t)b->rs.cap));
-        HIP_TRY(c, dalloc(&b->d_eigref, (size_t)b->rs.cap * 4096));
-        b->setqs_cap = (size_t)b->rs.cap * 12;
-      }
       // per set: keep (inactive, or settings as last built), warm (the
       // reference basis has the same pi: only kappa / omega differ), or cold
       if (one_chunk && b->eig_ok.size() != nk) {
@@ -444,18 +589,14 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
           eigmode[k] = kEigWarm;
         any = any || eigmode[k] != kEigKeep;
       }
+      HIP_TRY(c, set_params(c, b->rs, nk, rho + k0, act.data(), sm->qs + k0 * 12, eigmode.data()));
       if (any) {
         if (one_chunk)  // invalid until the launch below is issued
           for (size_t k = 0; k < nk; ++k) {
             if (eigmode[k] != kEigKeep) b->eig_ok[k] = 0;
             if (eigmode[k] == kEigCold) b->eig_ref_ok[k] = 0;
           }
-        HIP_TRY(c, hipMemcpyAsync(b->d_setqs, sm->qs + k0 * 12, nk * 12 * 8,
-                                  hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(c, hipMemcpyAsync(b->d_eigmode, eigmode.data(), nk, hipMemcpyHostToDevice,
-                                  c->stream));
-        HIP_TRY(c, launch_omega_eigen(b->d_setqs, b->d_eigmode, b->d_eigref, (int)nk, b->rs,
-                                      c->stream));
+        HIP_TRY(c, launch_omega_eigen((int)nk, b->rs, c->stream));
         if (one_chunk)
           for (size_t k = 0; k < nk; ++k) {
             const double* q = sm->qs + (k0 + k) * 12;
@@ -472,7 +613,7 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
     }
     float tp = 0.f;
     rc = run_pbuild(m, b->rs, nr * nm, rho + (size_t)r0 * nm, fmt, &tp,
-                    set_outputs(precision));
+                    set_outputs(precision), later);
     if (rc) {
       char buf[64];
       std::snprintf(buf, sizeof buf, " (region block from %d)", r0);
@@ -486,11 +627,14 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
             ? launch_forward_fp64m(m, b, ch, c->stream)
         : fp64 ? launch_prune_fp64_regions(m, b, ch, c->stream)
                : launch_prune_mfma_regions(m, b, precision, variant, ch, c->stream);
-    if (e == hipErrorInvalidValue && precision == PCSF_FP64)
+    if (e == hipErrorInvalidValue && precision == PCSF_FP64) {
+      // (the build's failure record goes unread)
+      (void)hipMemsetAsync(m->d_perr, 0xff, sizeof(unsigned long long), c->stream);
       return set_err(c, PCSF_EINVAL, "FP64 kernel: tree workspace exceeds 64 KiB of LDS");
+    }
     HIP_TRY(c, e);
     if (c->timing) HIP_TRY(c, hipEventRecord(b->ev[1], c->stream));
-    HIP_TRY(c, launch_region_reduce_aligned(b, ch, b->d_loglik, b->d_elpr, c->stream));
+    HIP_TRY(c, launch_region_reduce_aligned(b, ch, b->d_res, c->stream));
     if (c->timing) {
       HIP_TRY(c, hipEventRecord(b->ev[2], c->stream));
       HIP_TRY(c, hipEventSynchronize(b->ev[2]));
@@ -501,7 +645,8 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
       b->t_reduce += r;
     }
   }
-  return PCSF_OK;
+  return fetch_results(b, b->d_res, (size_t)b->nreg * nm, {loglik, elpr}, later && ran, rho, own,
+                       " (region block from 0)");
 }
 
 // Gradient pass at tree scales rho (nreg * nm) over the pairs in `active`
@@ -512,7 +657,7 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
 // per-region sums of d ln z / d t_br (nreg * nm * nbr); tangent = true: the
 // FP32 MFMA tangent pass (d lpr / d rho only).
 int adjoint_regions(pcsf_batch* b, const double* rho, const uint8_t* active, double* d_gbr,
-                    bool tangent = false) {
+                    bool tangent, double* loglik, double* grad, double* gsq) {
   pcsf_model* m = b->m;
   pcsf_ctx* c = m->ctx;
   const int nm = m->nm;
@@ -520,19 +665,11 @@ int adjoint_regions(pcsf_batch* b, const double* rho, const uint8_t* active, dou
   if (rc) return rc;
   // (sets with rate models of their own are not kept: the gradient passes
   // run on the models' eigensystems)
-  const bool keep = b->rs.d_eVT == nullptr;
-  const bool want_fp64 = !tangent || (keep && b->rs.fp64);
-  const bool want_tangent = tangent || (keep && b->rs.d_Dfrag != nullptr);
-  int cap = (int)std::max<size_t>(
-      nm, set_budget() / set_bytes(m, want_fp64, want_tangent) / nm * nm);
-  cap = std::min<int>(cap, std::max(nm, b->nreg * nm));
-  if (b->rs.cap < cap || (!tangent && !b->rs.fp64) || (tangent && !b->rs.d_Dfrag) || !keep) {
-    free_psets(b->rs);
-    b->eig_ok.clear();
-    b->eig_ref_ok.clear();
-    HIP_TRY(c, alloc_psets(b->rs, cap, m->nbr, want_fp64, 0, want_tangent));
-  }
+  const unsigned need = tangent ? (kBuildMfma | kBuildTangent) : (kBuildP64M | kBuildP64MT);
+  if ((rc = ensure_region_sets(b, need, false))) return rc;
   const int chunk_regions = b->rs.cap / nm;
+  const bool later = chunk_regions >= b->nreg && !c->timing;
+  bool ran = false;
   std::vector<uint8_t> act;
   for (int32_t r0 = 0; r0 < b->nreg; r0 += chunk_regions) {
     const int32_t nr = std::min<int32_t>(chunk_regions, b->nreg - r0);
@@ -551,13 +688,10 @@ int adjoint_regions(pcsf_batch* b, const double* rho, const uint8_t* active, dou
         (r0 + nr < b->nreg) ? b->al.block0[r0 + nr] : (b->al.ld / kAlignCols);
     ch.nblocks = end_block - ch.block0;
     ch.sets = &b->rs;
-    HIP_TRY(c, hipMemcpyAsync(b->rs.d_rho, rho + (size_t)r0 * nm, sizeof(double) * nr * nm,
-                              hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(b->rs.d_active, act.data(), act.size(), hipMemcpyHostToDevice,
-                              c->stream));
+    ran = true;
+    HIP_TRY(c, set_params(c, b->rs, (size_t)nr * nm, rho + (size_t)r0 * nm, act.data()));
     float tp = 0.f;
-    rc = run_pbuild(m, b->rs, nr * nm, rho + (size_t)r0 * nm, kFragF32, &tp,
-                    tangent ? (kBuildMfma | kBuildTangent) : (kBuildP64M | kBuildP64MT));
+    rc = run_pbuild(m, b->rs, nr * nm, rho + (size_t)r0 * nm, kFragF32, &tp, need, later);
     if (rc) return rc;
     hipError_t e;
     if (tangent) {
@@ -569,11 +703,10 @@ int adjoint_regions(pcsf_batch* b, const double* rho, const uint8_t* active, dou
                               b->d_adj_scratch, adjoint_mfma_grid(m), c->stream);
     }
     HIP_TRY(c, e);
-    HIP_TRY(c, launch_region_reduce_aligned(b, ch, b->d_gloglik, b->d_grad, c->stream,
-                                            b->d_gsq));
+    HIP_TRY(c, launch_region_reduce_aligned(b, ch, b->d_gres, c->stream));
   }
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  return PCSF_OK;
+  return fetch_results(b, b->d_gres, (size_t)b->nreg * nm, {loglik, grad, gsq}, later && ran, rho,
+                       false, "");
 }
 
 // ---- scratch of pcsf_forward_noalloc ---------------------------------------
@@ -645,6 +778,13 @@ int pcsf_ctx_create(int device, pcsf_ctx** out) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
     c->num_cus = prop.multiProcessorCount;
+  c->pool_id = pool().open();
+  // staging of small uploads and results (without it they go pageable)
+  constexpr size_t kPin = 1 << 20;
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->pin), kPin, hipHostMallocDefault) == hipSuccess)
+    c->pin_cap = kPin;
+  else
+    (void)hipGetLastError(), c->pin = nullptr;
   // the no-allocation forward's scratch on this device (looked up once per
   // device; a failure is reported by pcsf_forward_noalloc)
   hipError_t se = hipSuccess;
@@ -668,6 +808,8 @@ void pcsf_ctx_destroy(pcsf_ctx* c) {
     if (es.consumed[i]) (void)hipEventDestroy(es.consumed[i]);
   }
   if (es.copy) (void)hipStreamDestroy(es.copy);
+  pool().close(c->pool_id);  // (what models and batches still hold goes when they do)
+  if (c->pin) (void)hipHostFree(c->pin);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -684,7 +826,7 @@ void* pcsf_ctx_stream(pcsf_ctx* c) { return c ? reinterpret_cast<void*>(c->strea
 
 int pcsf_ctx_synchronize(pcsf_ctx* c) {
   if (!c) return PCSF_EINVAL;
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  HIP_TRY(c, ctx_wait(c));
   return PCSF_OK;
 }
 
@@ -867,18 +1009,18 @@ int pcsf_model_create(pcsf_ctx* c, int n, const int32_t* children, const double*
   }
 
   HIP_TRY(c, hipSetDevice(c->device));
-  HIP_TRY(c, dalloc(&m->d_VT, V.size()));
-  HIP_TRY(c, dalloc(&m->d_Vinv, Vi.size()));
-  HIP_TRY(c, dalloc(&m->d_lam, lam.size()));
-  HIP_TRY(c, dalloc(&m->d_pi, m->pi.size()));
-  HIP_TRY(c, dalloc(&m->d_lnpi, lnpi.size()));
-  HIP_TRY(c, dalloc(&m->d_QT, QT.size()));
-  HIP_TRY(c, dalloc(&m->d_branch, m->branch.size()));
-  HIP_TRY(c, dalloc(&m->d_lc, (size_t)n));
-  HIP_TRY(c, dalloc(&m->d_rc, (size_t)n));
-  HIP_TRY(c, dalloc(&m->d_prog, m->prog.size()));
-  HIP_TRY(c, dalloc(&m->d_prog_t, m->prog_t.size()));
-  HIP_TRY(c, dalloc(&m->d_cherries, std::max<size_t>(1, m->cherries.size())));
+  HIP_TRY(c, dalloc(c, &m->d_VT, V.size()));
+  HIP_TRY(c, dalloc(c, &m->d_Vinv, Vi.size()));
+  HIP_TRY(c, dalloc(c, &m->d_lam, lam.size()));
+  HIP_TRY(c, dalloc(c, &m->d_pi, m->pi.size()));
+  HIP_TRY(c, dalloc(c, &m->d_lnpi, lnpi.size()));
+  HIP_TRY(c, dalloc(c, &m->d_QT, QT.size()));
+  HIP_TRY(c, dalloc(c, &m->d_branch, m->branch.size()));
+  HIP_TRY(c, dalloc(c, &m->d_lc, (size_t)n));
+  HIP_TRY(c, dalloc(c, &m->d_rc, (size_t)n));
+  HIP_TRY(c, dalloc(c, &m->d_prog, m->prog.size()));
+  HIP_TRY(c, dalloc(c, &m->d_prog_t, m->prog_t.size()));
+  HIP_TRY(c, dalloc(c, &m->d_cherries, std::max<size_t>(1, m->cherries.size())));
   // leaves each program gathers (CHERRY operands, LEAFMUL operands)
   auto gathered = [&](const std::vector<int32_t>& ops) {
     std::vector<int16_t> out;
@@ -896,11 +1038,14 @@ int pcsf_model_create(pcsf_ctx* c, int n, const int32_t* children, const double*
   const std::vector<int16_t> lsl = gathered(m->prog), lsl_t = gathered(m->prog_t);
   m->n_lsl = (int)lsl.size();
   m->n_lsl_t = (int)lsl_t.size();
-  HIP_TRY(c, dalloc(&m->d_lsl, std::max<size_t>(1, lsl.size())));
-  HIP_TRY(c, dalloc(&m->d_lsl_t, std::max<size_t>(1, lsl_t.size())));
-  HIP_TRY(c, dalloc(&m->d_perr, (size_t)1));
+  HIP_TRY(c, dalloc(c, &m->d_lsl, std::max<size_t>(1, lsl.size())));
+  HIP_TRY(c, dalloc(c, &m->d_lsl_t, std::max<size_t>(1, lsl_t.size())));
+  HIP_TRY(c, dalloc(c, &m->d_perr, (size_t)1));
   if (!tree_only)
-    HIP_TRY(c, alloc_psets(m->fixed, nm, m->nbr, true, (int)m->cherries.size() / 3));
+    HIP_TRY(c, alloc_psets(c, m->fixed, nm, m->nbr,
+                           kBuildMfma | kBuildP64 | kBuildP64M | kBuildP64MT,
+                           (int)m->cherries.size() / 3));
+  HIP_TRY(c, hipMemset(m->d_perr, 0xff, sizeof(unsigned long long)));
   std::vector<int32_t> lc32(m->lc.begin(), m->lc.end()), rc32(m->rc.begin(), m->rc.end());
   auto up = [&](void* dst, const void* src, size_t bytes) {
     return bytes ? hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) : hipSuccess;
@@ -974,6 +1119,32 @@ int pcsf_model_transition(pcsf_model* m, int model, double rho, double* P_out) {
   return PCSF_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The device memory of a batch with m, ncols, ld and nreg set; results in one
+// piece per kind of pass, behind a copy of the P builder's failure record.
+hipError_t alloc_batch(pcsf_batch* b) {
+  pcsf_model* m = b->m;
+  pcsf_ctx* c = m->ctx;
+  const size_t np = (size_t)b->nreg * m->nm;
+  hipError_t e = dalloc(c, &b->d_codes, (size_t)m->nl * b->ld);
+  if (e == hipSuccess) e = dalloc(c, &b->d_offsets, (size_t)b->nreg + 1);
+  if (e == hipSuccess) e = dalloc(c, &b->d_logz, (size_t)m->nm * b->ld);
+  if (e == hipSuccess) e = dalloc(c, &b->d_colelpr, (size_t)m->nm * b->ld);
+  if (e == hipSuccess) e = dalloc(c, &b->d_res, 1 + 2 * np);
+  if (e == hipSuccess) e = dalloc(c, &b->d_gres, 1 + 3 * np);
+  if (e != hipSuccess) return e;
+  b->d_loglik = b->d_res + 1;
+  b->d_elpr = b->d_loglik + np;
+  return hipSuccess;
+}
+
+}  // namespace
+
+extern "C" {
+
 int pcsf_batch_create(pcsf_model* m, const uint8_t* codes, int64_t ncols,
                       const int64_t* off, int32_t nreg, pcsf_batch** out) {
   if (!m || !out || !m->ctx) return PCSF_EINVAL;
@@ -995,38 +1166,42 @@ int pcsf_batch_create(pcsf_model* m, const uint8_t* codes, int64_t ncols,
   b->offsets.assign(off, off + nreg + 1);
   b->ld = std::max<int64_t>(kGroupCols, (ncols + kGroupCols - 1) / kGroupCols * kGroupCols);
   HIP_TRY(c, hipSetDevice(c->device));
-  HIP_TRY(c, dalloc(&b->d_codes, (size_t)m->nl * b->ld));
-  HIP_TRY(c, dalloc(&b->d_offsets, (size_t)nreg + 1));
-  HIP_TRY(c, dalloc(&b->d_logz, (size_t)m->nm * b->ld));
-  HIP_TRY(c, dalloc(&b->d_colelpr, (size_t)m->nm * b->ld));
-  HIP_TRY(c, dalloc(&b->d_loglik, std::max<size_t>(1, (size_t)nreg * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_elpr, std::max<size_t>(1, (size_t)nreg * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_gloglik, std::max<size_t>(1, (size_t)nreg * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_grad, std::max<size_t>(1, (size_t)nreg * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_gsq, std::max<size_t>(1, (size_t)nreg * m->nm)));
-  HIP_TRY(c, hipMemcpy(b->d_offsets, off, sizeof(int64_t) * (nreg + 1), hipMemcpyHostToDevice));
+  HIP_TRY(c, alloc_batch(b));
+  HIP_TRY(c, upload(c, b->d_offsets, off, sizeof(int64_t) * (nreg + 1)));
   // upload through a staging buffer (with a flag word for invalid codes at
   // its end), then make leaf-major
+  constexpr const char* kBadCode =
+      "pcsf_batch_create: a leaf code is neither a codon index (0..63) nor "
+      "PCSF_MARGINALIZE (255)";
   uint8_t* stage = nullptr;
   const size_t bytes = (size_t)ncols * m->nl;
   const size_t flag_at = (bytes + 3) / 4 * 4;
-  HIP_TRY(c, dalloc(&stage, flag_at + 4));
+  HIP_TRY(c, dalloc(c, &stage, flag_at + 4));
   int* d_bad = reinterpret_cast<int*>(stage + flag_at);
   int bad = 0;
-  hipError_t e = hipMemsetAsync(d_bad, 0, 4, c->stream);
-  if (e == hipSuccess && bytes) e = hipMemcpyAsync(stage, codes, bytes, hipMemcpyHostToDevice,
-                                                    c->stream);
-  if (e == hipSuccess)
-    e = launch_transpose_codes(stage, ncols, m->nl, b->d_codes, b->ld, d_bad, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  (void)hipFree(stage);
+  hipError_t e = hipSuccess;
+  // a small batch is checked here and uploaded without a wait, a large one by
+  // the transpose (64 KB are a few us of a core, a wait is ten)
+  if (bytes <= (64 << 10)) {
+    uint8_t wrong = 0;
+    for (size_t i = 0; i < bytes; ++i)
+      wrong |= (uint8_t)((codes[i] > 63) & (codes[i] != PCSF_MARGINALIZE));
+    bad = wrong;
+    if (!bad) e = upload(c, stage, codes, bytes);
+    if (!bad && e == hipSuccess)
+      e = launch_transpose_codes(stage, ncols, m->nl, b->d_codes, b->ld, nullptr, c->stream);
+  } else {
+    e = hipMemsetAsync(d_bad, 0, 4, c->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(stage, codes, bytes, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess)
+      e = launch_transpose_codes(stage, ncols, m->nl, b->d_codes, b->ld, d_bad, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = ctx_wait(c);
+  }
+  dfree(stage);
   HIP_TRY(c, e);
-  if (bad)
-    return set_err(c, PCSF_EINVAL,
-                   "pcsf_batch_create: a leaf code is neither a codon index (0..63) nor "
-                   "PCSF_MARGINALIZE (255)");
-  for (auto& ev : b->ev) HIP_TRY(c, hipEventCreate(&ev));
+  if (bad) return set_err(c, PCSF_EINVAL, kBadCode);
   *out = guard.release();
   return PCSF_OK;
 }
@@ -1064,22 +1239,13 @@ int pcsf_batch_create_frames(pcsf_model* m, const uint8_t* nuc, int64_t n_nuc,
   b->offsets = foff;
   b->ld = std::max<int64_t>(kGroupCols, (ncols + kGroupCols - 1) / kGroupCols * kGroupCols);
   HIP_TRY(c, hipSetDevice(c->device));
-  HIP_TRY(c, dalloc(&b->d_codes, (size_t)m->nl * b->ld));
-  HIP_TRY(c, dalloc(&b->d_offsets, (size_t)nbr + 1));
-  HIP_TRY(c, dalloc(&b->d_logz, (size_t)m->nm * b->ld));
-  HIP_TRY(c, dalloc(&b->d_colelpr, (size_t)m->nm * b->ld));
-  HIP_TRY(c, dalloc(&b->d_loglik, std::max<size_t>(1, (size_t)nbr * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_elpr, std::max<size_t>(1, (size_t)nbr * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_gloglik, std::max<size_t>(1, (size_t)nbr * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_grad, std::max<size_t>(1, (size_t)nbr * m->nm)));
-  HIP_TRY(c, dalloc(&b->d_gsq, std::max<size_t>(1, (size_t)nbr * m->nm)));
-  HIP_TRY(c, hipMemcpy(b->d_offsets, foff.data(), sizeof(int64_t) * foff.size(),
-                       hipMemcpyHostToDevice));
+  HIP_TRY(c, alloc_batch(b));
+  HIP_TRY(c, upload(c, b->d_offsets, foff.data(), sizeof(int64_t) * foff.size()));
   uint8_t* d_nuc = nullptr;
   int64_t* d_roff = nullptr;
   const size_t bytes = (size_t)n_nuc * m->nl;
-  hipError_t e = dalloc(&d_nuc, std::max<size_t>(bytes, 1));
-  if (e == hipSuccess) e = dalloc(&d_roff, (size_t)nreg + 1);
+  hipError_t e = dalloc(c, &d_nuc, std::max<size_t>(bytes, 1));
+  if (e == hipSuccess) e = dalloc(c, &d_roff, (size_t)nreg + 1);
   if (e == hipSuccess && bytes) e = hipMemcpy(d_nuc, nuc, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(d_roff, roff, sizeof(int64_t) * (nreg + 1), hipMemcpyHostToDevice);
@@ -1093,7 +1259,6 @@ int pcsf_batch_create_frames(pcsf_model* m, const uint8_t* nuc, int64_t n_nuc,
   dfree(d_nuc);
   dfree(d_roff);
   HIP_TRY(c, e);
-  for (auto& ev : b->ev) HIP_TRY(c, hipEventCreate(&ev));
   *out = guard.release();
   return PCSF_OK;
 }
@@ -1104,20 +1269,14 @@ void pcsf_batch_destroy(pcsf_batch* b) {
   dfree(b->d_offsets);
   dfree(b->d_logz);
   dfree(b->d_colelpr);
-  dfree(b->d_loglik);
-  dfree(b->d_elpr);
+  dfree(b->d_res);
+  dfree(b->d_gres);
   dfree(b->al.d_codes);
   dfree(b->al.d_block_region);
   dfree(b->al.d_astart);
   dfree(b->d_alogz);
   dfree(b->d_acolelpr);
-  dfree(b->d_gloglik);
-  dfree(b->d_grad);
-  dfree(b->d_gsq);
   dfree(b->d_adj_scratch);
-  dfree(b->d_setqs);
-  dfree(b->d_eigmode);
-  dfree(b->d_eigref);
   free_psets(b->rs);
   for (auto& ev : b->ev)
     if (ev) (void)hipEventDestroy(ev);
@@ -1143,6 +1302,67 @@ int pcsf_batch_codes(pcsf_batch* b, uint8_t* codes, int64_t* region_offsets) {
   return PCSF_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The forward of every region at one tree scale per model, enqueued: results
+// (and, with `later`, the P builder's failure record) in the batch's d_res.
+int shared_pass(pcsf_batch* b, const double* r, int precision, bool later) {
+  pcsf_model* m = b->m;
+  pcsf_ctx* c = m->ctx;
+  float tp = 0.f;
+  int rc = ensure_transitions(m, r, frag_format(precision), set_outputs(precision), &tp,
+                              later && b->nreg > 0);
+  if (rc) return rc;
+  if (precision == PCSF_FP64M && b->nreg > 0) {
+    // region-aligned columns, the model's sets for every region
+    if ((rc = ensure_aligned(b))) return rc;
+  }
+  b->t_pbuild = tp;
+  b->last_rho.resize((size_t)b->nreg * m->nm);
+  b->last_precision = precision;
+  for (int32_t i = 0; i < b->nreg; ++i)
+    for (int q = 0; q < m->nm; ++q) b->last_rho[(size_t)i * m->nm + q] = r[q];
+  if (c->timing) {
+    HIP_TRY(c, ensure_events(b));
+    HIP_TRY(c, hipEventRecord(b->ev[0], c->stream));
+  }
+  hipError_t e;
+  RegionChunk all;
+  all.r0 = 0;
+  all.nreg = b->nreg;
+  all.block0 = 0;
+  all.nblocks = b->al.ld / kAlignCols;
+  all.sets = &m->fixed;
+  if (precision == PCSF_FP64M) {
+    e = b->nreg > 0 ? launch_forward_fp64m(m, b, all, c->stream) : hipSuccess;
+  } else if (precision == PCSF_FP64) {
+    e = launch_prune_fp64(m, b, c->stream);
+    if (e == hipErrorInvalidValue) {
+      (void)hipMemsetAsync(m->d_perr, 0xff, sizeof(unsigned long long), c->stream);
+      return set_err(c, PCSF_EINVAL, "FP64 kernel: tree workspace exceeds 64 KiB of LDS");
+    }
+  } else if (frag_format(precision) >= 0) {
+    e = launch_prune_mfma(m, b, precision, m->mfma_variant[precision], c->stream);
+  } else {
+    return set_err(c, PCSF_EINVAL, "pcsf_forward: unknown precision");
+  }
+  HIP_TRY(c, e);
+  if (c->timing) HIP_TRY(c, hipEventRecord(b->ev[1], c->stream));
+  if (precision == PCSF_FP64M) {
+    if (b->nreg > 0) HIP_TRY(c, launch_region_reduce_aligned(b, all, b->d_res, c->stream));
+  } else {
+    HIP_TRY(c, launch_region_reduce(b, c->stream));
+  }
+  if (c->timing) HIP_TRY(c, hipEventRecord(b->ev[2], c->stream));
+  return PCSF_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int pcsf_forward(pcsf_batch* b, const double* rho, int rho_per_region, int precision,
                  double* loglik, double* elpr, int save_for_backward) {
   if (!b || !rho) return PCSF_EINVAL;
@@ -1159,69 +1379,28 @@ int pcsf_forward(pcsf_batch* b, const double* rho, int rho_per_region, int preci
         return set_err(c, PCSF_EINVAL,
                        "CamlPaml.P14n.instantiate_tree: domain violation on variable 0");
     HIP_TRY(c, hipSetDevice(c->device));
-    int rc = forward_regions(b, rho, nullptr, precision);
+    int rc = forward_regions(b, rho, nullptr, precision, loglik, elpr);
     if (rc) return rc;
     b->last_rho.assign(rho, rho + nr);
     b->last_precision = precision;
-    if (loglik && nr)
-      HIP_TRY(c, hipMemcpyAsync(loglik, b->d_loglik, nr * 8, hipMemcpyDeviceToHost, c->stream));
-    if (elpr && nr)
-      HIP_TRY(c, hipMemcpyAsync(elpr, b->d_elpr, nr * 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
     return PCSF_OK;
   }
-  std::vector<double> r(rho, rho + m->nm);
-  for (double x : r)
-    if (!rho_valid(x))
+  for (int q = 0; q < m->nm; ++q)
+    if (!rho_valid(rho[q]))
       return set_err(c, PCSF_EINVAL,
                      "CamlPaml.P14n.instantiate_tree: domain violation on variable 0");
   HIP_TRY(c, hipSetDevice(c->device));
-  float tp = 0.f;
-  int rc = ensure_transitions(m, r.data(), frag_format(precision), set_outputs(precision), &tp);
+  const std::vector<double> r(rho, rho + m->nm);
+  int rc = shared_pass(b, r.data(), precision, !c->timing);
   if (rc) return rc;
-  if (precision == PCSF_FP64M && b->nreg > 0) {
-    // region-aligned columns, the model's sets for every region
-    if ((rc = ensure_aligned(b))) return rc;
-  }
-  b->t_pbuild = tp;
-  b->last_rho.resize((size_t)b->nreg * m->nm);
-  b->last_precision = precision;
-  for (int32_t i = 0; i < b->nreg; ++i)
-    for (int q = 0; q < m->nm; ++q) b->last_rho[(size_t)i * m->nm + q] = r[q];
-  if (c->timing) HIP_TRY(c, hipEventRecord(b->ev[0], c->stream));
-  hipError_t e;
-  RegionChunk all;
-  all.r0 = 0;
-  all.nreg = b->nreg;
-  all.block0 = 0;
-  all.nblocks = b->al.ld / kAlignCols;
-  all.sets = &m->fixed;
-  if (precision == PCSF_FP64M) {
-    e = b->nreg > 0 ? launch_forward_fp64m(m, b, all, c->stream) : hipSuccess;
-  } else if (precision == PCSF_FP64) {
-    e = launch_prune_fp64(m, b, c->stream);
-    if (e == hipErrorInvalidValue)
-      return set_err(c, PCSF_EINVAL, "FP64 kernel: tree workspace exceeds 64 KiB of LDS");
-  } else if (frag_format(precision) >= 0) {
-    e = launch_prune_mfma(m, b, precision, m->mfma_variant[precision], c->stream);
-  } else {
-    return set_err(c, PCSF_EINVAL, "pcsf_forward: unknown precision");
-  }
-  HIP_TRY(c, e);
-  if (c->timing) HIP_TRY(c, hipEventRecord(b->ev[1], c->stream));
-  if (precision == PCSF_FP64M) {
-    if (b->nreg > 0) HIP_TRY(c, launch_region_reduce_aligned(b, all, b->d_loglik, b->d_elpr,
-                                                              c->stream));
-  } else {
-    HIP_TRY(c, launch_region_reduce(b, c->stream));
-  }
-  if (c->timing) HIP_TRY(c, hipEventRecord(b->ev[2], c->stream));
   const size_t nres = (size_t)b->nreg * m->nm;
-  if (loglik && nres)
-    HIP_TRY(c, hipMemcpyAsync(loglik, b->d_loglik, nres * 8, hipMemcpyDeviceToHost, c->stream));
-  if (elpr && nres)
-    HIP_TRY(c, hipMemcpyAsync(elpr, b->d_elpr, nres * 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  rc = fetch_results(b, b->d_res, nres, {loglik, elpr}, !c->timing && b->nreg > 0, r.data(), false,
+                     "");
+  if (rc) {
+    m->cached_rho.clear();
+    m->built = 0;
+    return rc;
+  }
   if (c->timing) {
     HIP_TRY(c, hipEventElapsedTime(&b->t_prune, b->ev[0], b->ev[1]));
     HIP_TRY(c, hipEventElapsedTime(&b->t_reduce, b->ev[1], b->ev[2]));
@@ -1417,18 +1596,56 @@ struct PairState {
   }
 };
 
-// Evaluates lpr (and elpr) of every region and model at one shared tree scale.
-int eval_shared(pcsf_batch* b, double x, int precision, std::vector<double>& l,
-                std::vector<double>& e) {
+// Evaluates lpr (and elpr) of every region and model at K shared tree scales,
+// one wait for all of them where their results fit the pinned ring.
+int eval_shared(pcsf_batch* b, const double* x, int K, int precision, std::vector<double>* l,
+                std::vector<double>* e) {
   pcsf_model* m = b->m;
   pcsf_ctx* c = m->ctx;
-  std::vector<double> r(m->nm, x);
-  const size_t n = (size_t)b->nreg * m->nm;
-  l.assign(n, 0.0);
-  e.assign(n, 0.0);
-  int rc = pcsf_forward(b, r.data(), 0, precision, l.data(), e.data(), 0);
-  (void)c;
-  return rc;
+  const size_t n = (size_t)b->nreg * m->nm, count = 1 + 2 * n;
+  for (int k = 0; k < K; ++k) {
+    l[k].assign(n, 0.0);
+    e[k].assign(n, 0.0);
+  }
+  const size_t room = (size_t)K * (count * 8 + 256);
+  if (c->timing || n == 0 || !c->pin || room > c->pin_cap) {
+    for (int k = 0; k < K; ++k) {
+      const std::vector<double> r(m->nm, x[k]);
+      const int rc = pcsf_forward(b, r.data(), 0, precision, l[k].data(), e[k].data(), 0);
+      if (rc) return rc;
+    }
+    return PCSF_OK;
+  }
+  int rc0 = precision == PCSF_FP64M ? ensure_aligned(b) : PCSF_OK;  // (its uploads first)
+  if (rc0) return rc0;
+  // the ring must not wrap (and be reused) between these passes
+  if (c->pin_used + room > c->pin_cap) HIP_TRY(c, ctx_wait(c));
+  HIP_TRY(c, hipSetDevice(c->device));
+  std::vector<const double*> got(K);
+  for (int k = 0; k < K; ++k) {
+    const std::vector<double> r(m->nm, x[k]);
+    const int rc = shared_pass(b, r.data(), precision, true);
+    if (rc) return rc;
+    hipError_t he;
+    double* p = reinterpret_cast<double*>(pin_take(c, count * 8, &he));
+    HIP_TRY(c, he);
+    HIP_TRY(c, hipMemcpyAsync(p, b->d_res, count * 8, hipMemcpyDeviceToHost, c->stream));
+    got[k] = p;
+  }
+  HIP_TRY(c, ctx_wait(c));
+  for (int k = 0; k < K; ++k) {
+    unsigned long long key;
+    std::memcpy(&key, got[k], 8);
+    if (key != ~0ull) {
+      m->cached_rho.clear();
+      m->built = 0;
+      const std::vector<double> r(m->nm, x[k]);
+      return failed_build(m, key, r.data(), false);
+    }
+    std::memcpy(l[k].data(), got[k] + 1, n * 8);
+    std::memcpy(e[k].data(), got[k] + 1 + n, n * 8);
+  }
+  return PCSF_OK;
 }
 
 // The reference's maximize_lpr for every (region, model) pair at once
@@ -1437,20 +1654,19 @@ int eval_shared(pcsf_batch* b, double x, int precision, std::vector<double>& l,
 // within 1% of the estimate, then lpr at the estimate.
 int score_mle(pcsf_batch* b, int precision, std::vector<PairState>& st) {
   pcsf_model* m = b->m;
-  pcsf_ctx* c = m->ctx;
   const int nm = m->nm;
   const size_t np = (size_t)b->nreg * nm;
   const double lo = 1e-2, hi = 10.0, init = 1.0, accuracy = 0.01;
-  std::vector<double> Llo, Elo, Lhi, Ehi, L1, E1, Lv, Ev;
-  int rc;
-  if ((rc = eval_shared(b, lo, precision, Llo, Elo))) return rc;
-  if ((rc = eval_shared(b, hi, precision, Lhi, Ehi))) return rc;
-  if ((rc = eval_shared(b, init, precision, L1, E1))) return rc;
   pcsf::BrentMin probe;
   probe.x_lo = lo;
   probe.x_hi = hi;
   const double v = probe.golden_point();
-  if ((rc = eval_shared(b, v, precision, Lv, Ev))) return rc;
+  int rc;
+  std::vector<double> Ls[4], Es[4];
+  const double shared[4] = {lo, hi, init, v};
+  if ((rc = eval_shared(b, shared, 4, precision, Ls, Es))) return rc;
+  const std::vector<double>&Llo = Ls[0], &Elo = Es[0], &Lhi = Ls[1], &Ehi = Es[1], &L1 = Ls[2],
+                           &E1 = Es[2], &Lv = Ls[3], &Ev = Es[3];
   const std::vector<double> retries = pcsf::find_init_retries(lo, hi, 250);
   st.assign(np, PairState());
   auto start_brent = [&](PairState& s, size_t k) {
@@ -1521,11 +1737,8 @@ int score_mle(pcsf_batch* b, int precision, std::vector<PairState>& st) {
       any = any || act[k];
     }
     if (!any) break;
-    rc = forward_regions(b, rho.data(), act.data(), precision);
+    rc = forward_regions(b, rho.data(), act.data(), precision, L.data(), E.data());
     if (rc) return rc;
-    HIP_TRY(c, hipMemcpyAsync(L.data(), b->d_loglik, np * 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(E.data(), b->d_elpr, np * 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
     for (size_t k = 0; k < np; ++k) {
       if (!act[k]) continue;
       PairState& s = st[k];
@@ -1585,10 +1798,8 @@ int score_mle(pcsf_batch* b, int precision, std::vector<PairState>& st) {
       act[k] = st[k].status == PCSF_OK;
       rho[k] = act[k] ? st[k].res_x : 1.0;
     }
-    rc = forward_regions(b, rho.data(), act.data(), PCSF_FP64M);
+    rc = forward_regions(b, rho.data(), act.data(), PCSF_FP64M, L.data(), E.data());
     if (rc) return rc;
-    HIP_TRY(c, hipMemcpy(L.data(), b->d_loglik, np * 8, hipMemcpyDeviceToHost));
-    HIP_TRY(c, hipMemcpy(E.data(), b->d_elpr, np * 8, hipMemcpyDeviceToHost));
     for (size_t k = 0; k < np; ++k)
       if (act[k]) {
         st[k].res_lpr = L[k];
@@ -1610,7 +1821,6 @@ int score_mle(pcsf_batch* b, int precision, std::vector<PairState>& st) {
 // launches of pair k, the final forward included.
 int score_mle_grad(pcsf_batch* b, int precision, std::vector<PairState>& st) {
   pcsf_model* m = b->m;
-  pcsf_ctx* c = m->ctx;
   const size_t np = (size_t)b->nreg * m->nm;
   const double xlo = std::log(1e-2), xhi = std::log(10.0);
   // ln rho tolerance: lpr is flat to second order at the maximum, so an
@@ -1659,14 +1869,14 @@ int score_mle_grad(pcsf_batch* b, int precision, std::vector<PairState>& st) {
   {
     constexpr int K = 7;
     const double grid[K] = {-2.0, -1.2, -0.6, 0.0, 0.6, 1.2, 2.0};
-    std::vector<double> Lk[K], e;
+    std::vector<double> Lk[K], Ek[K];
     // FP64 evaluates the grid on the matrix cores (the plain kernel is the
     // slow one; both are FP64)
     const int gp = (precision == PCSF_FP64) ? PCSF_FP64M : precision;
-    for (int k = 0; k < K; ++k) {
-      const int rc = eval_shared(b, std::exp(grid[k]), gp, Lk[k], e);
-      if (rc) return rc;
-    }
+    double scale[K];
+    for (int k = 0; k < K; ++k) scale[k] = std::exp(grid[k]);
+    const int rc = eval_shared(b, scale, K, gp, Lk, Ek);
+    if (rc) return rc;
     for (size_t q = 0; q < np; ++q) {
       st[q].evals += K;
       int best = 0;
@@ -1737,12 +1947,8 @@ int score_mle_grad(pcsf_batch* b, int precision, std::vector<PairState>& st) {
   std::vector<uint8_t> act(np, 1);
   auto eval = [&]() -> int {
     // FP64: the outside-pass adjoint; MFMA precisions: the FP32 tangent pass
-    int rc = adjoint_regions(b, rho.data(), act.data(), nullptr, !fp64_precision(precision));
-    if (rc) return rc;
-    HIP_TRY(c, hipMemcpy(L.data(), b->d_gloglik, np * 8, hipMemcpyDeviceToHost));
-    HIP_TRY(c, hipMemcpy(D.data(), b->d_grad, np * 8, hipMemcpyDeviceToHost));
-    HIP_TRY(c, hipMemcpy(S.data(), b->d_gsq, np * 8, hipMemcpyDeviceToHost));
-    return PCSF_OK;
+    return adjoint_regions(b, rho.data(), act.data(), nullptr, !fp64_precision(precision),
+                           L.data(), D.data(), S.data());
   };
   for (int it = 0; it < 100; ++it) {
     bool any = false;
@@ -1867,10 +2073,8 @@ int score_mle_grad(pcsf_batch* b, int precision, std::vector<PairState>& st) {
   // of a few thousand codons, ~3e-3 dB) would otherwise reach the score
   for (size_t k = 0; k < np; ++k) rho[k] = std::exp(g[k].x);
   std::vector<uint8_t> all(np, 1);
-  int rc = forward_regions(b, rho.data(), all.data(), PCSF_FP64M);
+  int rc = forward_regions(b, rho.data(), all.data(), PCSF_FP64M, L.data(), D.data());
   if (rc) return rc;
-  HIP_TRY(c, hipMemcpy(L.data(), b->d_loglik, np * 8, hipMemcpyDeviceToHost));
-  HIP_TRY(c, hipMemcpy(D.data(), b->d_elpr, np * 8, hipMemcpyDeviceToHost));
   for (size_t k = 0; k < np; ++k) {
     st[k].res_x = rho[k];
     st[k].res_lpr = L[k];
@@ -1903,7 +2107,6 @@ struct OmegaPair {
 int score_omega(pcsf_batch* b, int precision, double omega_h1, double sigma_h1,
                 std::vector<OmegaPair>& st) {
   pcsf_model* m = b->m;
-  pcsf_ctx* c = m->ctx;
   const int R = b->nreg;
   const size_t np = (size_t)R * 2;
   const double rel_tol = fp64_precision(precision) ? 1.4901161193847656e-08 : 1e-5;
@@ -1960,9 +2163,8 @@ int score_omega(pcsf_batch* b, int precision, double omega_h1, double sigma_h1,
       any = true;
     }
     if (!any) break;
-    rc = forward_regions(b, rho.data(), act.data(), precision, &sm);
+    rc = forward_regions(b, rho.data(), act.data(), precision, L.data(), nullptr, &sm);
     if (rc) return rc;
-    HIP_TRY(c, hipMemcpy(L.data(), b->d_loglik, np * 8, hipMemcpyDeviceToHost));
     for (size_t k = 0; k < np; ++k) {
       if (!act[k]) continue;
       OmegaPair& p = st[k];
@@ -2019,9 +2221,8 @@ int score_omega(pcsf_batch* b, int precision, double omega_h1, double sigma_h1,
         act[k] = 0;
       }
     }
-    rc = forward_regions(b, rho.data(), act.data(), PCSF_FP64M, &sm);
+    rc = forward_regions(b, rho.data(), act.data(), PCSF_FP64M, L.data(), nullptr, &sm);
     if (rc) return rc;
-    HIP_TRY(c, hipMemcpy(L.data(), b->d_loglik, np * 8, hipMemcpyDeviceToHost));
     for (size_t k = 0; k < np; ++k)
       if (act[k]) {
         st[k].lpr = pcsf::omega_lpr_kappa(st[k].kappa) + L[k];
@@ -2131,20 +2332,18 @@ int pcsf_backward(pcsf_batch* b, const double* grad_loglik, double* grad_rho,
   double* d_gbr = nullptr;
   const size_t ngb = np * m->nbr;
   if (grad_branch && ngb) {
-    HIP_TRY(c, dalloc(&d_gbr, ngb));
+    HIP_TRY(c, dalloc(c, &d_gbr, ngb));
     HIP_TRY(c, hipMemsetAsync(d_gbr, 0, ngb * 8, c->stream));
   }
   // an MFMA-precision forward without per-branch gradients is differentiated
   // by the FP32 tangent pass; everything else by the FP64 outside pass
   const bool tangent = !fp64_precision(b->last_precision) && !d_gbr;
-  int rc = adjoint_regions(b, b->last_rho.data(), nullptr, d_gbr, tangent);
   std::vector<double> dl(np), gb;
-  if (!rc && np) {
-    hipError_t e = hipMemcpy(dl.data(), b->d_grad, np * 8, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && d_gbr) {
-      gb.resize(ngb);
-      e = hipMemcpy(gb.data(), d_gbr, ngb * 8, hipMemcpyDeviceToHost);
-    }
+  int rc = adjoint_regions(b, b->last_rho.data(), nullptr, d_gbr, tangent, nullptr, dl.data(),
+                           nullptr);
+  if (!rc && np && d_gbr) {
+    gb.resize(ngb);
+    const hipError_t e = hipMemcpy(gb.data(), d_gbr, ngb * 8, hipMemcpyDeviceToHost);
     if (e != hipSuccess) rc = set_err(c, PCSF_EDEVICE, hipGetErrorString(e));
   }
   dfree(d_gbr);
@@ -2204,8 +2403,8 @@ hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk, int grid)
     dfree(es.U);
     dfree(es.V);
     es.cap_uv = 0;
-    e = dalloc(&es.U, uv);
-    if (e == hipSuccess) e = dalloc(&es.V, uv);
+    e = dalloc(c, &es.U, uv);
+    if (e == hipSuccess) e = dalloc(c, &es.V, uv);
     if (e != hipSuccess) {
       dfree(es.U);
       dfree(es.V);
@@ -2217,7 +2416,7 @@ hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk, int grid)
   if (es.cap_scr < scr) {
     dfree(es.scr);
     es.cap_scr = 0;
-    if ((e = dalloc(&es.scr, scr)) != hipSuccess) return e;
+    if ((e = dalloc(c, &es.scr, scr)) != hipSuccess) return e;
     es.cap_scr = scr;
   }
   const size_t lv = (size_t)chunk * nl;
@@ -2229,10 +2428,12 @@ hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk, int grid)
     }
     es.cap_leaves = 0;
     for (int i = 0; i < 2 && e == hipSuccess; ++i) {
-      e = dalloc(&es.leaves[i], lv);
+      e = dalloc(c, &es.leaves[i], lv);
       if (e == hipSuccess)
         e = hipHostMalloc(reinterpret_cast<void**>(&es.staged[i]), lv * 4, hipHostMallocDefault);
     }
+    // the copy stream fills the slots; what used this memory before ran here
+    if (e == hipSuccess) e = ctx_wait(c);
     if (e != hipSuccess) {
       for (int i = 0; i < 2; ++i) {
         dfree(es.leaves[i]);
@@ -2271,17 +2472,17 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
   };
   chk(estep_cache(c, n, ldu, chunk, grid));
   EstepCache& es = c->es;
-  chk(dalloc(&d_lc, (size_t)n));
-  chk(dalloc(&d_rc, (size_t)n));
-  chk(dalloc(&d_P, (size_t)nbr * 4096));
-  chk(dalloc(&d_Pf, (size_t)nbr * 4096));
-  chk(dalloc(&d_PTf, (size_t)nbr * 4096));
-  chk(dalloc(&d_seq, std::max<size_t>(1, seq.size())));
-  chk(dalloc(&d_rs, (size_t)nbr * 64));
-  chk(dalloc(&d_prior, 64));
-  if (weights) chk(dalloc(&d_w, (size_t)ncols));
-  chk(dalloc(&d_z, (size_t)ncols));
-  chk(dalloc(&d_ec, (size_t)nbr * 4096));
+  chk(dalloc(c, &d_lc, (size_t)n));
+  chk(dalloc(c, &d_rc, (size_t)n));
+  chk(dalloc(c, &d_P, (size_t)nbr * 4096));
+  chk(dalloc(c, &d_Pf, (size_t)nbr * 4096));
+  chk(dalloc(c, &d_PTf, (size_t)nbr * 4096));
+  chk(dalloc(c, &d_seq, std::max<size_t>(1, seq.size())));
+  chk(dalloc(c, &d_rs, (size_t)nbr * 64));
+  chk(dalloc(c, &d_prior, 64));
+  if (weights) chk(dalloc(c, &d_w, (size_t)ncols));
+  chk(dalloc(c, &d_z, (size_t)ncols));
+  chk(dalloc(c, &d_ec, (size_t)nbr * 4096));
   auto up = [&](void* dst, const void* src, size_t bytes) {
     if (e == hipSuccess && bytes) e = hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
   };
@@ -2413,22 +2614,22 @@ int lik_impl(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P
     if (e == hipSuccess) e = x;
   };
   const int64_t cmax = std::min(ncols, chunk);
-  chk(dalloc(&d_lc, (size_t)n));
-  chk(dalloc(&d_rc, (size_t)n));
-  chk(dalloc(&d_par, (size_t)n));
-  chk(dalloc(&d_sib, (size_t)n));
-  chk(dalloc(&d_P, (size_t)(n - 1) * k * k));
-  chk(dalloc(&d_prior, (size_t)k));
-  chk(dalloc(&d_leaves, (size_t)cmax * nl));
-  if (dist) chk(dalloc(&d_dist, (size_t)cmax * nl * k));
-  if (weights) chk(dalloc(&d_w, (size_t)cmax));
-  chk(dalloc(&d_z, (size_t)cmax));
-  if (post_mode) chk(dalloc(&d_post, (size_t)cmax * (post_mode == 2 ? n : 1) * k));
-  chk(dalloc(&d_ws, (size_t)grid_max * 2 * n * k));
+  chk(dalloc(c, &d_lc, (size_t)n));
+  chk(dalloc(c, &d_rc, (size_t)n));
+  chk(dalloc(c, &d_par, (size_t)n));
+  chk(dalloc(c, &d_sib, (size_t)n));
+  chk(dalloc(c, &d_P, (size_t)(n - 1) * k * k));
+  chk(dalloc(c, &d_prior, (size_t)k));
+  chk(dalloc(c, &d_leaves, (size_t)cmax * nl));
+  if (dist) chk(dalloc(c, &d_dist, (size_t)cmax * nl * k));
+  if (weights) chk(dalloc(c, &d_w, (size_t)cmax));
+  chk(dalloc(c, &d_z, (size_t)cmax));
+  if (post_mode) chk(dalloc(c, &d_post, (size_t)cmax * (post_mode == 2 ? n : 1) * k));
+  chk(dalloc(c, &d_ws, (size_t)grid_max * 2 * n * k));
   if (estep) {
-    chk(dalloc(&d_U, (size_t)(n - 1) * grid_max * k));
-    chk(dalloc(&d_V, (size_t)(n - 1) * grid_max * k));
-    chk(dalloc(&d_ec, (size_t)(n - 1) * k * k));
+    chk(dalloc(c, &d_U, (size_t)(n - 1) * grid_max * k));
+    chk(dalloc(c, &d_V, (size_t)(n - 1) * grid_max * k));
+    chk(dalloc(c, &d_ec, (size_t)(n - 1) * k * k));
   }
   auto up = [&](void* dst, const void* src, size_t bytes) {
     if (e == hipSuccess && bytes) e = hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);

@@ -35,7 +35,7 @@ int frag_format(int precision);  // -1 for a precision without MFMA tiles
 struct PSets {
   int cap = 0;                 // sets allocated
   int fmt = -1;                // format of d_Pfrag as last built
-  bool fp64 = false;           // P64T and P64F allocated
+  unsigned outputs = 0;        // kBuild* outputs allocated
   double* d_P64T = nullptr;    // cap * nbr * 4096 FP64 P^T (P64T[b][a] = P[a][b])
   double* d_P64F = nullptr;    // cap * nbr * kTile64 FP64 P for the matrix-core forward:
                                //   an internal branch's P in v_mfma_f64_16x16x4f64
@@ -50,8 +50,13 @@ struct PSets {
   // tangent data (allocated on request): D = dP/drho = b Q P(rho b)
   float* d_DT32 = nullptr;     // cap * nbr * 65 * 64: row c < 64 D[a][c] / P[c][c], row 64 0
   float* d_Dfrag = nullptr;    // cap * nbr * 4096: D in the FP32 A-operand order
-  double* d_rho = nullptr;     // cap tree scales
-  uint8_t* d_active = nullptr; // cap flags: 0 = set not needed by this launch
+  // a pass's parameters in one piece (one upload); the pointers below into it
+  // are those of the last pass
+  uint8_t* d_params = nullptr;
+  double* d_rho = nullptr;     // tree scales
+  uint8_t* d_active = nullptr; // flags: 0 = set not needed by this launch
+  double* d_qs = nullptr;      // twelve omega settings per set (own rate models only)
+  uint8_t* d_mode = nullptr;   // kEigCold / kEigWarm / kEigKeep per set (likewise)
   // cherry tables (fixed scales only): message P_c (P_a[:,x] o P_b[:,y]) of
   // cherry c above its two leaves a, b, normalised to max 1, and its ln max
   float* d_ctab = nullptr;     // cap * nctab * 65 * 65 * 64
@@ -64,6 +69,7 @@ struct PSets {
   double* d_elam = nullptr;    // cap * 64
   double* d_epi = nullptr;     // cap * 64 root prior
   double* d_elnpi = nullptr;   // cap * 64 its logarithm
+  double* d_eref = nullptr;    // cap * 4096 the reference basis of its warm starts
 };
 
 // Device and pinned buffers of the E-step (capi.hip estep_mfma), kept by the
@@ -86,6 +92,9 @@ struct pcsf_ctx {
   std::string err;
   bool timing = false;
   int num_cus = 256;
+  uint64_t pool_id = 0;      // the device memory it keeps (devpool.hpp)
+  uint8_t* pin = nullptr;    // pinned host ring for small uploads and results
+  size_t pin_cap = 0, pin_used = 0;
   EstepCache es;
 };
 
@@ -161,8 +170,10 @@ struct pcsf_batch {
   int64_t* d_offsets = nullptr;    // nreg + 1
   double* d_logz = nullptr;        // nm * ld
   double* d_colelpr = nullptr;     // nm * ld
-  double* d_loglik = nullptr;      // nreg * nm
-  double* d_elpr = nullptr;        // nreg * nm
+  // the P builder's failure record, then loglik and elpr (nreg * nm each)
+  double* d_res = nullptr;
+  double* d_loglik = nullptr;      // nreg * nm (in d_res)
+  double* d_elpr = nullptr;        // nreg * nm (in d_res)
   hipEvent_t ev[6] = {};
   float t_pbuild = 0, t_prune = 0, t_reduce = 0;
   std::vector<int64_t> offsets;     // host copy
@@ -172,17 +183,13 @@ struct pcsf_batch {
   PSets rs;                         // per-region transition sets (one chunk)
   double* d_alogz = nullptr;        // nm * al.ld, per aligned column
   double* d_acolelpr = nullptr;
-  // gradient passes (pcsf_backward, mle_grad) reduce into these, so that the
-  // last forward's d_loglik / d_elpr stay as they were
-  double* d_gloglik = nullptr;      // nreg * nm: lpr at the differentiated scales
-  double* d_grad = nullptr;         // nreg * nm: d lpr / d rho
-  double* d_gsq = nullptr;          // nreg * nm: sum over columns of (d ln z / d rho)^2
+  // gradient passes (pcsf_backward, mle_grad) reduce into their own piece, so
+  // that the last forward's d_loglik / d_elpr stay as they were: the failure
+  // record, then per pair lpr at the differentiated scales, d lpr / d rho and
+  // the sum over columns of (d ln z / d rho)^2
+  double* d_gres = nullptr;
   double* d_adj_scratch = nullptr;  // FP64 outside pass: node tiles per resident wave
   size_t adj_scratch = 0;           // its size in doubles
-  double* d_setqs = nullptr;        // per-set model settings of a chunk (omega test)
-  size_t setqs_cap = 0;             // its size in doubles
-  uint8_t* d_eigmode = nullptr;     // per set: kEigCold / kEigWarm / kEigKeep
-  double* d_eigref = nullptr;       // per set: the reference basis of its warm starts
   // the settings each set of `rs` was last built from and those of its
   // reference basis (host), valid while a pass fits in one chunk (set k is
   // pair k) and `rs` is not reallocated
@@ -269,22 +276,21 @@ hipError_t launch_adjoint_mfma(const pcsf_model* m, const pcsf_batch* b, const R
 hipError_t launch_forward_fp64m(const pcsf_model* m, const pcsf_batch* b, const RegionChunk& ch,
                                 hipStream_t s);
 // the omega test's rate model of every active set of a chunk from its twelve
-// settings (d_qs: nsets * 12): eigensystem and root prior into the sets'
-// own-model arrays
+// settings (PSets::d_qs): eigensystem and root prior into the sets' own-model
+// arrays
 // Per-set modes of launch_omega_eigen: build from scratch (and store the
-// eigenvectors as the set's reference basis in d_ref, 4096 doubles a set),
+// eigenvectors as the set's reference basis in d_eref, 4096 doubles a set),
 // start from that basis (same pi), or keep the outputs.
 constexpr uint8_t kEigCold = 0, kEigWarm = 1, kEigKeep = 2;
-hipError_t launch_omega_eigen(const double* d_qs, const uint8_t* d_mode, double* d_ref,
-                              int nsets, const PSets& sets, hipStream_t s);
+hipError_t launch_omega_eigen(int nsets, const PSets& sets, hipStream_t s);
 hipError_t launch_prune_tangent_regions(const pcsf_model* m, const pcsf_batch* b,
                                         const RegionChunk& ch, hipStream_t s);
-// sums over each region of the chunk into loglik / elpr (nreg * nm)
-// (sq, optional: the sums of the squared per-column second values -- with
-// d ln z / d rho there, the outer-product estimate of lpr's curvature)
-hipError_t launch_region_reduce_aligned(const pcsf_batch* b, const RegionChunk& ch,
-                                        double* loglik, double* elpr, hipStream_t s,
-                                        double* sq = nullptr);
+// sums over each region of the chunk into res, the batch's d_res or d_gres:
+// a copy of the P builder's failure record, loglik, elpr and, in d_gres, the
+// sums of the squared per-column second values (with d ln z / d rho there,
+// the outer-product estimate of lpr's curvature)
+hipError_t launch_region_reduce_aligned(const pcsf_batch* b, const RegionChunk& ch, double* res,
+                                        hipStream_t s);
 // Launch shapes of the fused kernel that the autotuner chooses among.
 struct MfmaVariant {
   int wpg;        // waves per workgroup (16 columns each) sharing one LDS P tile

@@ -45,9 +45,11 @@ __global__ void transpose_codes_kernel(const uint8_t* __restrict__ src, int64_t 
 __global__ __launch_bounds__(256) void region_reduce_kernel(
     const double* __restrict__ logz, const double* __restrict__ colelpr,
     const int64_t* __restrict__ off, int nm, int64_t ld, double* __restrict__ loglik,
-    double* __restrict__ elpr) {
+    double* __restrict__ elpr, const unsigned long long* __restrict__ perr,
+    double* __restrict__ head) {
   __shared__ double s0[256], s1[256];
   const int r = blockIdx.x, q = blockIdx.y, tid = threadIdx.x;
+  if (head && r == 0 && q == 0 && tid == 0) *head = __longlong_as_double((long long)*perr);
   const int64_t lo = off[r], hi = off[r + 1];
   double a = 0.0, b = 0.0;
   for (int64_t c = lo + tid; c < hi; c += 256) {
@@ -94,9 +96,12 @@ __global__ __launch_bounds__(256) void region_reduce_aligned_kernel(
     const double* __restrict__ logz, const double* __restrict__ colelpr,
     const int64_t* __restrict__ off, const int64_t* __restrict__ astart,
     const uint8_t* __restrict__ active, int r0, int nm, int64_t ald,
-    double* __restrict__ loglik, double* __restrict__ elpr, double* __restrict__ sq) {
+    double* __restrict__ loglik, double* __restrict__ elpr, double* __restrict__ sq,
+    const unsigned long long* __restrict__ perr, double* __restrict__ head) {
   __shared__ double s0[256], s1[256], s2[256];
   const int r = r0 + blockIdx.x, q = blockIdx.y, tid = threadIdx.x;
+  // the failure record of the pass's P build travels with its results
+  if (blockIdx.x == 0 && q == 0 && tid == 0) *head = __longlong_as_double((long long)*perr);
   if (active && !active[(size_t)blockIdx.x * nm + q]) return;
   const int64_t lo = astart[r], hi = lo + (off[r + 1] - off[r]);
   double a = 0.0, b = 0.0, d = 0.0;
@@ -136,16 +141,17 @@ hipError_t launch_align_codes(const pcsf_batch* b, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_region_reduce_aligned(const pcsf_batch* b, const RegionChunk& ch,
-                                        double* loglik, double* elpr, hipStream_t s,
-                                        double* sq) {
+hipError_t launch_region_reduce_aligned(const pcsf_batch* b, const RegionChunk& ch, double* res,
+                                        hipStream_t s) {
   if (ch.nreg == 0) return hipSuccess;
+  const size_t np = (size_t)b->nreg * b->m->nm;
   dim3 grid(ch.nreg, b->m->nm);
   // the model's own sets (one per model, shared by every region) are all live
   const uint8_t* active = (ch.sets == &b->m->fixed) ? nullptr : ch.sets->d_active;
   hipLaunchKernelGGL(region_reduce_aligned_kernel, grid, dim3(256), 0, s, b->d_alogz,
                      b->d_acolelpr, b->d_offsets, b->al.d_astart, active, ch.r0,
-                     b->m->nm, b->al.ld, loglik, elpr, sq);
+                     b->m->nm, b->al.ld, res + 1, res + 1 + np,
+                     res == b->d_gres ? res + 1 + 2 * np : nullptr, b->m->d_perr, res);
   return hipGetLastError();
 }
 
@@ -230,6 +236,6 @@ hipError_t launch_region_reduce(const pcsf_batch* b, hipStream_t s) {
   if (b->nreg == 0) return hipSuccess;
   dim3 grid(b->nreg, b->m->nm);
   hipLaunchKernelGGL(region_reduce_kernel, grid, dim3(256), 0, s, b->d_logz, b->d_colelpr,
-                     b->d_offsets, b->m->nm, b->ld, b->d_loglik, b->d_elpr);
+                     b->d_offsets, b->m->nm, b->ld, b->d_loglik, b->d_elpr, b->m->d_perr, b->d_res);
   return hipGetLastError();
 }

@@ -283,10 +283,9 @@ __global__ __launch_bounds__(256) void omega_eigen_kernel(
 
 }  // namespace
 
-hipError_t launch_omega_eigen(const double* d_qs, const uint8_t* d_mode, double* d_ref,
-                              int nsets, const PSets& sets, hipStream_t s) {
+hipError_t launch_omega_eigen(int nsets, const PSets& sets, hipStream_t s) {
   if (nsets <= 0) return hipSuccess;
-  hipLaunchKernelGGL(omega_eigen_kernel, dim3(nsets), dim3(256), 0, s, d_qs, d_mode, d_ref,
+  hipLaunchKernelGGL(omega_eigen_kernel, dim3(nsets), dim3(256), 0, s, sets.d_qs, sets.d_mode, sets.d_eref,
                      sets.d_eVT, sets.d_eVinv, sets.d_elam, sets.d_epi, sets.d_elnpi);
   return hipGetLastError();
 }

@@ -448,10 +448,10 @@ hipError_t launch_cherry_tables(const pcsf_model* m, const PSets& sets, int nset
 hipError_t launch_pbuild(const pcsf_model* m, const PSets& sets, int nsets, int fmt,
                          unsigned outputs, hipStream_t s) {
   if (nsets <= 0) return hipSuccess;
-  const bool p64 = (outputs & kBuildP64) && sets.fp64;
-  const bool p64m = (outputs & kBuildP64M) && sets.fp64;
-  const bool p64mt = (outputs & kBuildP64MT) && sets.fp64;
-  const bool mfma = (outputs & kBuildMfma) != 0;
+  const bool p64 = (outputs & kBuildP64) && sets.d_P64T;
+  const bool p64m = (outputs & kBuildP64M) && sets.d_P64F;
+  const bool p64mt = (outputs & kBuildP64MT) && sets.d_P64FT;
+  const bool mfma = (outputs & kBuildMfma) && sets.d_Pfrag;
   const bool tangent = (outputs & kBuildTangent) && sets.d_Dfrag;
   // several branches per workgroup once there are enough matrices to fill
   // the device; one each for the few sets of a fixed-strategy model
