@@ -2563,9 +2563,89 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
   return PCSF_OK;
 }
 
+// Likelihoods and root posteriors for small alphabets (lik_small_kernel): one
+// upload of the states and one launch per chunk.  Without leaf_dist the kernel
+// checks the states (*bad_state: one is below -1; nothing is written then).
+hipError_t lik_small(pcsf_ctx* c, int k, int n, const std::vector<int32_t>& lc,
+                     const std::vector<int32_t>& rc, const double* P, const double* prior,
+                     const int32_t* leaves, const double* leaf_dist, int64_t ncols, double* z,
+                     double* post, bool* bad_state) {
+  const int nl = (n + 1) / 2, K = lik_small_states(k);
+  std::vector<double> pad((size_t)(n - 1) * K * K + K, 0.0);
+  for (int br = 0; br < n - 1; ++br)
+    for (int a = 0; a < k; ++a)
+      std::copy(P + ((size_t)br * k + a) * k, P + ((size_t)br * k + a + 1) * k,
+                pad.begin() + ((size_t)br * K + a) * K);
+  std::copy(prior, prior + k, pad.end() - K);
+  const size_t per_col = (size_t)nl * 4 + (leaf_dist ? (size_t)nl * k * 8 : 0) + 8 + (size_t)k * 8;
+  const int64_t chunk = std::min<int64_t>(
+      ncols, std::max<int64_t>(64, (int64_t)(((size_t)512 << 20) / per_col) / 64 * 64));
+  const int grid = (int)std::min<int64_t>((chunk + 63) / 64, 4096);
+  int32_t *d_tree = nullptr, *d_leaves = nullptr, *d_bad = nullptr;
+  double *d_P = nullptr, *d_dist = nullptr, *d_out = nullptr, *d_ws = nullptr;
+  hipError_t e = hipSuccess;
+  auto chk = [&](hipError_t x) {
+    if (e == hipSuccess) e = x;
+  };
+  chk(dalloc(c, &d_tree, (size_t)2 * n));
+  chk(dalloc(c, &d_bad, 1));
+  chk(dalloc(c, &d_P, pad.size()));
+  chk(dalloc(c, &d_leaves, (size_t)chunk * nl));
+  if (leaf_dist) chk(dalloc(c, &d_dist, (size_t)chunk * nl * k));
+  chk(dalloc(c, &d_out, (size_t)chunk * (1 + k)));
+  chk(dalloc(c, &d_ws, (size_t)grid * (n - nl) * K * 64));
+  if (e == hipSuccess) chk(upload(c, d_tree, lc.data(), (size_t)n * 4));
+  if (e == hipSuccess) chk(upload(c, d_tree + n, rc.data(), (size_t)n * 4));
+  if (e == hipSuccess) chk(upload(c, d_P, pad.data(), pad.size() * 8));
+  if (e == hipSuccess) chk(hipMemsetAsync(d_bad, 0, 4, c->stream));
+  int bad = 0;
+  for (int64_t c0 = 0; c0 < ncols && e == hipSuccess && !bad; c0 += chunk) {
+    const int64_t nc = std::min(chunk, ncols - c0);
+    LikArgs a;
+    a.k = k;
+    a.n = n;
+    a.lc = d_tree;
+    a.rc = d_tree + n;
+    a.P = d_P;
+    a.prior = d_P + (pad.size() - K);
+    a.leaves = d_leaves;
+    a.leaf_dist = d_dist;
+    a.ncols = nc;
+    a.ws = d_ws;
+    a.z = d_out;
+    a.post_mode = post ? 1 : 0;
+    a.post = d_out + nc;
+    chk(hipMemcpyAsync(d_leaves, leaves + c0 * nl, (size_t)nc * nl * 4, hipMemcpyHostToDevice,
+                       c->stream));
+    if (leaf_dist)
+      chk(hipMemcpyAsync(d_dist, leaf_dist + (size_t)c0 * nl * k, (size_t)nc * nl * k * 8,
+                         hipMemcpyHostToDevice, c->stream));
+    if (e == hipSuccess)
+      e = launch_lik_small(a, (int)std::min<int64_t>((nc + 63) / 64, grid), d_bad, c->stream);
+    chk(hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, c->stream));
+    chk(ctx_wait(c));
+    if (e != hipSuccess || bad) break;
+    chk(hipMemcpyAsync(z + c0, d_out, (size_t)nc * 8, hipMemcpyDeviceToHost, c->stream));
+    if (post)
+      chk(hipMemcpyAsync(post + (size_t)c0 * k, d_out + nc, (size_t)nc * k * 8,
+                         hipMemcpyDeviceToHost, c->stream));
+    chk(ctx_wait(c));
+  }
+  *bad_state = bad != 0;
+  dfree(d_tree);
+  dfree(d_bad);
+  dfree(d_P);
+  dfree(d_leaves);
+  dfree(d_dist);
+  dfree(d_out);
+  dfree(d_ws);
+  return e;
+}
+
 int lik_impl(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P,
              const double* prior, const int32_t* leaves, const double* leaf_dist, int64_t ncols,
-             const double* weights, double* z, int post_mode, double* post, double* ecounts) {
+             const double* weights, double* z, int post_mode, double* post, double* ecounts,
+             bool columns_entry) {
   if (!c) return PCSF_EINVAL;
   if (k < 1 || k > 64 || n < 3 || n % 2 == 0 || !children || !P || !prior || !z ||
       (ncols > 0 && !leaves) || ncols < 0)
@@ -2582,6 +2662,19 @@ int lik_impl(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P
     sib[a] = b;
     sib[b] = a;
   }
+  const bool small = lik_small_states(k) > 0 && !ecounts && post_mode != 2 && ncols > 0;
+  double* root_post = post_mode == 1 ? post : nullptr;
+  if (small && columns_entry) {  // its kernel checks the states
+    HIP_TRY(c, hipSetDevice(c->device));
+    bool bad = false;
+    HIP_TRY(c, lik_small(c, k, n, lc, rc, P, prior, leaves, nullptr, ncols, z, root_post, &bad));
+    if (bad) return set_err(c, PCSF_EINVAL, "CamlPaml.Infer.prepare: leaf state out of range");
+    return PCSF_OK;
+  }
+  if (columns_entry)  // that entry takes `Certain and `Marginalize leaves only
+    for (int64_t e = 0; e < ncols * nl; ++e)
+      if (leaves[e] < -1)
+        return set_err(c, PCSF_EINVAL, "CamlPaml.Infer.prepare: leaf state out of range");
   // a state >= k is a leaf vector of zeros, as raw_leaf makes it
   // (PhyloLik.ml:11); below -2 is no leaf kind.  One branch-free pass (it
   // vectorises) over what can be a few hundred MB of states.
@@ -2597,6 +2690,12 @@ int lik_impl(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P
     return set_err(c, PCSF_EINVAL, "CamlPaml.Infer.prepare: `Distribution leaves need leaf_dist");
   if (ncols == 0) return PCSF_OK;
   HIP_TRY(c, hipSetDevice(c->device));
+  if (small) {
+    bool bad = false;
+    HIP_TRY(c, lik_small(c, k, n, lc, rc, P, prior, leaves, dist ? leaf_dist : nullptr, ncols, z,
+                         root_post, &bad));
+    return PCSF_OK;
+  }
   const bool estep = ecounts != nullptr;
   if (estep && k == 64 && !dist && post_mode == 0)
     return estep_mfma(c, n, lc, rc, P, prior, leaves, ncols, weights, z, ecounts);
@@ -2698,13 +2797,8 @@ extern "C" {
 int pcsf_lik_columns(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P,
                      const double* prior, const int32_t* leaves, int64_t ncols, double* z,
                      double* root_post) {
-  if (!c) return PCSF_EINVAL;
-  if (leaves)  // this entry takes `Certain and `Marginalize leaves only
-    for (int64_t e = 0; e < ncols * ((n + 1) / 2); ++e)
-      if (leaves[e] < -1)
-        return set_err(c, PCSF_EINVAL, "CamlPaml.Infer.prepare: leaf state out of range");
   return lik_impl(c, k, n, children, P, prior, leaves, nullptr, ncols, nullptr, z,
-                  root_post ? 1 : 0, root_post, nullptr);
+                  root_post ? 1 : 0, root_post, nullptr, true);
 }
 
 int pcsf_lik_posteriors(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P,
@@ -2712,7 +2806,7 @@ int pcsf_lik_posteriors(pcsf_ctx* c, int k, int n, const int32_t* children, cons
                         int64_t ncols, const double* weights, double* z, double* node_post,
                         double* ecounts) {
   return lik_impl(c, k, n, children, P, prior, leaves, leaf_dist, ncols, weights, z,
-                  node_post ? 2 : 0, node_post, ecounts);
+                  node_post ? 2 : 0, node_post, ecounts, false);
 }
 
 }  // extern "C"

@@ -326,6 +326,12 @@ struct LikArgs {
   double* V = nullptr;
   double* ecounts = nullptr;        // (n-1) x k x k, added to
 };
+// Likelihoods and root posteriors (post_mode 0 or 1, no U) for k <= 24: P and
+// prior padded with zeros to lik_small_states(k) states (0: k is too large), ws
+// for grid x (n - nl) x states x 64; *bad is set by a state below -1 without
+// leaf_dist.
+int lik_small_states(int k);
+hipError_t launch_lik_small(const LikArgs& a, int grid, int* bad, hipStream_t s);
 // grid workgroups; with U set, ncols must not exceed grid
 hipError_t launch_lik_posteriors(const LikArgs& a, int grid, hipStream_t s);
 // The E-step on FP64 matrix cores for k = 64 without `Distribution leaves

@@ -17,7 +17,13 @@
 //                        rank-C update per branch instead of k^2 updates per
 //                        column.
 //
-// Lane a owns state a.  alpha (rows 0..nl-1: the leaf vectors) and beta live
+//   lik_small_kernel     likelihood and root posterior for alphabets of at most
+//                        24 states (nucleotides, dinucleotide classes, amino
+//                        acids), one column per lane: the column kernel below
+//                        gives such a column a whole wave (60 of 64 lanes idle
+//                        at k = 4).
+//
+// Otherwise lane a owns state a.  alpha (rows 0..nl-1: the leaf vectors) and beta live
 // in a global workspace per workgroup, so the tree size is not bounded by LDS.
 // With the E-step factors requested (U non-null) every workgroup takes one
 // column per launch: U and V hold one slot per workgroup and branch.
@@ -114,6 +120,94 @@ __global__ __launch_bounds__(64) void lik_columns_kernel(
   }
 }
 
+// One column per lane, k <= K states.  P and prior come padded with zeros to K
+// (a padded term adds 0 to a sum, so the sums are those of k terms) and are
+// uniform over the wave: scalar loads feed the multiply-adds.  A wave's 64 rows
+// of leaf states are staged in LDS (ldsl; trees over 256 leaves read them from
+// memory); internal nodes' alpha lie in ws as [node][state][lane].  Bound by
+// those (66,000 columns of 58 leaves at k = 4: 85 us, 2.3 ms with a column per
+// wave).  With no leaf_dist a state below -1 sets *bad.
+template <int K>
+__global__ __launch_bounds__(64) void lik_small_kernel(
+    int k, int n, const int32_t* __restrict__ lc, const int32_t* __restrict__ rc,
+    const double* __restrict__ P, const double* __restrict__ prior,
+    const int32_t* __restrict__ leaves, const double* __restrict__ leaf_dist, int64_t ncols,
+    double* __restrict__ ws, double* __restrict__ zout, int post_mode,
+    double* __restrict__ post, int* __restrict__ bad, int ldsl) {
+  extern __shared__ int32_t st[];  // 64 rows of nl states
+  const int lane = threadIdx.x, nl = (n + 1) / 2;
+  double* alpha = ws + (size_t)blockIdx.x * (n - nl) * K * 64 + lane;
+  for (int64_t c0 = (int64_t)blockIdx.x * 64; c0 < ncols; c0 += (int64_t)gridDim.x * 64) {
+    const int64_t col = min(c0 + lane, ncols - 1);  // lanes past the end repeat the last column
+    const int32_t* row = leaves + col * nl;
+    if (ldsl) {
+      const int64_t total = min((int64_t)64, ncols - c0) * nl;
+      for (int e = lane; e < total; e += 64) st[e] = leaves[c0 * nl + e];
+      __syncthreads();
+    }
+    const int32_t* own = st + (col - c0) * nl;
+    bool wrong = false;
+    // the vector of node c: e_i, ones, zeros or the given distribution for a leaf
+    auto vec = [&](int c, double (&v)[K]) {
+      if (c < nl) {
+        const int s = ldsl ? own[c] : row[c];
+        if (s == -2 && leaf_dist) {
+#pragma unroll
+          for (int a = 0; a < K; ++a) v[a] = a < k ? leaf_dist[(col * nl + c) * k + a] : 0.0;
+        } else {
+          wrong = wrong || s < -1;
+#pragma unroll
+          for (int a = 0; a < K; ++a) v[a] = (s == a || (s < 0 && a < k)) ? 1.0 : 0.0;
+        }
+      } else {
+#pragma unroll
+        for (int a = 0; a < K; ++a) v[a] = alpha[(size_t)((c - nl) * K + a) * 64];
+      }
+    };
+    double z = 0.0;
+    for (int i = nl; i < n; ++i) {
+      const int l = lc[i], r = rc[i];
+      double al[K], ar[K];
+      vec(l, al);
+      vec(r, ar);
+      const double* Pl = P + (size_t)l * K * K;
+      const double* Pr = P + (size_t)r * K * K;
+      if (i == n - 1) {
+        double root[K];
+#pragma unroll
+        for (int a = 0; a < K; ++a) {
+          double x = 0.0, y = 0.0;
+#pragma unroll
+          for (int b = 0; b < K; ++b) x = fma(Pl[a * K + b], al[b], x);
+#pragma unroll
+          for (int b = 0; b < K; ++b) y = fma(Pr[a * K + b], ar[b], y);
+          root[a] = x * y;
+          z = fma(root[a], prior[a], z);
+        }
+        if (c0 + lane < ncols) {
+          zout[col] = z;
+          if (post_mode == 1)
+#pragma unroll
+            for (int a = 0; a < K; ++a)
+              if (a < k) post[col * k + a] = (z == 0.0) ? 0.0 : root[a] * prior[a] / z;
+        }
+      } else {
+#pragma unroll
+        for (int a = 0; a < K; ++a) {
+          double x = 0.0, y = 0.0;
+#pragma unroll
+          for (int b = 0; b < K; ++b) x = fma(Pl[a * K + b], al[b], x);
+#pragma unroll
+          for (int b = 0; b < K; ++b) y = fma(Pr[a * K + b], ar[b], y);
+          alpha[(size_t)((i - nl) * K + a) * 64] = x * y;
+        }
+      }
+    }
+    if (__any(wrong) && lane == 0) atomicOr(bad, 1);
+    if (ldsl) __syncthreads();  // (one wave; the rows are overwritten)
+  }
+}
+
 // ecounts_br[a][b] += P_br[a][b] sum_j U[br][j][a] V[br][j][b] over the
 // nj column slots of one pass; one 256-thread workgroup per branch, each
 // thread 16 outputs (row a = t / 4, columns 16 (t % 4) ..), the slots staged
@@ -168,4 +262,25 @@ hipError_t launch_lik_posteriors(const LikArgs& x, int grid, hipStream_t s) {
   hipLaunchKernelGGL(branch_counts_kernel, dim3(x.n - 1), dim3(256), 0, s, x.k, grid, x.U, x.V,
                      x.P, x.ecounts);
   return hipGetLastError();
+}
+
+int lik_small_states(int k) { return k <= 4 ? 4 : k <= 8 ? 8 : k <= 16 ? 16 : k <= 24 ? 24 : 0; }
+
+hipError_t launch_lik_small(const LikArgs& x, int grid, int* bad, hipStream_t s) {
+  if (x.ncols <= 0) return hipSuccess;
+  const int nl = (x.n + 1) / 2;
+  const int ldsl = nl <= 256 ? 1 : 0;
+  const size_t lds = ldsl ? (size_t)64 * nl * 4 : 0;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), lds, s, x.k, x.n, x.lc, x.rc, x.P, x.prior,
+                       x.leaves, x.leaf_dist, x.ncols, x.ws, x.z, x.post_mode, x.post, bad, ldsl);
+    return hipGetLastError();
+  };
+  switch (lik_small_states(x.k)) {
+    case 4: return go(lik_small_kernel<4>);
+    case 8: return go(lik_small_kernel<8>);
+    case 16: return go(lik_small_kernel<16>);
+    case 24: return go(lik_small_kernel<24>);
+    default: return hipErrorInvalidValue;
+  }
 }
