@@ -493,12 +493,10 @@ struct SetModels {
   const double* qs;
 };
 
-// Node tiles of the FP64 outside pass (adjoint_mfma.hip): one
-// set per resident wave, allocated on first use.
-int ensure_adj_scratch(pcsf_batch* b) {
-  const pcsf_model* m = b->m;
-  pcsf_ctx* c = m->ctx;
-  const size_t need = adjoint_mfma_scratch_doubles(m, adjoint_mfma_grid(m));
+// Node tiles of the FP64 outside pass (adjoint_mfma.hip), one set per resident
+// workgroup or wave.
+int ensure_adj_scratch(pcsf_batch* b, size_t need) {
+  pcsf_ctx* c = b->m->ctx;
   if (b->adj_scratch >= need) return PCSF_OK;
   dfree(b->d_adj_scratch);
   b->adj_scratch = 0;
@@ -697,10 +695,11 @@ int adjoint_regions(pcsf_batch* b, const double* rho, const uint8_t* active, dou
     if (tangent) {
       e = launch_prune_tangent_regions(m, b, ch, c->stream);
     } else {
-      rc = ensure_adj_scratch(b);
+      const AdjointPlan plan = adjoint_plan(m, ch.nblocks);
+      rc = ensure_adj_scratch(b, plan.scratch);
       if (rc) return rc;
-      e = launch_adjoint_mfma(m, b, ch, d_gbr ? d_gbr + (size_t)r0 * nm * m->nbr : nullptr,
-                              b->d_adj_scratch, adjoint_mfma_grid(m), c->stream);
+      e = launch_adjoint_mfma(m, b, ch, plan, d_gbr ? d_gbr + (size_t)r0 * nm * m->nbr : nullptr,
+                              b->d_adj_scratch, c->stream);
     }
     HIP_TRY(c, e);
     HIP_TRY(c, launch_region_reduce_aligned(b, ch, b->d_gres, c->stream));

@@ -239,9 +239,9 @@ hipError_t launch_align_codes(const pcsf_batch* b, hipStream_t s);
 hipError_t launch_frames(const uint8_t* nuc, int64_t nlen, const int64_t* d_roff,
                          const int64_t* d_foff, int32_t nreg, int frames, int nl, uint8_t* dst,
                          int64_t ld, hipStream_t s);
-// The outside pass on FP64 matrix cores (kernels/adjoint_mfma.hip): region-
-// aligned blocks of 64 columns per workgroup; scratch holds one 64 x 16 FP64
-// tile per internal node for each of the grid's waves.
+// The outside pass on FP64 matrix cores (kernels/adjoint_mfma.hip): 16 columns
+// of a region-aligned block per workgroup; scratch holds two 64 x 16 FP64 tiles
+// per internal node for each workgroup of the grid.
 struct AdjointArgs {
   const uint8_t* codes;
   int64_t ld, ald;           // leading dimensions of codes and of the per-column outputs
@@ -249,7 +249,7 @@ struct AdjointArgs {
   int n, nl, nm, nbr;
   const int32_t *lc, *rc;
   const double* P64F;        // sets: P per branch (PSets::d_P64F layout)
-  const double* P64FT;       // sets: P^T per branch in A-fragment order
+  const double* P64FT;       // sets: P^T per branch in A-fragment order; a leaf's Q P by columns
   const double* QT;          // per model: Q^T
   const double* pi;          // per model, or per set with prior_per_set
   const double* lnpi;        // its logarithm
@@ -266,10 +266,15 @@ struct AdjointArgs {
   double* grad_branch;       // (region - r0) x nm x nbr, added to (may be null)
   double* scratch;
 };
-int adjoint_mfma_grid(const pcsf_model* m);
-size_t adjoint_mfma_scratch_doubles(const pcsf_model* m, int grid);
+// workgroups and doubles of scratch of the outside pass over `nblocks` blocks
+struct AdjointPlan {
+  int grid;
+  size_t scratch;
+};
+AdjointPlan adjoint_plan(const pcsf_model* m, int64_t nblocks);
 hipError_t launch_adjoint_mfma(const pcsf_model* m, const pcsf_batch* b, const RegionChunk& ch,
-                               double* grad_branch, double* scratch, int grid, hipStream_t s);
+                               const AdjointPlan& plan, double* grad_branch, double* scratch,
+                               hipStream_t s);
 // The FP64 forward on matrix cores (precision PCSF_FP64M, prune_fp64m.hip):
 // ln z and the root's expected ln pi per column of the chunk's region blocks
 // into the batch's aligned per-column buffers, from the sets' P64F.

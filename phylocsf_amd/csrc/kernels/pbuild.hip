@@ -33,7 +33,8 @@
 //         an internal branch's P in v_mfma_f64_16x16x4f64 A-fragment order,
 //         a leaf branch's 65 messages (columns of P, then all ones)
 //   P64FT FP64 P^T of internal branches in that A-fragment order (the outside
-//         pass's products)
+//         pass's products); of a leaf branch the columns of Q P, column c's row
+//         16 mo + 4 v + g at c * 64 + 16 mo + 4 g + v
 //   DT32, Dfrag  (tangent sets only) D = dP(rho b)/drho = b Q P in the layouts
 //         of PT32 (divided by P[c][c]; row 64 zero) and of the FP32 tile
 //         (dense), for leaf and internal branches respectively.
@@ -97,7 +98,10 @@ __device__ __forceinline__ unsigned long long fail_key(int set, int nbr, int br,
   return (pos << 2) | (unsigned long long)check;
 }
 
-template <bool WITH_D>
+// WITH_D: D as well, of every branch for the tangent pass (kTangent: D = b Q P)
+// or of leaf branches for the outside pass (kLeafQ: Q P).
+constexpr int kNoD = 0, kTangent = 1, kLeafQ = 2;
+template <int WITH_D>
 __global__ __launch_bounds__(256, WITH_D ? 2 : 3) void pbuild_kernel(
     const double* __restrict__ VT, const double* __restrict__ Vinv,
     const double* __restrict__ lam, const double* __restrict__ branch,
@@ -133,7 +137,8 @@ __global__ __launch_bounds__(256, WITH_D ? 2 : 3) void pbuild_kernel(
     {
       // every wave makes e[lane] itself and takes e[k] from lane k
       const double el = exp(t * lm);
-      const double dl = WITH_D ? bl * lm * el : 0.0;
+      const double dl = WITH_D == kTangent ? bl * lm * el : lm * el;
+      const bool want_d = WITH_D == kTangent || (WITH_D == kLeafQ && br < nl);
       const int sw = (lk & 1) << 4;
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll 4
@@ -148,7 +153,7 @@ __global__ __launch_bounds__(256, WITH_D ? 2 : 3) void pbuild_kernel(
           // column 16 ct + lr of B as stored in row k
           const double bv = Bs[k * 64 + ((16 * ct + lr) ^ sw)];
           acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bv, acc[ct], 0, 0, 0);
-          if constexpr (WITH_D)
+          if (WITH_D && want_d)
             dacc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(ad, bv, dacc[ct], 0, 0, 0);
         }
       }
@@ -274,6 +279,16 @@ __global__ __launch_bounds__(256, WITH_D ? 2 : 3) void pbuild_kernel(
         for (int r = 0; r < 4; ++r)
           out[(16 * w + 4 * ct + (lr >> 2)) * 64 + 4 * r + lk + 16 * (lr & 3)] = acc[ct][r];
     }
+    if constexpr (WITH_D == kLeafQ) {
+      if (leaf) {
+        double* out = P64FT + sb * 4096;
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            out[(16 * w + 4 * r + lk) * 64 + 16 * ct + 4 * (lr & 3) + (lr >> 2)] = dacc[ct][r];
+      }
+    }
     if (leaf && PT32) {
       float* out = PT32 + sb * (kLeafRows * 64);
 #pragma unroll
@@ -338,7 +353,7 @@ __global__ __launch_bounds__(256, WITH_D ? 2 : 3) void pbuild_kernel(
       }
       if (tid < 64) out[4096 + tid] = (float)(pdiag[tid] - 1.0);
     }
-    if constexpr (WITH_D) {
+    if constexpr (WITH_D == kTangent) {
       // D = dP(rho b)/drho = b Q P(t) for the tangent kernel, in the layout
       // of P: leaf rows D[a][c] / P[c][c] (row 64 zero: `Marginalize does not
       // depend on rho) for a leaf branch, the dense FP32 tile in the order of
@@ -457,7 +472,7 @@ hipError_t launch_pbuild(const pcsf_model* m, const PSets& sets, int nsets, int 
   // the device; one each for the few sets of a fixed-strategy model
   const int nbw = ((size_t)nsets * m->nbr >= 16384) ? 8 : 1;
   dim3 grid((m->nbr + nbw - 1) / nbw, nsets);
-  auto* k = tangent ? pbuild_kernel<true> : pbuild_kernel<false>;
+  auto* k = tangent ? pbuild_kernel<kTangent> : p64mt ? pbuild_kernel<kLeafQ> : pbuild_kernel<kNoD>;
   // the eigensystem of set s is model s % nm's, or the set's own when the
   // sets carry rate models (then s % cap = s)
   const bool own = sets.d_eVT != nullptr;
