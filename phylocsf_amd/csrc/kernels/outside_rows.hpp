@@ -20,13 +20,11 @@
 namespace outside {
 
 using fp64t::f64x4;
+using pcsf_mfma::kNowhere;
 using pcsf_mfma::Rsrc;
 
 constexpr int kNT = 256;              // threads: four waves
 constexpr int kSlot = 64 * 16;        // doubles of one 64 x 16 tile
-
-// A buffer offset past every buffer: the load returns zeros and reads nothing.
-constexpr uint32_t kNowhere = 0x80000000u;
 
 __device__ __forceinline__ f64x4 load4(Rsrc r, uint32_t off, uint32_t so) {
   const double2 a = __builtin_bit_cast(double2, pcsf_mfma::bload4(r, off, so));

@@ -50,31 +50,38 @@ struct Walk64 {
   bool has_next = false;
   int next_set = 0;
   int kg = 0;  // products done (selects the LDS buffer)
+  Tile64 pf;   // the next op's (first) leaf message, issued during a product
 
   __device__ __forceinline__ int oset() const {
     int s = set;
     asm volatile("" : "+s"(s));
     return s;
   }
-  // the message of leaf `leaf` for this lane's codon (message 64: ones)
-  __device__ __forceinline__ Tile64 leaf(int leaf) const {
+  // the message of leaf `leaf` for this lane's codon (message 64: ones), in
+  // eight pieces of two rows
+  struct LeafAt {
+    Rsrc r;
+    uint32_t off, so;
+  };
+  __device__ __forceinline__ LeafAt leaf_at(int leaf) const {
     const int code = codes_s[leaf * kGC + ccol];
     const uint32_t c = code == PCSF_MARGINALIZE ? 64u : (uint32_t)code;
     constexpr uint32_t kBranchBytes = kTile64 * 8;
-    const Rsrc r = make_rsrc(p.P64F + (size_t)oset() * p.nbr * kTile64,
-                                        p.nbr * kBranchBytes);
-    const uint32_t off = c * 512u + (uint32_t)grp * 32u;
+    return {make_rsrc(p.P64F + (size_t)oset() * p.nbr * kTile64, p.nbr * kBranchBytes),
+            c * 512u + (uint32_t)grp * 32u, leaf * kBranchBytes};
+  }
+  __device__ __forceinline__ static void leaf_piece(Tile64& t, const LeafAt& at, int k) {
+    const int mo = k >> 1, h = k & 1;
+    const double2 d =
+        __builtin_bit_cast(double2, bload4(at.r, at.off + 128u * mo + 16u * h, at.so));
+    t.r[mo][2 * h] = d.x;
+    t.r[mo][2 * h + 1] = d.y;
+  }
+  __device__ __forceinline__ Tile64 leaf(int leaf) const {
+    const LeafAt at = leaf_at(leaf);
     Tile64 t;
 #pragma unroll
-    for (int mo = 0; mo < 4; ++mo)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, off + 128u * mo + 16u * h,
-                                                             leaf * kBranchBytes, 0);
-        const double2 d = __builtin_bit_cast(double2, x);
-        t.r[mo][2 * h] = d.x;
-        t.r[mo][2 * h + 1] = d.y;
-      }
+    for (int k = 0; k < 8; ++k) leaf_piece(t, at, k);
     return t;
   }
   __device__ __forceinline__ static void mul(Tile64& s, const Tile64& o) {
@@ -82,14 +89,17 @@ struct Walk64 {
     for (int mo = 0; mo < 4; ++mo) s.r[mo] *= o.r[mo];
   }
   // s = leaf a0 o leaf a1
-  __device__ __forceinline__ void cherry(Tile64& s, NoMask&, int a0, int a1, bool) {
-    s = leaf(a0);
-    mul(s, leaf(a1));
+  __device__ __forceinline__ void cherry(Tile64& s, NoMask&, int a0, int a1, bool use_pf) {
+    const Tile64 o = leaf(a1);
+    s = use_pf ? pf : leaf(a0);
+    mul(s, o);
   }
   // the no-table programs have no table reads
   __device__ __forceinline__ void cherryt(Tile64&, NoMask&, int, int, int, bool) {}
   // s = s o leaf a0
-  __device__ __forceinline__ void leafmul(Tile64& s, NoMask&, int a0, bool) { mul(s, leaf(a0)); }
+  __device__ __forceinline__ void leafmul(Tile64& s, NoMask&, int a0, bool use_pf) {
+    mul(s, use_pf ? pf : leaf(a0));
+  }
   // s = s o o
   __device__ __forceinline__ void mulpop(Tile64& s, NoMask&, const Tile64& o, const NoMask&) {
     mul(s, o);
@@ -97,21 +107,20 @@ struct Walk64 {
   // s = P s for the tile staged in LDS; the next product's tile (branch
   // next_br of this set, or the next task's first) is loaded meanwhile into
   // the idle buffer, 16 bytes per lane at the wave's base + 16 lane: the
-  // layout the tile has in memory
-  __device__ __forceinline__ void gemm(Tile64& s, const NoMask&, int next_br, int, uint32_t) {
+  // layout the tile has in memory; and the next leaf op's message into pf.
+  // The loads stand between the MFMAs (in one burst in front of them each
+  // would keep the wave from its first for some 50 clocks), and the fragments
+  // are read from LDS kAhead steps before their MFMA (the compiler left two
+  // MFMAs between a read and its use).  100vertebrates, 120 regions of 100 to
+  // 3000 columns at a scale of their own: 7.49 -> 6.51 ms with the three.
+  __device__ __forceinline__ void gemm(Tile64& s, const NoMask&, int next_br, int pf_leaf,
+                                       uint32_t) {
+    constexpr int kAhead = 6;
     __syncthreads();  // Pbuf[kg&1] complete; Pbuf[(kg&1)^1] no longer read
+    __builtin_amdgcn_sched_barrier(0);  // a product is a scheduling region of its own
     L3* dst = Pbuf3[(kg & 1) ^ 1];
     constexpr int kPer = kTileBytes / 16 / kNT;  // 16-byte pieces per thread
-    if (next_br != kNoBranch) {
-      const Rsrc r = make_rsrc(p.P64F + (size_t)oset() * p.nbr * kTile64,
-                                          p.nbr * kTile64 * 8u);
-      const uint32_t so = next_br * (kTile64 * 8u);
-#pragma unroll
-      for (int k = 0; k < kPer; ++k)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsPtr)(dst + (64 * wave_s + kNT * k) * 2),
-                                                 16, (uint32_t)tid * 16u, so + 16u * kNT * k, 0,
-                                                 0);
-    } else if (has_next) {
+    if (next_br == kNoBranch && has_next) {
       typedef const __attribute__((address_space(1))) void* GPtr;
       const double* nsrc = p.P64F + ((size_t)next_set * p.nbr + p.first_gemm_br) * kTile64;
 #pragma unroll
@@ -119,7 +128,29 @@ struct Walk64 {
         __builtin_amdgcn_global_load_lds((GPtr)(nsrc + (tid + kNT * k) * 2),
                                          (LdsPtr)(dst + (64 * wave_s + kNT * k) * 2), 16, 0, 0);
     }
-    s = fp64t::gemm(Pbuf[kg & 1], s, lane);
+    const Rsrc rt = make_rsrc(p.P64F + (size_t)oset() * p.nbr * kTile64, p.nbr * kTile64 * 8u);
+    const uint32_t so = next_br * (kTile64 * 8u);
+    const bool ahead = pf_leaf != kNoBranch;
+    const LeafAt at = leaf_at(ahead ? pf_leaf : 0);
+    const double* frag = Pbuf[kg & 1] + lane;
+    double a[kAhead];
+#pragma unroll
+    for (int t = 0; t < kAhead; ++t) a[t] = frag[t * 64];
+    Tile64 m;
+#pragma unroll
+    for (int t = 0; t < 64; ++t) {
+      const int mo = t >> 4, k = t & 15, i = t >> 2;
+      f64x4 c = k == 0 ? (f64x4){0.0, 0.0, 0.0, 0.0} : m.r[mo];
+      m.r[mo] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t % kAhead], s.r[k >> 2][k & 3], c, 0, 0, 0);
+      if (t + kAhead < 64) a[t % kAhead] = frag[(t + kAhead) * 64];
+      if ((t & 3) == 0 && i < 8 && next_br != kNoBranch)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (LdsPtr)(dst + (64 * wave_s + kNT * i) * 2),
+                                                 16, (uint32_t)tid * 16u, so + 16u * kNT * i, 0, 0);
+      if ((t & 3) == 2 && i < 8 && ahead) leaf_piece(pf, at, i);
+      if (t & 1) __builtin_amdgcn_sched_barrier(0);  // the order stays as written
+    }
+    s = m;
+    __builtin_amdgcn_sched_barrier(0);
     ++kg;
   }
   // ln z and the root posterior's expected ln pi of this lane's column

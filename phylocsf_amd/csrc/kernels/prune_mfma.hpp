@@ -184,6 +184,9 @@ __device__ __forceinline__ double bload_f64(Rsrc r, uint32_t voff, uint32_t soff
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
 }
 
+// A buffer offset past every buffer: the load returns zero and reads nothing.
+constexpr uint32_t kNowhere = 0x80000000u;
+
 struct Gathered {
   Tile t;
   bool marg;
@@ -204,10 +207,14 @@ __device__ __forceinline__ void gather(Gathered& g, const MfmaParams& p, const u
   for (int mb = 0; mb < 4; ++mb) g.t.r[mb] = bload4(r, off + 64u * mb, leaf * kRowsBytes);
 }
 
-// Sum of ln P[c][c] over the gathered leaves of this lane's column.
+// Sum of ln P[c][c] over the gathered leaves of this lane's column, in the
+// lanes that write it out (group 0).  The vector L1 looks up one address per
+// clock and gathering lane, and the split-FP16 forward keeps it 92% busy: a
+// read repeated by the column's other three lanes would cost as much again.
 __device__ __forceinline__ double leaf_log_sum(const MfmaParams& p, const uint8_t* codes_s,
-                                              int gc, int set, int ccol) {
+                                              int gc, int set, int ccol, int grp) {
   double ls = 0.0;
+  if (grp != 0) return ls;
 #pragma unroll 8
   for (int i = 0; i < p.n_ls; ++i) {
     const int leaf = p.ls_leaves[i];
@@ -409,6 +416,8 @@ struct Walk {
   static constexpr int NT = 64 * WPG;        // threads
   static constexpr int PER = 4096 / NT / 4;  // float4 of the fragments per thread
   static constexpr int GC = 16 * WPG * G;    // columns per workgroup
+  // FP32: a product takes long enough to copy the next tile a quarter at a time
+  static constexpr bool SPREAD = PREC == kPrecF32 && PER == 4;
   using T = TileG<G>;
   using M = MaskG<G>;
   const MfmaParams& p;
@@ -485,7 +494,7 @@ struct Walk {
       for (int mbk = 0; mbk < 4; ++mbk)
         g[c].t.r[mbk] =
             bload4(rt, e * 256u + (uint32_t)grp * 16u + 64u * mbk, tab * kPairs * 256u);
-      ls[c] = bload_f64(rl, e * 8u, tab * kPairs * 8u);
+      ls[c] = bload_f64(rl, grp == 0 ? e * 8u : kNowhere, tab * kPairs * 8u);  // (leaf_log_sum)
       g[c].marg = ma && mb;
     }
   }
@@ -541,32 +550,32 @@ struct Walk {
     // barrier that opens the next GEMM waits for it.  Each instruction
     // writes 16 bytes per lane at the wave's LDS base + 16 * lane, the
     // layout the tile has in memory.
-    {
-      L3* dst = Pbuf3[(kg & 1) ^ 1];
-      typedef __attribute__((address_space(3))) void* LdsPtr;
-      if (next_br != kNoBranch) {
-        constexpr uint32_t kTileBytes = kTileFloats * 4;
-        const Rsrc r = make_rsrc(p.Pfrag + (size_t)st * p.nbr * kTileFloats, p.nbr * kTileBytes);
-        const uint32_t so = next_br * kTileBytes;
+    L3* dst = Pbuf3[(kg & 1) ^ 1];
+    typedef __attribute__((address_space(3))) void* LdsPtr;
+    constexpr uint32_t kTileBytes = kTileFloats * 4;
+    const Rsrc rt = make_rsrc(p.Pfrag + (size_t)st * p.nbr * kTileFloats, p.nbr * kTileBytes);
+    const uint32_t so = next_br * kTileBytes;
+    auto piece = [&](int q4) {  // a wave's q4-th KB of this set's next tile
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (LdsPtr)(dst + (64 * wave_s + NT * q4) * 4), 16,
+                                               (uint32_t)tid * 16u, so + 16u * NT * q4, 0, 0);
+    };
+    if (next_br != kNoBranch) {
+      if (tid < 16)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (LdsPtr)(dst + 4096), 16,
+                                                 (uint32_t)tid * 16u, so + 16384u, 0, 0);
+      if constexpr (!SPREAD)
 #pragma unroll
-        for (int q4 = 0; q4 < PER; ++q4)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              r, (LdsPtr)(dst + (64 * wave_s + NT * q4) * 4), 16, (uint32_t)tid * 16u,
-              so + 16u * NT * q4, 0, 0);
-        if (tid < 16)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsPtr)(dst + 4096), 16,
-                                                   (uint32_t)tid * 16u, so + 16384u, 0, 0);
-      } else if (has_next) {
-        typedef const __attribute__((address_space(1))) void* GPtr;
-        const float* nsrc = p.Pfrag + ((size_t)next_set * p.nbr + p.first_gemm_br) * kTileFloats;
+        for (int q4 = 0; q4 < PER; ++q4) piece(q4);
+    } else if (has_next) {
+      typedef const __attribute__((address_space(1))) void* GPtr;
+      const float* nsrc = p.Pfrag + ((size_t)next_set * p.nbr + p.first_gemm_br) * kTileFloats;
 #pragma unroll
-        for (int q4 = 0; q4 < PER; ++q4)
-          __builtin_amdgcn_global_load_lds((GPtr)(nsrc + (tid + NT * q4) * 4),
-                                           (LdsPtr)(dst + (64 * wave_s + NT * q4) * 4), 16, 0, 0);
-        if (tid < 16)
-          __builtin_amdgcn_global_load_lds((GPtr)(nsrc + 4096 + tid * 4), (LdsPtr)(dst + 4096),
-                                           16, 0, 0);
-      }
+      for (int q4 = 0; q4 < PER; ++q4)
+        __builtin_amdgcn_global_load_lds((GPtr)(nsrc + (tid + NT * q4) * 4),
+                                         (LdsPtr)(dst + (64 * wave_s + NT * q4) * 4), 16, 0, 0);
+      if (tid < 16)
+        __builtin_amdgcn_global_load_lds((GPtr)(nsrc + 4096 + tid * 4), (LdsPtr)(dst + 4096),
+                                         16, 0, 0);
     }
     const float* Ab = Pbuf[kg & 1];
     if constexpr (PREC == kPrecF32) {
@@ -576,12 +585,22 @@ struct Walk {
 #pragma unroll
         for (int mo = 0; mo < 4; ++mo) acc[c][mo] = (f32x4)(0.0f);
       if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        f32x4 A[4];
+      // A quarter's fragments are read during the quarter before, and a quarter
+      // of the next tile is copied in each (six frames of 120mammals: 12.1 ->
+      // 11.3 ms; the split-FP16 product, bound by the vector L1's gathers, has
+      // neither the registers nor the need).
+      f32x4 A[2][4];
+      auto read = [&](int mb) {
 #pragma unroll
         for (int mo = 0; mo < 4; ++mo)
-          A[mo] = *reinterpret_cast<const f32x4*>(Ab + ((mo * 4 + mb) * 64 + lane) * 4);
+          A[mb & 1][mo] = *reinterpret_cast<const f32x4*>(Ab + ((mo * 4 + mb) * 64 + lane) * 4);
+      };
+      read(0);
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        if (mb < 3) read(mb + 1);
+        if constexpr (SPREAD)
+          if (next_br != kNoBranch) piece(mb);
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
@@ -589,8 +608,10 @@ struct Walk {
             const float bv = s.g[c].r[mb][v];
 #pragma unroll
             for (int mo = 0; mo < 4; ++mo)
-              acc[c][mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[mo][v], bv, acc[c][mo], 0, 0, 0);
+              acc[c][mo] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(A[mb & 1][mo][v], bv, acc[c][mo], 0, 0, 0);
           }
+        __builtin_amdgcn_sched_barrier(0);  // the order stays as written
       }
       if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
       // m = alpha + (P_aa - 1) alpha + offdiag(P) alpha, the diagonal term in
@@ -765,7 +786,7 @@ __global__ __launch_bounds__(64 * WPG, MINW) void prune_mfma_kernel(MfmaParams p
     for (int c = 0; c < G; ++c) {
       w.col[c] = gabs * GC + w.ccol[c];
       w.E[c] = 0;
-      w.LS[c] = leaf_log_sum(p, codes_s, GC, cur.set, w.ccol[c]);
+      w.LS[c] = leaf_log_sum(p, codes_s, GC, cur.set, w.ccol[c], grp);
     }
     PROG::run(w, S, K);
     if (!has_next) break;

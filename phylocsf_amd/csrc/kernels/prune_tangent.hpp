@@ -24,6 +24,7 @@
 
 namespace pcsf_mfma {
 
+constexpr int kPairFloats = kTileFloats + 4096;  // a P tile and a D tile
 constexpr int kTWpg = 4;  // waves per workgroup (64 columns: one aligned block)
 
 struct TTile {  // a partial and its tangent
@@ -66,12 +67,13 @@ struct TWalk {
   static constexpr int PER = 4096 / NT / 4;  // float4 per thread of a 4096-float tile
   typedef __attribute__((address_space(3))) float L3;
   const MfmaParams& p;
-  const float (*Pbuf)[kTileFloats];  // LDS: double-buffered P and D tiles
-  const float (*Dbuf)[4096];
-  L3 (*Pbuf3)[kTileFloats];          // the same, as LDS addresses
-  L3 (*Dbuf3)[4096];
+  // LDS: double-buffered tiles, P then D (one array: with two, the compiler
+  // marks which of them an access belongs to, and then lets a product's reads
+  // wait for the copies into the other buffer of the same array)
+  const float (*Tbuf)[kPairFloats];
+  L3 (*Tbuf3)[kPairFloats];          // the same, as LDS addresses
   const uint8_t* codes_s;
-  int tid, lane, grp, ccol;
+  int tid, wave_s, lane, grp, ccol;
   int q = 0, set = 0;
   int64_t col = 0;
   bool has_next = false;
@@ -100,7 +102,7 @@ struct TWalk {
       g.d.r[mb] = bload4(rd, off + 64u * mb, leaf * kRowsBytes);
     }
     const Rsrc rl = make_rsrc(p.lnPcc + s0 * kLeafRows, p.nbr * kLeafRows * 8u);
-    LS += bload_f64(rl, c * 8u, leaf * kLeafRows * 8u);
+    LS += bload_f64(rl, grp == 0 ? c * 8u : kNowhere, leaf * kLeafRows * 8u);  // (leaf_log_sum)
     asm("" : "+v"(LS));
   }
   __device__ __forceinline__ void cherry(TTile& x, uint64_t& k, int a0, int a1, bool) {
@@ -142,59 +144,69 @@ struct TWalk {
   // tiles go straight from memory into the idle LDS buffers (as in Walk::gemm)
   __device__ __forceinline__ void gemm(TTile& x, uint64_t k, int next_br, int, uint32_t) {
     __syncthreads();  // tiles of buffer kg&1 complete; the other buffers are free
-    {
-      typedef __attribute__((address_space(3))) void* LdsPtr;
-      L3* dp = Pbuf3[(kg & 1) ^ 1];
-      L3* dd = Dbuf3[(kg & 1) ^ 1];
-      const int nset = (next_br != kNoBranch) ? oset() : next_set;
-      const int nbr = (next_br != kNoBranch) ? next_br : p.first_gemm_br;
-      if (next_br != kNoBranch || has_next) {
-        constexpr uint32_t kTileBytes = kTileFloats * 4;
-        const Rsrc rp = make_rsrc(p.Pfrag + (size_t)nset * p.nbr * kTileFloats, p.nbr * kTileBytes);
-        const Rsrc rd = make_rsrc(p.Dfrag + (size_t)nset * p.nbr * 4096, p.nbr * 16384u);
-#pragma unroll
-        for (int q4 = 0; q4 < PER; ++q4) {
-          const uint32_t w0 = (uint32_t)((tid & ~63) + NT * q4) * 4;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (LdsPtr)(dp + w0), 16, (uint32_t)tid * 16u,
-                                                   nbr * kTileBytes + 16u * NT * q4, 0, 0);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, (LdsPtr)(dd + w0), 16, (uint32_t)tid * 16u,
-                                                   nbr * 16384u + 16u * NT * q4, 0, 0);
-        }
-        if (tid < 16)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (LdsPtr)(dp + 4096), 16,
-                                                   (uint32_t)tid * 16u, nbr * kTileBytes + 16384u,
-                                                   0, 0);
-      }
-    }
-    const float* Ab = Pbuf[kg & 1];
-    const float* Db = Dbuf[kg & 1];
+    __builtin_amdgcn_sched_barrier(0);  // a product is a scheduling region of its own
+    typedef __attribute__((address_space(3))) void* LdsPtr;
+    L3* dp = Tbuf3[(kg & 1) ^ 1];
+    const int nset = (next_br != kNoBranch) ? oset() : next_set;
+    const int nbr = (next_br != kNoBranch) ? next_br : p.first_gemm_br;
+    const bool copy = next_br != kNoBranch || has_next;
+    constexpr uint32_t kTileBytes = kTileFloats * 4;
+    const Rsrc rp = make_rsrc(p.Pfrag + (size_t)nset * p.nbr * kTileFloats, p.nbr * kTileBytes);
+    const Rsrc rd = make_rsrc(p.Dfrag + (size_t)nset * p.nbr * 4096, p.nbr * 16384u);
+    if (copy && tid < 16)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (LdsPtr)(dp + 4096), 16, (uint32_t)tid * 16u,
+                                               nbr * kTileBytes + 16384u, 0, 0);
+    auto piece = [&](int i) {  // a wave's i-th KB of the next P (even i) or D (odd i) tile
+      const int q4 = i >> 1;
+      const uint32_t w0 = (uint32_t)(64 * wave_s + NT * q4) * 4;
+      if (i & 1)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, (LdsPtr)(dp + kTileFloats + w0), 16,
+                                                 (uint32_t)tid * 16u, nbr * 16384u + 16u * NT * q4,
+                                                 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (LdsPtr)(dp + w0), 16, (uint32_t)tid * 16u,
+                                                 nbr * kTileBytes + 16u * NT * q4, 0, 0);
+    };
+    const float* Ab = Tbuf[kg & 1];
+    const float* Db = Ab + kTileFloats;
     // P a' and D a stay in separate accumulators: summed in one (the MFMA's
     // FP32 accumulation rounds toward zero) the gradients measured 2-4x less
     // accurate against the FP64 adjoint
     f32x4 as[4], at[4], ad[4];
 #pragma unroll
     for (int mo = 0; mo < 4; ++mo) as[mo] = at[mo] = ad[mo] = (f32x4)(0.0f);
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      f32x4 A[4];
+    // The fragments of a quarter product are read from LDS during the one before
+    // (P and D alternate), a piece of the next tiles is copied in each: at one
+    // wave per SIMD (512 registers; 256 would spill 593) nothing else hides
+    // them.  100vertebrates, 100 regions: 11.0 -> 10.2 ms, where each product
+    // had waited for the copies that it started itself (Tbuf).
+    static_assert(PER == 4, "eight pieces per wave");
+    f32x4 A[2][4];
+    auto read = [&](int i) {
+      const float* src = (i & 1) ? Db : Ab;
 #pragma unroll
       for (int mo = 0; mo < 4; ++mo)
-        A[mo] = *reinterpret_cast<const f32x4*>(Ab + ((mo * 4 + mb) * 64 + lane) * 4);
+        A[i & 1][mo] = *reinterpret_cast<const f32x4*>(src + ((mo * 4 + (i >> 1)) * 64 + lane) * 4);
+    };
+    read(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int mb = i >> 1;
+      if (i + 1 < 8) read(i + 1);
+      if (copy) piece(i);
 #pragma unroll
       for (int v = 0; v < 4; ++v)
 #pragma unroll
         for (int mo = 0; mo < 4; ++mo) {
-          as[mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[mo][v], x.s.r[mb][v], as[mo], 0, 0, 0);
-          at[mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[mo][v], x.t.r[mb][v], at[mo], 0, 0, 0);
+          const float a = A[i & 1][mo][v];
+          if (i & 1) {
+            ad[mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x.s.r[mb][v], ad[mo], 0, 0, 0);
+          } else {
+            as[mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x.s.r[mb][v], as[mo], 0, 0, 0);
+            at[mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x.t.r[mb][v], at[mo], 0, 0, 0);
+          }
         }
-#pragma unroll
-      for (int mo = 0; mo < 4; ++mo)
-        A[mo] = *reinterpret_cast<const f32x4*>(Db + ((mo * 4 + mb) * 64 + lane) * 4);
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-#pragma unroll
-        for (int mo = 0; mo < 4; ++mo)
-          ad[mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[mo][v], x.s.r[mb][v], ad[mo], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
     const bool cst = (k >> lane) & 1;
 #pragma unroll
@@ -235,10 +247,9 @@ struct TWalk {
 template <int NS, class PROG>
 __global__ __launch_bounds__(64 * kTWpg, 1) void prune_tangent_kernel(MfmaParams p) {
   constexpr int NT = TWalk::NT, GC = TWalk::GC, PER = TWalk::PER;
-  __shared__ __attribute__((aligned(16))) float Pbuf[2][kTileFloats];
-  __shared__ __attribute__((aligned(16))) float Dbuf[2][4096];
+  __shared__ __attribute__((aligned(16))) float Tbuf[2][kPairFloats];
   extern __shared__ __attribute__((aligned(16))) uint8_t codes_s[];  // nl x GC
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
 
   TTile S[NS];
   uint64_t K[NS];
@@ -256,17 +267,17 @@ __global__ __launch_bounds__(64 * kTWpg, 1) void prune_tangent_kernel(MfmaParams
     const float* ds = p.Dfrag + ((size_t)cur.set * p.nbr + p.first_gemm_br) * 4096;
 #pragma unroll
     for (int r = 0; r < PER; ++r) {
-      *reinterpret_cast<f32x4*>(&Pbuf[0][(tid + NT * r) * 4]) =
+      *reinterpret_cast<f32x4*>(&Tbuf[0][(tid + NT * r) * 4]) =
           *reinterpret_cast<const f32x4*>(ps + (tid + NT * r) * 4);
-      *reinterpret_cast<f32x4*>(&Dbuf[0][(tid + NT * r) * 4]) =
+      *reinterpret_cast<f32x4*>(&Tbuf[0][kTileFloats + (tid + NT * r) * 4]) =
           *reinterpret_cast<const f32x4*>(ds + (tid + NT * r) * 4);
     }
     if (tid < 16)
-      *reinterpret_cast<f32x4*>(&Pbuf[0][4096 + tid * 4]) =
+      *reinterpret_cast<f32x4*>(&Tbuf[0][4096 + tid * 4]) =
           *reinterpret_cast<const f32x4*>(ps + 4096 + tid * 4);
   }
-  TWalk w{p, Pbuf, Dbuf, (TWalk::L3 (*)[kTileFloats])Pbuf, (TWalk::L3 (*)[4096])Dbuf,
-          codes_s, tid, lane, lane >> 4, wave * 16 + (lane & 15)};
+  TWalk w{p, Tbuf, (TWalk::L3 (*)[kPairFloats])Tbuf, codes_s, tid, wave, lane, lane >> 4,
+          wave * 16 + (lane & 15)};
   for (;;) {
     Task nxt;
     int64_t jn = jc + 1;
