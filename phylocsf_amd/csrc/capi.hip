@@ -997,9 +997,14 @@ int pcsf_model_create(pcsf_ctx* c, int n, const int32_t* children, const double*
   m->tree_t = find_tree_program(m->prog_t, true);
   // default launch shape until pcsf_autotune: three waves per SIMD for the
   // straight-line programs (the fastest shape on every shipped tree measured),
-  // two for the interpreter, whose switch needs more registers
-  if (m->tree_p && m->tree_t)
+  // two for the interpreter, whose switch needs more registers; in FP32 with
+  // the next leaf's rows loaded ahead (1.03 to 1.14 times as fast over 12 to
+  // 120 leaves and 1 to 1000 regions; in split FP16, bound by those gathers
+  // themselves, 0.97 to 1.05)
+  if (m->tree_p && m->tree_t) {
     for (int& v : m->mfma_variant) v = 2;
+    m->mfma_variant[PCSF_FP32] = 5;
+  }
   if (m->slots > kMaxSlots)
     return set_err(c, PCSF_EINVAL, "tree needs more than 6 live partial tiles");
   if (!c) {  // host-only model: simulation and model facts, no device work

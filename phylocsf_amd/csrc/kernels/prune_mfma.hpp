@@ -560,9 +560,17 @@ struct Walk {
                                                (uint32_t)tid * 16u, so + 16u * NT * q4, 0, 0);
     };
     if (next_br != kNoBranch) {
-      if (tid < 16)
+      // the diagonal: by every wave where leaf rows may be in flight (a branch
+      // for one wave leaves the compiler with two counts of the loads in
+      // flight, and it waits for the lower one), by one where the vector L1 is
+      // what bounds the kernel
+      if constexpr (SPREAD) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (LdsPtr)(dst + 4096), 4, (uint32_t)lane * 4u,
+                                                 so + 16384u, 0, 0);
+      } else if (tid < 16) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (LdsPtr)(dst + 4096), 16,
                                                  (uint32_t)tid * 16u, so + 16384u, 0, 0);
+      }
       if constexpr (!SPREAD)
 #pragma unroll
         for (int q4 = 0; q4 < PER; ++q4) piece(q4);

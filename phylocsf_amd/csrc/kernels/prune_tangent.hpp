@@ -62,6 +62,16 @@ __device__ __forceinline__ void rescale2(Tile& s, Tile& t, int& E) {
   asm("" : "+v"(E));  // a running sum (see mul_rescale)
 }
 
+// t m + s d, with one rounding of s d and one of the sum (written out: left to
+// the compiler the generated programs and the interpreter need not agree)
+__device__ __forceinline__ f32x4 product_rule(const f32x4& t, const f32x4& m, const f32x4& s,
+                                              const f32x4& d) {
+  f32x4 r;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) r[v] = fmaf(t[v], m[v], s[v] * d[v]);
+  return r;
+}
+
 struct TWalk {
   static constexpr int NT = 64 * kTWpg, GC = 16 * kTWpg;
   static constexpr int PER = 4096 / NT / 4;  // float4 per thread of a 4096-float tile
@@ -81,38 +91,68 @@ struct TWalk {
   int kg = 0;
   int E = 0;
   double LS = 0.0;
+  TGathered pf;     // the next op's first leaf, and its ln P[c][c]
+  double lpf = 0.0;
 
   __device__ __forceinline__ int oset() const {
     int s = set;
     asm volatile("" : "+s"(s));
     return s;
   }
-  __device__ __forceinline__ void tgather(TGathered& g, int leaf) {
+  // a leaf's rows M and D, in eight pieces, and its ln P[c][c]
+  struct LeafAt {
+    Rsrc rm, rd, rl;
+    uint32_t c, off;
+    int leaf;
+  };
+  static constexpr uint32_t kRowsBytes = kLeafRows * 64 * 4;
+  __device__ __forceinline__ LeafAt leaf_at(TGathered& g, int leaf) const {
     const int code = codes_s[leaf * GC + ccol];
     g.marg = code == PCSF_MARGINALIZE;
     const uint32_t c = g.marg ? 64 : code;
-    constexpr uint32_t kRowsBytes = kLeafRows * 64 * 4;
     const size_t s0 = (size_t)oset() * p.nbr;
-    const Rsrc rm = make_rsrc(p.PT32 + s0 * (kLeafRows * 64), p.nbr * kRowsBytes);
-    const Rsrc rd = make_rsrc(p.DT32 + s0 * (kLeafRows * 64), p.nbr * kRowsBytes);
-    const uint32_t off = c * 256u + (uint32_t)grp * 16u;
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      g.m.r[mb] = bload4(rm, off + 64u * mb, leaf * kRowsBytes);
-      g.d.r[mb] = bload4(rd, off + 64u * mb, leaf * kRowsBytes);
-    }
-    const Rsrc rl = make_rsrc(p.lnPcc + s0 * kLeafRows, p.nbr * kLeafRows * 8u);
-    LS += bload_f64(rl, grp == 0 ? c * 8u : kNowhere, leaf * kLeafRows * 8u);  // (leaf_log_sum)
+    return {make_rsrc(p.PT32 + s0 * (kLeafRows * 64), p.nbr * kRowsBytes),
+            make_rsrc(p.DT32 + s0 * (kLeafRows * 64), p.nbr * kRowsBytes),
+            make_rsrc(p.lnPcc + s0 * kLeafRows, p.nbr * kLeafRows * 8u),
+            c, c * 256u + (uint32_t)grp * 16u, leaf};
+  }
+  __device__ __forceinline__ static void leaf_piece(TGathered& g, const LeafAt& at, int i) {
+    const int mb = i >> 1;
+    if (i & 1)
+      g.d.r[mb] = bload4(at.rd, at.off + 64u * mb, at.leaf * kRowsBytes);
+    else
+      g.m.r[mb] = bload4(at.rm, at.off + 64u * mb, at.leaf * kRowsBytes);
+  }
+  __device__ __forceinline__ double leaf_log(const LeafAt& at) const {  // (leaf_log_sum)
+    return bload_f64(at.rl, grp == 0 ? at.c * 8u : kNowhere, at.leaf * kLeafRows * 8u);
+  }
+  __device__ __forceinline__ void add_log(double l) {
+    LS += l;
     asm("" : "+v"(LS));
   }
-  __device__ __forceinline__ void cherry(TTile& x, uint64_t& k, int a0, int a1, bool) {
+  __device__ __forceinline__ void tgather(TGathered& g, int leaf) {
+    const LeafAt at = leaf_at(g, leaf);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) leaf_piece(g, at, i);
+    add_log(leaf_log(at));
+  }
+  // the op's first leaf: loaded during the product before it (use_pf), or now
+  __device__ __forceinline__ void first_leaf(TGathered& g, int leaf, bool use_pf) {
+    if (use_pf) {
+      g = pf;
+      add_log(lpf);
+    } else {
+      tgather(g, leaf);
+    }
+  }
+  __device__ __forceinline__ void cherry(TTile& x, uint64_t& k, int a0, int a1, bool use_pf) {
     TGathered g0, g1;
-    tgather(g0, a0);
+    first_leaf(g0, a0, use_pf);
     tgather(g1, a1);
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
       x.s.r[mb] = g0.m.r[mb] * g1.m.r[mb];
-      x.t.r[mb] = g0.d.r[mb] * g1.m.r[mb] + g0.m.r[mb] * g1.d.r[mb];
+      x.t.r[mb] = product_rule(g0.d.r[mb], g1.m.r[mb], g0.m.r[mb], g1.d.r[mb]);
     }
     k = __ballot(g0.marg && g1.marg);
     rescale2(x.s, x.t, E);
@@ -120,12 +160,12 @@ struct TWalk {
   // programs with cherry tables never reach this kernel (a table message has
   // no tangent row); the op exists so the program drivers compile
   __device__ __forceinline__ void cherryt(TTile&, uint64_t&, int, int, int, bool) {}
-  __device__ __forceinline__ void leafmul(TTile& x, uint64_t& k, int a0, bool) {
+  __device__ __forceinline__ void leafmul(TTile& x, uint64_t& k, int a0, bool use_pf) {
     TGathered g;
-    tgather(g, a0);
+    first_leaf(g, a0, use_pf);
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
-      x.t.r[mb] = x.t.r[mb] * g.m.r[mb] + x.s.r[mb] * g.d.r[mb];
+      x.t.r[mb] = product_rule(x.t.r[mb], g.m.r[mb], x.s.r[mb], g.d.r[mb]);
       x.s.r[mb] = x.s.r[mb] * g.m.r[mb];
     }
     k &= __ballot(g.marg);
@@ -134,15 +174,16 @@ struct TWalk {
   __device__ __forceinline__ void mulpop(TTile& x, uint64_t& k, const TTile& o, uint64_t ko) {
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
-      x.t.r[mb] = x.t.r[mb] * o.s.r[mb] + x.s.r[mb] * o.t.r[mb];
+      x.t.r[mb] = product_rule(x.t.r[mb], o.s.r[mb], x.s.r[mb], o.t.r[mb]);
       x.s.r[mb] = x.s.r[mb] * o.s.r[mb];
     }
     k &= ko;
     rescale2(x.s, x.t, E);
   }
   // m = P s, m' = P t + D s for the tiles staged in LDS; the next P and D
-  // tiles go straight from memory into the idle LDS buffers (as in Walk::gemm)
-  __device__ __forceinline__ void gemm(TTile& x, uint64_t k, int next_br, int, uint32_t) {
+  // tiles go straight from memory into the idle LDS buffers (as in Walk::gemm),
+  // the next leaf op's rows into pf
+  __device__ __forceinline__ void gemm(TTile& x, uint64_t k, int next_br, int pf_leaf, uint32_t) {
     __syncthreads();  // tiles of buffer kg&1 complete; the other buffers are free
     __builtin_amdgcn_sched_barrier(0);  // a product is a scheduling region of its own
     typedef __attribute__((address_space(3))) void* LdsPtr;
@@ -153,8 +194,16 @@ struct TWalk {
     constexpr uint32_t kTileBytes = kTileFloats * 4;
     const Rsrc rp = make_rsrc(p.Pfrag + (size_t)nset * p.nbr * kTileFloats, p.nbr * kTileBytes);
     const Rsrc rd = make_rsrc(p.Dfrag + (size_t)nset * p.nbr * 4096, p.nbr * 16384u);
-    if (copy && tid < 16)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (LdsPtr)(dp + 4096), 16, (uint32_t)tid * 16u,
+    // (the code is read before the first copy starts: a read of the codes waits
+    // for the copies in flight)
+    const bool ahead = pf_leaf != kNoBranch;
+    const LeafAt leaf = leaf_at(pf, ahead ? pf_leaf : 0);
+    if (ahead) lpf = leaf_log(leaf);
+    __builtin_amdgcn_sched_barrier(0);
+    // the diagonal, by every wave: a branch for one would leave the compiler
+    // with two counts of the loads in flight, and waits for the lower one
+    if (copy)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (LdsPtr)(dp + 4096), 4, (uint32_t)lane * 4u,
                                                nbr * kTileBytes + 16384u, 0, 0);
     auto piece = [&](int i) {  // a wave's i-th KB of the next P (even i) or D (odd i) tile
       const int q4 = i >> 1;
@@ -176,10 +225,13 @@ struct TWalk {
 #pragma unroll
     for (int mo = 0; mo < 4; ++mo) as[mo] = at[mo] = ad[mo] = (f32x4)(0.0f);
     // The fragments of a quarter product are read from LDS during the one before
-    // (P and D alternate), a piece of the next tiles is copied in each: at one
-    // wave per SIMD (512 registers; 256 would spill 593) nothing else hides
-    // them.  100vertebrates, 100 regions: 11.0 -> 10.2 ms, where each product
-    // had waited for the copies that it started itself (Tbuf).
+    // (P and D alternate), a piece of the next tiles and of the next leaf's rows
+    // is loaded in each.  100vertebrates, 120 regions of 100 to 3000 columns:
+    // 11.0 -> 10.2 ms where each product had waited for the copies that it
+    // started itself (Tbuf), 7.9 with the rows loaded ahead and, with fewer
+    // loads counted wrongly and so fewer values held back in registers, two
+    // workgroups per CU (35 registers spilled; 593 before the diagonal's copy
+    // lost its branch).
     static_assert(PER == 4, "eight pieces per wave");
     f32x4 A[2][4];
     auto read = [&](int i) {
@@ -194,6 +246,7 @@ struct TWalk {
       const int mb = i >> 1;
       if (i + 1 < 8) read(i + 1);
       if (copy) piece(i);
+      if (ahead) leaf_piece(pf, leaf, i);
 #pragma unroll
       for (int v = 0; v < 4; ++v)
 #pragma unroll
@@ -245,7 +298,7 @@ struct TWalk {
 };
 
 template <int NS, class PROG>
-__global__ __launch_bounds__(64 * kTWpg, 1) void prune_tangent_kernel(MfmaParams p) {
+__global__ __launch_bounds__(64 * kTWpg, 2) void prune_tangent_kernel(MfmaParams p) {
   constexpr int NT = TWalk::NT, GC = TWalk::GC, PER = TWalk::PER;
   __shared__ __attribute__((aligned(16))) float Tbuf[2][kPairFloats];
   extern __shared__ __attribute__((aligned(16))) uint8_t codes_s[];  // nl x GC
