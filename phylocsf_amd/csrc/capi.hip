@@ -797,9 +797,8 @@ void pcsf_ctx_destroy(pcsf_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   EstepCache& es = c->es;
   if (es.copy) (void)hipStreamSynchronize(es.copy);
-  dfree(es.U);
-  dfree(es.V);
-  dfree(es.scr);
+  dfree(es.M);
+  dfree(es.B);
   for (int i = 0; i < 2; ++i) {
     dfree(es.leaves[i]);
     if (es.staged[i]) (void)hipHostFree(es.staged[i]);
@@ -2386,14 +2385,14 @@ namespace {
 // kernels/lik.hip.  Columns go in chunks whose device buffers stay within
 // ~512 MB; post_mode 1 = the root's posterior, 2 = every node's.
 // The E-step for 64 states without `Distribution leaves on the FP64 matrix
-// cores (kernels/estep.hip): columns in chunks of up to 32,768, u and v of
-// every (branch, column) of a chunk in device memory, the counts added per
-// chunk.
+// cores (kernels/estep.hip): columns in chunks of up to 32,768, message and
+// beta of every (internal node, column) of a chunk in device memory, the counts
+// added per chunk.
 // The context's E-step buffers for chunks of `chunk` columns (grown, never
 // shrunk; a failed growth leaves them released).
-hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk, int grid) {
+hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk) {
   EstepCache& es = c->es;
-  const int nl = (n + 1) / 2, nbr = n - 1;
+  const int nl = (n + 1) / 2;
   hipError_t e = hipSuccess;
   if (!es.copy) e = hipStreamCreateWithFlags(&es.copy, hipStreamNonBlocking);
   for (int i = 0; i < 2 && e == hipSuccess; ++i) {
@@ -2402,26 +2401,19 @@ hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk, int grid)
       e = hipEventCreateWithFlags(&es.consumed[i], hipEventDisableTiming);
   }
   if (e != hipSuccess) return e;
-  const size_t uv = (size_t)nbr * ldu * 64;
-  if (es.cap_uv < uv) {
-    dfree(es.U);
-    dfree(es.V);
-    es.cap_uv = 0;
-    e = dalloc(c, &es.U, uv);
-    if (e == hipSuccess) e = dalloc(c, &es.V, uv);
+  const size_t mb = (size_t)(n - nl) * ldu * 64;
+  if (es.cap_mb < mb) {
+    dfree(es.M);
+    dfree(es.B);
+    es.cap_mb = 0;
+    e = dalloc(c, &es.M, mb);
+    if (e == hipSuccess) e = dalloc(c, &es.B, mb);
     if (e != hipSuccess) {
-      dfree(es.U);
-      dfree(es.V);
+      dfree(es.M);
+      dfree(es.B);
       return e;
     }
-    es.cap_uv = uv;
-  }
-  const size_t scr = estep_scratch_doubles(n, grid);
-  if (es.cap_scr < scr) {
-    dfree(es.scr);
-    es.cap_scr = 0;
-    if ((e = dalloc(c, &es.scr, scr)) != hipSuccess) return e;
-    es.cap_scr = scr;
+    es.cap_mb = mb;
   }
   const size_t lv = (size_t)chunk * nl;
   if (es.cap_leaves < lv) {
@@ -2458,31 +2450,29 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
   const int nl = (n + 1) / 2, nbr = n - 1;
   const int64_t chunk = std::min<int64_t>(ncols, 32768);
   const int64_t ldu = (chunk + 63) / 64 * 64;
-  const int grid = estep_grid(c);
-  std::vector<double> rowsum((size_t)nbr * 64);
-  for (int br = 0; br < nbr; ++br)
-    for (int a = 0; a < 64; ++a) {
-      double t = 0.0;
-      for (int b = 0; b < 64; ++b) t += P[((size_t)br * 64 + a) * 64 + b];
-      rowsum[(size_t)br * 64 + a] = t;
-    }
+  std::vector<int32_t> parent((size_t)n, 0);
+  for (int i = nl; i < n; ++i) parent[lc[i]] = parent[rc[i]] = i;
   const std::vector<int32_t> seq = estep_sequence(n, lc, rc);
-  int32_t *d_lc = nullptr, *d_rc = nullptr, *d_seq = nullptr;
-  double *d_P = nullptr, *d_rs = nullptr, *d_prior = nullptr, *d_w = nullptr, *d_z = nullptr,
+  int32_t *d_lc = nullptr, *d_rc = nullptr, *d_up = nullptr, *d_seq = nullptr;
+  uint8_t* d_codes = nullptr;
+  double *d_P = nullptr, *d_Lm = nullptr, *d_scale = nullptr, *d_prior = nullptr, *d_w = nullptr, *d_z = nullptr,
          *d_ec = nullptr, *d_Pf = nullptr, *d_PTf = nullptr;
   hipError_t e = hipSuccess;
   auto chk = [&](hipError_t x) {
     if (e == hipSuccess) e = x;
   };
-  chk(estep_cache(c, n, ldu, chunk, grid));
+  chk(estep_cache(c, n, ldu, chunk));
   EstepCache& es = c->es;
   chk(dalloc(c, &d_lc, (size_t)n));
   chk(dalloc(c, &d_rc, (size_t)n));
+  chk(dalloc(c, &d_up, (size_t)n));
+  chk(dalloc(c, &d_codes, (size_t)nl * ldu));
+  chk(dalloc(c, &d_scale, (size_t)ldu));
+  chk(dalloc(c, &d_Lm, (size_t)nl * estep_leaf_table_doubles()));
   chk(dalloc(c, &d_P, (size_t)nbr * 4096));
   chk(dalloc(c, &d_Pf, (size_t)nbr * 4096));
   chk(dalloc(c, &d_PTf, (size_t)nbr * 4096));
   chk(dalloc(c, &d_seq, std::max<size_t>(1, seq.size())));
-  chk(dalloc(c, &d_rs, (size_t)nbr * 64));
   chk(dalloc(c, &d_prior, 64));
   if (weights) chk(dalloc(c, &d_w, (size_t)ncols));
   chk(dalloc(c, &d_z, (size_t)ncols));
@@ -2495,10 +2485,10 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
   };
   up(d_lc, lc.data(), (size_t)n * 4);
   up(d_rc, rc.data(), (size_t)n * 4);
+  up(d_up, parent.data(), (size_t)n * 4);
   up(d_P, P, (size_t)nbr * 4096 * 8);
   up(d_seq, seq.data(), seq.size() * 4);
-  if (e == hipSuccess) e = launch_estep_frags(d_P, nbr, d_Pf, d_PTf, c->stream);
-  up(d_rs, rowsum.data(), rowsum.size() * 8);
+  if (e == hipSuccess) e = launch_estep_frags(d_P, nl, nbr, d_Pf, d_PTf, d_Lm, c->stream);
   up(d_prior, prior, 64 * 8);
   up(d_ec, ecounts, (size_t)nbr * 4096 * 8);  // add_branch_posteriors adds
   if (weights) up(d_w, weights, (size_t)ncols * 8);
@@ -2535,17 +2525,18 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
     a.PTf = d_PTf;
     a.seq = d_seq;
     a.nseq = (int)seq.size();
-    a.rowsum = d_rs;
+    a.parent = d_up;
+    a.Lm = d_Lm;
     a.prior = d_prior;
-    a.leaves = es.leaves[sl];
+    a.codes = d_codes;
     a.weights = d_w ? d_w + c0 : nullptr;
     a.ncols = nc;
     a.z = d_z + c0;
-    a.U = es.U;
-    a.V = es.V;
+    a.scale = d_scale;
+    a.M = es.M;
+    a.B = es.B;
     a.ldu = ldu;
-    a.scratch = es.scr;
-    if (e == hipSuccess) e = launch_estep(a, d_P, d_ec, grid, c->stream);
+    if (e == hipSuccess) e = launch_estep(a, es.leaves[sl], d_ec, c->num_cus, c->stream);
     chk(hipEventRecord(es.consumed[sl], c->stream));
   }
   // both streams drain before any buffer of this call is released
@@ -2555,11 +2546,12 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
   chk(s2);
   down(z, d_z, (size_t)ncols * 8);
   down(ecounts, d_ec, (size_t)nbr * 4096 * 8);
-  for (auto* q : {d_lc, d_rc, d_seq}) {
+  for (auto* q : {d_lc, d_rc, d_up, d_seq}) {
     int32_t* x = q;
     dfree(x);
   }
-  for (auto* q : {d_P, d_rs, d_prior, d_w, d_z, d_ec, d_Pf, d_PTf}) {
+  dfree(d_codes);
+  for (auto* q : {d_P, d_Lm, d_scale, d_prior, d_w, d_z, d_ec, d_Pf, d_PTf}) {
     double* x = q;
     dfree(x);
   }

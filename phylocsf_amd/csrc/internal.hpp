@@ -73,12 +73,12 @@ struct PSets {
 };
 
 // Device and pinned buffers of the E-step (capi.hip estep_mfma), kept by the
-// context between calls and grown as needed: the u, v hand-over of a chunk
-// (gigabytes), the passes' node tiles, and two leaf-state slots that a second
-// stream fills (from pinned staging) while the previous chunk computes.
+// context between calls and grown as needed: the messages and betas of a chunk
+// (gigabytes), and two leaf-state slots that a second stream fills (from pinned
+// staging) while the previous chunk computes.
 struct EstepCache {
-  double *U = nullptr, *V = nullptr, *scr = nullptr;
-  size_t cap_uv = 0, cap_scr = 0;  // doubles of U (= of V) and of scr
+  double *M = nullptr, *B = nullptr;
+  size_t cap_mb = 0;                        // doubles of M (= of B)
   int32_t* leaves[2] = {nullptr, nullptr};
   int32_t* staged[2] = {nullptr, nullptr};  // pinned host
   size_t cap_leaves = 0;                    // int32 per slot
@@ -345,29 +345,32 @@ hipError_t launch_lik_posteriors(const LikArgs& a, int grid, hipStream_t s);
 struct EstepArgs {
   int n = 0, nl = 0;
   const int32_t *lc = nullptr, *rc = nullptr;
+  const int32_t* parent = nullptr;  // of every node but the root
   const double* P = nullptr;        // (n-1) x 64 x 64, row-major per branch
   const double* Pf = nullptr;       // (n-1) x 4096: P in A-fragment order (fp64_tiles.hpp)
   const double* PTf = nullptr;      // (n-1) x 4096: P^T in A-fragment order
+  const double* Lm = nullptr;       // nl tables of leaf messages (estep_leaf_table_doubles)
   const int32_t* seq = nullptr;     // the passes' products in order: branch b for P_b,
                                     //   -1 - b for P_b^T (estep_sequence)
   int nseq = 0;
-  const double* rowsum = nullptr;   // (n-1) x 64: P's row sums (`Marginalize leaf messages)
   const double* prior = nullptr;    // 64
-  const int32_t* leaves = nullptr;  // ncols x nl: state, -1 `Marginalize, >= 64 zeros
+  uint8_t* codes = nullptr;         // nl x ldu: the chunk's states as rows of Lm
   const double* weights = nullptr;  // ncols (null: 1)
   int64_t ncols = 0;
   double* z = nullptr;              // ncols
-  double* U = nullptr;              // (n-1) x ldu x 64
-  double* V = nullptr;
-  int64_t ldu = 0;                  // columns per branch in U, V (>= ncols rounded up to 64)
-  double* scratch = nullptr;        // estep_scratch_doubles(n, grid)
+  double* scale = nullptr;          // ldu: weight / z, 0 where nothing is counted
+  double* M = nullptr;              // ldu / 16 x (n - nl) tiles: messages of internal nodes
+  double* B = nullptr;              // the same: their betas
+  int64_t ldu = 0;                  // columns in codes, M, B (>= ncols, a multiple of 64)
 };
-int estep_grid(const pcsf_ctx* c);
-size_t estep_scratch_doubles(int n, int grid);
+size_t estep_leaf_table_doubles();
 // the products of estep_passes_kernel in the order it runs them
 std::vector<int32_t> estep_sequence(int n, const std::vector<int32_t>& lc,
                                     const std::vector<int32_t>& rc);
-// Pf and PTf of EstepArgs from P (nbr row-major 64 x 64 matrices)
-hipError_t launch_estep_frags(const double* P, int nbr, double* Pf, double* PTf, hipStream_t s);
-hipError_t launch_estep(const EstepArgs& a, const double* P, double* ecounts, int grid,
+// Pf, PTf (internal branches) and Lm (leaf branches) of EstepArgs from P (nbr
+// row-major 64 x 64 matrices)
+hipError_t launch_estep_frags(const double* P, int nl, int nbr, double* Pf, double* PTf,
+                              double* Lm, hipStream_t s);
+// leaves: ncols x nl: state, -1 `Marginalize, >= 64 zeros
+hipError_t launch_estep(const EstepArgs& a, const int32_t* leaves, double* ecounts, int num_cus,
                         hipStream_t s);
