@@ -493,8 +493,8 @@ struct SetModels {
   const double* qs;
 };
 
-// Node tiles of the FP64 outside pass (adjoint_mfma.hip), one set per resident
-// workgroup or wave.
+// Node tiles of the FP64 outside pass (adjoint_mfma.hip), one set per workgroup of
+// its grid.
 int ensure_adj_scratch(pcsf_batch* b, size_t need) {
   pcsf_ctx* c = b->m->ctx;
   if (b->adj_scratch >= need) return PCSF_OK;

@@ -188,7 +188,7 @@ struct pcsf_batch {
   // record, then per pair lpr at the differentiated scales, d lpr / d rho and
   // the sum over columns of (d ln z / d rho)^2
   double* d_gres = nullptr;
-  double* d_adj_scratch = nullptr;  // FP64 outside pass: node tiles per resident wave
+  double* d_adj_scratch = nullptr;  // FP64 outside pass: node tiles per workgroup
   size_t adj_scratch = 0;           // its size in doubles
   // the settings each set of `rs` was last built from and those of its
   // reference basis (host), valid while a pass fits in one chunk (set k is
