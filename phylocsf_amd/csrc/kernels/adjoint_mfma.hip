@@ -34,8 +34,9 @@
 // 100vertebrates; 12 such regions 1973 -> 1081 there; 60 regions of 800 10787
 // -> 9991.  The small calls are a chain of products a quarter as long; the
 // large ones wait for memory (26 GB of messages and w at 3.2 TB/s with the
-// matrix cores 46% busy), where reloading P's fragments costs 2.0 of 8.0 ms,
-// the leaf gathers 1.1 and the inside pass's stores 1.2.
+// matrix cores 46% busy), where reloading P's fragments cost 2.0 of 8.0 ms,
+// the leaf gathers 1.1 and the inside pass's stores 1.2; with the gathers by
+// pairs of lanes it is 7.6.
 #include "outside_rows.hpp"
 
 namespace {
@@ -132,23 +133,33 @@ __global__ __launch_bounds__(kNT, 2) void adjoint_rows_kernel(AdjointArgs p) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) prior[v] = p.pi[pq * 64 + 16 * wave + 4 * v + g];
     __syncthreads();
-    // own rows of the message of node c, a leaf's from P's columns, an internal
-    // node's from its slot (an absent one: something in range)
+    // the message of node c, a leaf's from P's columns (by pairs of lanes: own()
+    // when it is used), an internal node's own rows from its slot (an absent one:
+    // something in range)
+    const uint32_t piece = g * 32u + (j & 1) * 16u;
+    auto two = [&](int lf) -> uint32_t {  // the codes of this pair's columns
+      return *reinterpret_cast<const uint16_t*>(codes_s + lf * 16 + (j & ~1));
+    };
     auto message = [&](int c, bool on) -> f64x4 {
       const bool slot = on && c >= nl;
       const int lf = on && !slot ? c : 0;
-      uint32_t row = codes_s[lf * 16 + j];
-      row = row == PCSF_MARGINALIZE || !on ? 64 : row;
-      asm volatile("" : "+v"(row));
+      uint32_t w2 = two(lf);
+      if (!on) w2 = 64u << 8 | 64u;
+      asm volatile("" : "+v"(w2));
+      const uint32_t even = min(w2 & 0xffu, 64u), odd = min(w2 >> 8, 64u);  // 255: `Marginalize
       return w.read(slot, (slot ? c - nl : 0) * (kSlot * 8u), lf * (kTile64 * 8u) + wave * 128u,
-                    row * 512u + g * 32u);
+                    even * 512u + piece, odd * 512u + piece);
     };
-    auto leaf_q = [&](int c) -> f64x4 {  // own rows of Q m_c for a leaf c (zeros otherwise)
+    auto leaf_q = [&](int c) -> f64x4 {  // Q m_c for a leaf c, by pairs (zeros otherwise)
       const int lf = c < nl ? c : 0;
-      uint32_t off = codes_s[lf * 16 + j];
-      off = off == PCSF_MARGINALIZE || c >= nl ? kNowhere : off * 512u + g * 32u;
-      asm volatile("" : "+v"(off));
-      return load4(rT, off, lf * 32768u + wave * 128u);
+      const uint32_t w2 = two(lf), e = w2 & 0xffu, o = w2 >> 8;
+      uint32_t even = e == PCSF_MARGINALIZE || c >= nl ? kNowhere : e * 512u + piece;
+      uint32_t odd = o == PCSF_MARGINALIZE || c >= nl ? kNowhere : o * 512u + piece;
+      asm volatile("" : "+v"(even), "+v"(odd));
+      const uint32_t so = lf * 32768u + wave * 128u;
+      const double2 x = __builtin_bit_cast(double2, pcsf_mfma::bload4(rT, even, so));
+      const double2 y = __builtin_bit_cast(double2, pcsf_mfma::bload4(rT, odd, so));
+      return (f64x4){x.x, x.y, y.x, y.y};
     };
     auto kids = [&](int k) {
       const int2 v = BIG ? make_int2(p.lc[nl + k], p.rc[nl + k]) : node[k];
@@ -162,7 +173,7 @@ __global__ __launch_bounds__(kNT, 2) void adjoint_rows_kernel(AdjointArgs p) {
     settle();
 #pragma unroll 1
     for (int k = 0; k < nin - 1; ++k) {
-      w.share((lastl ? last : ml) * (lastr ? last : mr));
+      w.share((lastl ? last : own(ml, kd.x < nl, lane)) * (lastr ? last : own(mr, kd.y < nl, lane)));
       w.operand(B);
       kd = kids(k + 1);
       lastl = kd.x == nl + k;
@@ -176,8 +187,8 @@ __global__ __launch_bounds__(kNT, 2) void adjoint_rows_kernel(AdjointArgs p) {
                              in ? (nl + k + 1) * (kTile64 * 8u) : (uint32_t)(n - 2) * 32768u);
       w.put(k, last);
     }
-    ml = lastl ? last : ml;
-    mr = lastr ? last : mr;
+    ml = lastl ? last : own(ml, kd.x < nl, lane);
+    mr = lastr ? last : own(mr, kd.y < nl, lane);
     const double zp = over_groups(dot4(ml * mr, prior));
     if (g == 0) part[wave][j] = zp;
     __syncthreads();
@@ -218,7 +229,7 @@ __global__ __launch_bounds__(kNT, 2) void adjoint_rows_kernel(AdjointArgs p) {
       mk = right ? mr : ml;
     };
     kd = kids(nin - 1);
-    descend(nin - 1, kd, prior, ml, mr, leaf_q(kd.x), leaf_q(kd.y));
+    descend(nin - 1, kd, prior, ml, mr, own(leaf_q(kd.x), true, lane), own(leaf_q(kd.y), true, lane));
     kd = kids(max(nin - 2, 0));
     ml = message(kd.x, true);
     mr = message(kd.y, true);
@@ -257,7 +268,8 @@ __global__ __launch_bounds__(kNT, 2) void adjoint_rows_kernel(AdjointArgs p) {
       }
       ++w.kx;
       branch_done(nl + k, dot4(mk, qa));
-      descend(k, c, acc, ml, mr, d0, d1);
+      descend(k, c, acc, own(ml, c.x < nl, lane), own(mr, c.y < nl, lane), own(d0, true, lane),
+              own(d1, true, lane));
     };
     settle();
     f64x4 ln, rn;
