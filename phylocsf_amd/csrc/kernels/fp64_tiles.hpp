@@ -1,6 +1,7 @@
 // fp64_tiles.hpp -- FP64 64 x 16 column tiles on v_mfma_f64_16x16x4f64,
-// shared by the FP64 matrix-core kernels (the outside pass and forward in
-// adjoint_mfma.hip, the E-step in estep.hip).
+// shared by the FP64 matrix-core kernels that give a wave whole columns (the
+// generated programs' forward in prune_fp64m.hpp, the E-step's passes in
+// estep.hip, the cherry tables in pbuild.hip).
 //
 // A wave owns 16 columns as a 64 x 16 tile: lane j + 16 g holds column j,
 // rows 16 mo + 4 v + g in element v of r[mo] -- the accumulator layout of
@@ -25,41 +26,6 @@ constexpr int kWaves = 4;                    // waves per workgroup
 constexpr int kCols = 16 * kWaves;           // columns per workgroup (= kAlignCols)
 static_assert(kCols == kAlignCols, "a workgroup covers one region-aligned block");
 constexpr int kTileDoubles = 64 * 16;        // one 64 x 16 tile
-
-// A 64 x 64 matrix M into LDS in A-fragment order: M[row][col] goes to
-// ((row / 16) * 16 + col / 4) * 64 + (row % 16) + 16 (col % 4).  `src`
-// gives M either as M[row][col] = src[row * 64 + col] (by_rows) or as
-// M[row][col] = src[col * 64 + row]; the global reads run in src order.
-// fetch() takes a thread's share (elements tid + 256 k) into registers, so
-// that the next tile's reads are in flight during a matrix product; put()
-// writes the share to LDS.
-constexpr int kShare = 4096 / (64 * kWaves);
-struct Share {
-  double v[kShare];
-};
-__device__ __forceinline__ void fetch(Share& r, const double* __restrict__ src, int tid) {
-#pragma unroll
-  for (int k = 0; k < kShare; ++k) r.v[k] = src[tid + 64 * kWaves * k];
-}
-__device__ __forceinline__ void put(double* __restrict__ frag, const Share& r, bool by_rows,
-                                    int tid) {
-#pragma unroll
-  for (int k = 0; k < kShare; ++k) {
-    const int e = tid + 64 * kWaves * k, hi = e >> 6, lo = e & 63;
-    const int row = by_rows ? hi : lo, col = by_rows ? lo : hi;
-    frag[((row >> 4) * 16 + (col >> 2)) * 64 + (row & 15) + 16 * (col & 3)] = r.v[k];
-  }
-}
-// both at once, a few elements at a time (fewer registers)
-__device__ __forceinline__ void stage(double* __restrict__ frag, const double* __restrict__ src,
-                                      bool by_rows, int tid) {
-#pragma unroll 4
-  for (int e = tid; e < 4096; e += 64 * kWaves) {
-    const int hi = e >> 6, lo = e & 63;
-    const int row = by_rows ? hi : lo, col = by_rows ? lo : hi;
-    frag[((row >> 4) * 16 + (col >> 2)) * 64 + (row & 15) + 16 * (col & 3)] = src[e];
-  }
-}
 
 typedef __attribute__((address_space(3))) double L3;
 typedef __attribute__((address_space(3))) void* LdsPtr;
