@@ -31,6 +31,11 @@ constexpr int kMaxSlots = 6;
 constexpr uint32_t kPfTable = 0x80000000u;  // word3 of a GEMM: a table row is issued ahead
 constexpr int kPfLeafMax = 0xfff, kPfTableMax = 0x7f;
 
+// The branch whose tile a kernel reads for the op in words w0, w1: a product's
+// own; branch 0's, which every tree has, for the root (no product: what is read
+// is not used, but a tree of two leaves has no branch above its leaves').
+constexpr int step_branch(int w0, int w1) { return (w0 & 0xff) == OP_GEMM ? w1 & 0xffff : 0; }
+
 namespace pcsf {
 
 struct Program {

@@ -248,13 +248,13 @@ __global__ __launch_bounds__(kNT, 2) void prune_fp64r_kernel(MfmaParams p, int s
       return uniform(prog[e], prog[e + 1]);
     };
     // step s's leaf messages and product's tile.  Operands that the op does
-    // not have are loads that read nothing (the root's tile is any tile): a
+    // not have are loads that read nothing (the root's tile is branch 0's): a
     // branch around the loads would move registers at its join
     auto fetch = [&](const Step& s, f64x4 (&l0)[CT], f64x4 (&l1)[CT], double (&a)[16]) {
       const int op = s.e0 & 0xff;
       w.leaf(l0, s.e1 & 0xffff, op != OP_MULPOP);
       w.leaf(l1, (s.e1 >> 16) & 0xffff, op == OP_CHERRY);
-      w.tile(a, (s.g0 & 0xff) == OP_GEMM ? s.g1 & 0xffff : p.nl);
+      w.tile(a, step_branch(s.g0, s.g1));
     };
 #pragma unroll
     for (int i = 0; i < NA - 1; ++i) {
