@@ -1109,6 +1109,7 @@ int pcsf_model_transition(pcsf_model* m, int model, double rho, double* P_out) {
   if (model < 0 || model >= m->nm) return set_err(c, PCSF_EINVAL, "model index out of range");
   if (!rho_valid(rho))
     return set_err(c, PCSF_EINVAL, "CamlPaml.P14n.instantiate_tree: domain violation on variable 0");
+  HIP_TRY(c, hipSetDevice(c->device));
   std::vector<double> r(m->nm, rho);
   int rc = ensure_transitions(m, r.data(), kFragF32, kBuildP64, nullptr);
   if (rc) return rc;
@@ -1623,7 +1624,6 @@ int eval_shared(pcsf_batch* b, const double* x, int K, int precision, std::vecto
   if (rc0) return rc0;
   // the ring must not wrap (and be reused) between these passes
   if (c->pin_used + room > c->pin_cap) HIP_TRY(c, ctx_wait(c));
-  HIP_TRY(c, hipSetDevice(c->device));
   std::vector<const double*> got(K);
   for (int k = 0; k < K; ++k) {
     const std::vector<double> r(m->nm, x[k]);
@@ -2246,6 +2246,7 @@ int pcsf_score(pcsf_batch* b, int strategy, int precision, double* score, double
   if (m->tree_only) return set_err(c, PCSF_EINVAL, kTreeOnly);
   if (m->nm != 2)
     return set_err(c, PCSF_EINVAL, "pcsf_score: needs exactly two models (coding, noncoding)");
+  HIP_TRY(c, hipSetDevice(c->device));
   const int R = b->nreg;
   const double db = 10.0 / std::log(10.0);
   std::vector<double> l(2 * (size_t)R), e(2 * (size_t)R), r(2 * (size_t)R, 1.0);
