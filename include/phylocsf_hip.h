@@ -289,7 +289,10 @@ int pcsf_model_specialized(pcsf_model *m, int enable, int *available);
  * n_regions*n_models each) and the kernel times when timing is enabled.
  * pcsf_backward does not change them (its passes reduce into buffers of
  * their own); pcsf_score with an mle strategy runs forwards of its own, so
- * afterwards they hold its last evaluation's values. */
+ * afterwards they hold its last evaluation's values.  Each array is 256-byte
+ * aligned.  Work on other streams may read them until the batch's next forward
+ * or its destruction; pcsf_batch_destroy of a batch whose pointers were asked
+ * for waits for the device. */
 int pcsf_batch_device_results(pcsf_batch *b, const double **d_loglik, const double **d_elpr);
 int pcsf_batch_last_timing(const pcsf_batch *b, double *prune_ms, double *reduce_ms,
                            double *pbuild_ms);

@@ -448,7 +448,7 @@ int fetch_results(pcsf_batch* b, const double* d_res, size_t np,
                   const char* where) {
   pcsf_model* m = b->m;
   pcsf_ctx* c = m->ctx;
-  const size_t count = 1 + np * out.size();
+  const size_t count = result_at(np, (int)out.size());
   hipError_t e;
   std::vector<double> h;
   double* p = reinterpret_cast<double*>(pin_take(c, count * 8, &e));
@@ -468,9 +468,9 @@ int fetch_results(pcsf_batch* b, const double* d_res, size_t np,
       return rc;
     }
   }
-  size_t k = 0;
+  int k = 0;
   for (double* o : out) {
-    if (o) std::memcpy(o, p + 1 + np * k, np * 8);
+    if (o) std::memcpy(o, p + result_at(np, k), np * 8);
     ++k;
   }
   return PCSF_OK;
@@ -1137,11 +1137,11 @@ hipError_t alloc_batch(pcsf_batch* b) {
   if (e == hipSuccess) e = dalloc(c, &b->d_offsets, (size_t)b->nreg + 1);
   if (e == hipSuccess) e = dalloc(c, &b->d_logz, (size_t)m->nm * b->ld);
   if (e == hipSuccess) e = dalloc(c, &b->d_colelpr, (size_t)m->nm * b->ld);
-  if (e == hipSuccess) e = dalloc(c, &b->d_res, 1 + 2 * np);
-  if (e == hipSuccess) e = dalloc(c, &b->d_gres, 1 + 3 * np);
+  if (e == hipSuccess) e = dalloc(c, &b->d_res, result_at(np, 2));
+  if (e == hipSuccess) e = dalloc(c, &b->d_gres, result_at(np, 3));
   if (e != hipSuccess) return e;
-  b->d_loglik = b->d_res + 1;
-  b->d_elpr = b->d_loglik + np;
+  b->d_loglik = b->d_res + result_at(np, 0);
+  b->d_elpr = b->d_res + result_at(np, 1);
   return hipSuccess;
 }
 
@@ -1269,6 +1269,12 @@ int pcsf_batch_create_frames(pcsf_model* m, const uint8_t* nuc, int64_t n_nuc,
 
 void pcsf_batch_destroy(pcsf_batch* b) {
   if (!b) return;
+  // results that a caller may still be reading on a stream of their own: wait
+  // for the device before any block of the batch finds a new user
+  if (b->handed_out) {
+    pool().release(b->d_res);
+    b->d_res = nullptr;
+  }
   dfree(b->d_codes);
   dfree(b->d_offsets);
   dfree(b->d_logz);
@@ -1606,7 +1612,7 @@ int eval_shared(pcsf_batch* b, const double* x, int K, int precision, std::vecto
                 std::vector<double>* e) {
   pcsf_model* m = b->m;
   pcsf_ctx* c = m->ctx;
-  const size_t n = (size_t)b->nreg * m->nm, count = 1 + 2 * n;
+  const size_t n = (size_t)b->nreg * m->nm, count = result_at(n, 2);
   for (int k = 0; k < K; ++k) {
     l[k].assign(n, 0.0);
     e[k].assign(n, 0.0);
@@ -1645,8 +1651,8 @@ int eval_shared(pcsf_batch* b, const double* x, int K, int precision, std::vecto
       const std::vector<double> r(m->nm, x[k]);
       return failed_build(m, key, r.data(), false);
     }
-    std::memcpy(l[k].data(), got[k] + 1, n * 8);
-    std::memcpy(e[k].data(), got[k] + 1 + n, n * 8);
+    std::memcpy(l[k].data(), got[k] + result_at(n, 0), n * 8);
+    std::memcpy(e[k].data(), got[k] + result_at(n, 1), n * 8);
   }
   return PCSF_OK;
 }
@@ -2363,6 +2369,7 @@ int pcsf_backward(pcsf_batch* b, const double* grad_loglik, double* grad_rho,
 
 int pcsf_batch_device_results(pcsf_batch* b, const double** d_loglik, const double** d_elpr) {
   if (!b) return PCSF_EINVAL;
+  b->handed_out = true;
   if (d_loglik) *d_loglik = b->d_loglik;
   if (d_elpr) *d_elpr = b->d_elpr;
   return PCSF_OK;

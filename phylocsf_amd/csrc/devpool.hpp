@@ -77,6 +77,12 @@ class DevPool {
     it->second.blocks.emplace(was.bytes, p);
     it->second.bytes += was.bytes;
   }
+  // back to the driver, not kept: for memory whose address a caller may have
+  // given to streams of their own (hipFree waits for the whole device)
+  void release(void* p) {
+    std::lock_guard<std::mutex> lock(mu_);
+    if (live_.erase(p)) (void)hipFree(p);
+  }
 
  private:
   struct Kept {

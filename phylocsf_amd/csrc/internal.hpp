@@ -162,6 +162,10 @@ struct Aligned {
   std::vector<int64_t> block0;      // per region: first block
 };
 
+// Where array k of the results of np pairs begins (doubles from the failure
+// record), each 256-byte aligned.
+inline size_t result_at(size_t np, int k) { return 32 + (np + 31) / 32 * 32 * k; }
+
 struct pcsf_batch {
   pcsf_model* m = nullptr;
   int64_t ncols = 0, ld = 0;  // ld = padded column count (multiple of kGroupCols)
@@ -170,10 +174,11 @@ struct pcsf_batch {
   int64_t* d_offsets = nullptr;    // nreg + 1
   double* d_logz = nullptr;        // nm * ld
   double* d_colelpr = nullptr;     // nm * ld
-  // the P builder's failure record, then loglik and elpr (nreg * nm each)
+  // the P builder's failure record, then loglik and elpr (result_at)
   double* d_res = nullptr;
   double* d_loglik = nullptr;      // nreg * nm (in d_res)
   double* d_elpr = nullptr;        // nreg * nm (in d_res)
+  bool handed_out = false;         // a caller has the addresses of the two
   hipEvent_t ev[6] = {};
   float t_pbuild = 0, t_prune = 0, t_reduce = 0;
   std::vector<int64_t> offsets;     // host copy

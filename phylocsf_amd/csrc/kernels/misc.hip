@@ -150,8 +150,8 @@ hipError_t launch_region_reduce_aligned(const pcsf_batch* b, const RegionChunk& 
   const uint8_t* active = (ch.sets == &b->m->fixed) ? nullptr : ch.sets->d_active;
   hipLaunchKernelGGL(region_reduce_aligned_kernel, grid, dim3(256), 0, s, b->d_alogz,
                      b->d_acolelpr, b->d_offsets, b->al.d_astart, active, ch.r0,
-                     b->m->nm, b->al.ld, res + 1, res + 1 + np,
-                     res == b->d_gres ? res + 1 + 2 * np : nullptr, b->m->d_perr, res);
+                     b->m->nm, b->al.ld, res + result_at(np, 0), res + result_at(np, 1),
+                     res == b->d_gres ? res + result_at(np, 2) : nullptr, b->m->d_perr, res);
   return hipGetLastError();
 }
 
