@@ -1316,6 +1316,15 @@ int pcsf_batch_codes(pcsf_batch* b, uint8_t* codes, int64_t* region_offsets) {
 
 namespace {
 
+// A forward at one tree scale per model has succeeded: pcsf_backward
+// differentiates it.
+void note_forward(pcsf_batch* b, const double* r, int precision) {
+  const int nm = b->m->nm;
+  b->last_rho.resize((size_t)b->nreg * nm);
+  b->last_precision = precision;
+  for (int32_t i = 0; i < b->nreg; ++i) std::copy(r, r + nm, b->last_rho.begin() + (size_t)i * nm);
+}
+
 // The forward of every region at one tree scale per model, enqueued: results
 // (and, with `later`, the P builder's failure record) in the batch's d_res.
 int shared_pass(pcsf_batch* b, const double* r, int precision, bool later) {
@@ -1330,10 +1339,6 @@ int shared_pass(pcsf_batch* b, const double* r, int precision, bool later) {
     if ((rc = ensure_aligned(b))) return rc;
   }
   b->t_pbuild = tp;
-  b->last_rho.resize((size_t)b->nreg * m->nm);
-  b->last_precision = precision;
-  for (int32_t i = 0; i < b->nreg; ++i)
-    for (int q = 0; q < m->nm; ++q) b->last_rho[(size_t)i * m->nm + q] = r[q];
   if (c->timing) {
     HIP_TRY(c, ensure_events(b));
     HIP_TRY(c, hipEventRecord(b->ev[0], c->stream));
@@ -1411,6 +1416,7 @@ int pcsf_forward(pcsf_batch* b, const double* rho, int rho_per_region, int preci
     m->built = 0;
     return rc;
   }
+  note_forward(b, r.data(), precision);
   if (c->timing) {
     HIP_TRY(c, hipEventElapsedTime(&b->t_prune, b->ev[0], b->ev[1]));
     HIP_TRY(c, hipEventElapsedTime(&b->t_reduce, b->ev[1], b->ev[2]));
@@ -1645,12 +1651,13 @@ int eval_shared(pcsf_batch* b, const double* x, int K, int precision, std::vecto
   for (int k = 0; k < K; ++k) {
     unsigned long long key;
     std::memcpy(&key, got[k], 8);
+    const std::vector<double> r(m->nm, x[k]);
     if (key != ~0ull) {
       m->cached_rho.clear();
       m->built = 0;
-      const std::vector<double> r(m->nm, x[k]);
       return failed_build(m, key, r.data(), false);
     }
+    note_forward(b, r.data(), precision);
     std::memcpy(l[k].data(), got[k] + result_at(n, 0), n * 8);
     std::memcpy(e[k].data(), got[k] + result_at(n, 1), n * 8);
   }

@@ -49,7 +49,9 @@ __global__ __launch_bounds__(256) void region_reduce_kernel(
     double* __restrict__ head) {
   __shared__ double s0[256], s1[256];
   const int r = blockIdx.x, q = blockIdx.y, tid = threadIdx.x;
-  if (head && r == 0 && q == 0 && tid == 0) *head = __longlong_as_double((long long)*perr);
+  const unsigned long long failed = head ? *perr : ~0ull;
+  if (head && r == 0 && q == 0 && tid == 0) *head = __longlong_as_double((long long)failed);
+  if (failed != ~0ull) return;  // the results stay those of the last good forward
   const int64_t lo = off[r], hi = off[r + 1];
   double a = 0.0, b = 0.0;
   for (int64_t c = lo + tid; c < hi; c += 256) {
@@ -100,8 +102,11 @@ __global__ __launch_bounds__(256) void region_reduce_aligned_kernel(
     const unsigned long long* __restrict__ perr, double* __restrict__ head) {
   __shared__ double s0[256], s1[256], s2[256];
   const int r = r0 + blockIdx.x, q = blockIdx.y, tid = threadIdx.x;
-  // the failure record of the pass's P build travels with its results
-  if (blockIdx.x == 0 && q == 0 && tid == 0) *head = __longlong_as_double((long long)*perr);
+  // the failure record of the pass's P build travels with its results; after a
+  // failure they stay those of the last good pass
+  const unsigned long long failed = *perr;
+  if (blockIdx.x == 0 && q == 0 && tid == 0) *head = __longlong_as_double((long long)failed);
+  if (failed != ~0ull) return;
   if (active && !active[(size_t)blockIdx.x * nm + q]) return;
   const int64_t lo = astart[r], hi = lo + (off[r + 1] - off[r]);
   double a = 0.0, b = 0.0, d = 0.0;
