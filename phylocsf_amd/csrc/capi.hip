@@ -300,6 +300,21 @@ int run_pbuild(pcsf_model* m, PSets& ps, int nsets, const double* rho_host, int 
   return PCSF_OK;
 }
 
+// A pass with a P build whose check comes with its results.  One that ends
+// before those are looked at (done) leaves no record behind for the next call to
+// report as its own, nor sets that count as built.
+struct DeferredBuild {
+  pcsf_model* m;
+  bool pending;
+  void done() { pending = false; }
+  ~DeferredBuild() {
+    if (!pending) return;
+    (void)hipMemsetAsync(m->d_perr, 0xff, sizeof(unsigned long long), m->ctx->stream);
+    m->cached_rho.clear();
+    m->built = 0;
+  }
+};
+
 // Transition sets of the fixed scales rho[0 .. nm) (one per model) holding
 // `need` (kBuild* outputs), P tiles in format fmt, and the cherry tables where
 // the MFMA kernels will read them; what the model already holds at these
@@ -528,6 +543,7 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
   const bool one_chunk = chunk_regions >= b->nreg;
   // one chunk: a failed P build is reported with the results
   const bool later = one_chunk && !c->timing;
+  DeferredBuild build{m, later};
   bool ran = false;
   if (!one_chunk) {
     b->eig_ok.clear();
@@ -625,11 +641,8 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
             ? launch_forward_fp64m(m, b, ch, c->stream)
         : fp64 ? launch_prune_fp64_regions(m, b, ch, c->stream)
                : launch_prune_mfma_regions(m, b, precision, variant, ch, c->stream);
-    if (e == hipErrorInvalidValue && precision == PCSF_FP64) {
-      // (the build's failure record goes unread)
-      (void)hipMemsetAsync(m->d_perr, 0xff, sizeof(unsigned long long), c->stream);
+    if (e == hipErrorInvalidValue && precision == PCSF_FP64)
       return set_err(c, PCSF_EINVAL, "FP64 kernel: tree workspace exceeds 64 KiB of LDS");
-    }
     HIP_TRY(c, e);
     if (c->timing) HIP_TRY(c, hipEventRecord(b->ev[1], c->stream));
     HIP_TRY(c, launch_region_reduce_aligned(b, ch, b->d_res, c->stream));
@@ -643,8 +656,10 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
       b->t_reduce += r;
     }
   }
-  return fetch_results(b, b->d_res, (size_t)b->nreg * nm, {loglik, elpr}, later && ran, rho, own,
-                       " (region block from 0)");
+  rc = fetch_results(b, b->d_res, (size_t)b->nreg * nm, {loglik, elpr}, later && ran, rho, own,
+                     " (region block from 0)");
+  if (!rc) build.done();
+  return rc;
 }
 
 // Gradient pass at tree scales rho (nreg * nm) over the pairs in `active`
@@ -667,6 +682,7 @@ int adjoint_regions(pcsf_batch* b, const double* rho, const uint8_t* active, dou
   if ((rc = ensure_region_sets(b, need, false))) return rc;
   const int chunk_regions = b->rs.cap / nm;
   const bool later = chunk_regions >= b->nreg && !c->timing;
+  DeferredBuild build{m, later};
   bool ran = false;
   std::vector<uint8_t> act;
   for (int32_t r0 = 0; r0 < b->nreg; r0 += chunk_regions) {
@@ -704,8 +720,10 @@ int adjoint_regions(pcsf_batch* b, const double* rho, const uint8_t* active, dou
     HIP_TRY(c, e);
     HIP_TRY(c, launch_region_reduce_aligned(b, ch, b->d_gres, c->stream));
   }
-  return fetch_results(b, b->d_gres, (size_t)b->nreg * nm, {loglik, grad, gsq}, later && ran, rho,
-                       false, "");
+  rc = fetch_results(b, b->d_gres, (size_t)b->nreg * nm, {loglik, grad, gsq}, later && ran, rho,
+                     false, "");
+  if (!rc) build.done();
+  return rc;
 }
 
 // ---- scratch of pcsf_forward_noalloc ---------------------------------------
@@ -1354,10 +1372,8 @@ int shared_pass(pcsf_batch* b, const double* r, int precision, bool later) {
     e = b->nreg > 0 ? launch_forward_fp64m(m, b, all, c->stream) : hipSuccess;
   } else if (precision == PCSF_FP64) {
     e = launch_prune_fp64(m, b, c->stream);
-    if (e == hipErrorInvalidValue) {
-      (void)hipMemsetAsync(m->d_perr, 0xff, sizeof(unsigned long long), c->stream);
+    if (e == hipErrorInvalidValue)
       return set_err(c, PCSF_EINVAL, "FP64 kernel: tree workspace exceeds 64 KiB of LDS");
-    }
   } else if (frag_format(precision) >= 0) {
     e = launch_prune_mfma(m, b, precision, m->mfma_variant[precision], c->stream);
   } else {
@@ -1406,16 +1422,14 @@ int pcsf_forward(pcsf_batch* b, const double* rho, int rho_per_region, int preci
                      "CamlPaml.P14n.instantiate_tree: domain violation on variable 0");
   HIP_TRY(c, hipSetDevice(c->device));
   const std::vector<double> r(rho, rho + m->nm);
+  DeferredBuild build{m, !c->timing && b->nreg > 0};
   int rc = shared_pass(b, r.data(), precision, !c->timing);
   if (rc) return rc;
   const size_t nres = (size_t)b->nreg * m->nm;
   rc = fetch_results(b, b->d_res, nres, {loglik, elpr}, !c->timing && b->nreg > 0, r.data(), false,
                      "");
-  if (rc) {
-    m->cached_rho.clear();
-    m->built = 0;
-    return rc;
-  }
+  if (rc) return rc;
+  build.done();
   note_forward(b, r.data(), precision);
   if (c->timing) {
     HIP_TRY(c, hipEventElapsedTime(&b->t_prune, b->ev[0], b->ev[1]));
@@ -1636,6 +1650,7 @@ int eval_shared(pcsf_batch* b, const double* x, int K, int precision, std::vecto
   if (rc0) return rc0;
   // the ring must not wrap (and be reused) between these passes
   if (c->pin_used + room > c->pin_cap) HIP_TRY(c, ctx_wait(c));
+  DeferredBuild build{m, true};
   std::vector<const double*> got(K);
   for (int k = 0; k < K; ++k) {
     const std::vector<double> r(m->nm, x[k]);
@@ -1652,15 +1667,12 @@ int eval_shared(pcsf_batch* b, const double* x, int K, int precision, std::vecto
     unsigned long long key;
     std::memcpy(&key, got[k], 8);
     const std::vector<double> r(m->nm, x[k]);
-    if (key != ~0ull) {
-      m->cached_rho.clear();
-      m->built = 0;
-      return failed_build(m, key, r.data(), false);
-    }
+    if (key != ~0ull) return failed_build(m, key, r.data(), false);
     note_forward(b, r.data(), precision);
     std::memcpy(l[k].data(), got[k] + result_at(n, 0), n * 8);
     std::memcpy(e[k].data(), got[k] + result_at(n, 1), n * 8);
   }
+  build.done();
   return PCSF_OK;
 }
 

@@ -12,6 +12,7 @@
 #include <functional>
 #include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -36,6 +37,7 @@ long n_malloc = 0, n_free = 0, n_wait = 0, n_foreign = 0;
 double fail_rho = -1.0;       // a P build at this tree scale fails
 int fail_launch = 0;          // countdown: the n-th launch of `fail_kernel` fails
 std::string fail_kernel;
+hipError_t last_error = hipSuccess;
 struct Config {
   dim3 grid, block;
   size_t lds;
@@ -165,7 +167,7 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
   p->multiProcessorCount = 256;
   return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return std::exchange(last_error, hipSuccess); }
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 
 hipError_t hipMalloc(void** p, size_t bytes) {
@@ -261,7 +263,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, hipStream_t s) {
   const std::string& name = kernels[f];
   if (fail_launch > 0 && name.find(fail_kernel) != std::string::npos && --fail_launch == 0)
-    return hipErrorLaunchFailure;
+    return last_error = hipErrorLaunchFailure;
   launched.push_back(name);
   if (of(s)->device != device_now) ++n_foreign;
   if (auto run = emulate(name, grid, args)) of(s)->work.push_back(run);

@@ -44,3 +44,58 @@ def test_destroy_waits_for_readers_of_device_results(on_fake):
     del b
     assert fake.fake_count(FREES) == 0 and fake.fake_count(WAITS) == 0
     """)
+
+
+@pytest.mark.parametrize("kernel,nth", [("region_reduce", 2), ("prune", 3)])
+def test_error_between_passes_leaves_no_failure_record(on_fake, kernel, nth):
+    """A launch that fails after a failed build of the same call: the next calls, at good
+    scales, are not told of that build."""
+    on_fake("""
+    ctx = P.Context(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "12flies")
+    for strategy in ("mle", "mle_grad"):
+        b = batch(m, 2, 70)
+        fake.fake_fail_rho(0.01 if strategy == "mle" else float(np.exp(-2.0)))
+        fake.fake_fail_launch(%r, %d)
+        try:
+            P.score(b, strategy, P.PCSF_FP64M)
+        except P.Failure:
+            raise
+        except P.PcsfError as e:
+            assert e.code == _lib.PCSF_EDEVICE
+        else:
+            raise AssertionError("no error")
+        b.forward(1.0, P.PCSF_FP64M)
+        b.forward(np.full((2, 2), 1.5), P.PCSF_FP64M, per_region=True)
+        m.transition(0, 1.0)
+    """ % (kernel.encode(), nth))
+
+
+def test_refused_forward_leaves_no_built_sets(on_fake):
+    """FP64 on a tree whose workspace exceeds LDS is refused; a failed build in front of it
+    must not count as built."""
+    on_fake("""
+    ctx = P.Context(0)
+    text = "a0:0.1"
+    for i in range(1, 200):
+        text = "(%s,a%d:0.1)%s" % (text, i, ":0.1" if i < 199 else "")
+    prefix = P.paramset_prefix("12flies")
+    ecms = [P.import_parameters(prefix + "_%s.ECM" % w) for w in ("coding", "noncoding")]
+    m = P.PhyloCSFModel(ctx, P.newick_tree(text + ";"), ecms)
+    b = batch(m, 2, 5)
+    fake.fake_fail_rho(2.5)
+    for per_region in (False, True):
+        try:
+            b.forward(np.full((2, 2), 2.5) if per_region else 2.5, P.PCSF_FP64, per_region=per_region)
+        except P.InvalidArgument as e:
+            assert "LDS" in str(e)
+        else:
+            raise AssertionError("not refused")
+        for _ in range(2):
+            try:
+                m.transition(0, 2.5)
+            except P.Failure:
+                continue
+            raise AssertionError("a failed build passed for a good one")
+        m.transition(0, 1.0)
+    """)
