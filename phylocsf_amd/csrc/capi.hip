@@ -2587,8 +2587,9 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
 }
 
 // Likelihoods and root posteriors for small alphabets (lik_small_kernel): one
-// upload of the states and one launch per chunk.  Without leaf_dist the kernel
-// checks the states (*bad_state: one is below -1; nothing is written then).
+// upload of the states and one launch per chunk.  With bad_state the states are
+// still to be checked (*bad_state: one is below -1; nothing is written then):
+// by the kernel, or here in front of the first of several chunks.
 hipError_t lik_small(pcsf_ctx* c, int k, int n, const std::vector<int32_t>& lc,
                      const std::vector<int32_t>& rc, const double* P, const double* prior,
                      const int32_t* leaves, const double* leaf_dist, int64_t ncols, double* z,
@@ -2603,6 +2604,12 @@ hipError_t lik_small(pcsf_ctx* c, int k, int n, const std::vector<int32_t>& lc,
   const size_t per_col = (size_t)nl * 4 + (leaf_dist ? (size_t)nl * k * 8 : 0) + 8 + (size_t)k * 8;
   const int64_t chunk = std::min<int64_t>(
       ncols, std::max<int64_t>(64, (int64_t)(((size_t)512 << 20) / per_col) / 64 * 64));
+  if (bad_state) {
+    int32_t vmin = 0;
+    for (int64_t e = 0; chunk < ncols && e < ncols * nl; ++e) vmin = std::min(vmin, leaves[e]);
+    *bad_state = vmin < -1;
+    if (*bad_state) return hipSuccess;
+  }
   const int grid = (int)std::min<int64_t>((chunk + 63) / 64, 4096);
   int32_t *d_tree = nullptr, *d_leaves = nullptr, *d_bad = nullptr;
   double *d_P = nullptr, *d_dist = nullptr, *d_out = nullptr, *d_ws = nullptr;
@@ -2654,7 +2661,7 @@ hipError_t lik_small(pcsf_ctx* c, int k, int n, const std::vector<int32_t>& lc,
                          hipMemcpyDeviceToHost, c->stream));
     chk(ctx_wait(c));
   }
-  *bad_state = bad != 0;
+  if (bad_state) *bad_state = bad != 0;
   dfree(d_tree);
   dfree(d_bad);
   dfree(d_P);
@@ -2714,9 +2721,8 @@ int lik_impl(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P
   if (ncols == 0) return PCSF_OK;
   HIP_TRY(c, hipSetDevice(c->device));
   if (small) {
-    bool bad = false;
     HIP_TRY(c, lik_small(c, k, n, lc, rc, P, prior, leaves, dist ? leaf_dist : nullptr, ncols, z,
-                         root_post, &bad));
+                         root_post, nullptr));
     return PCSF_OK;
   }
   const bool estep = ecounts != nullptr;

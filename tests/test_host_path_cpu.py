@@ -99,3 +99,31 @@ def test_refused_forward_leaves_no_built_sets(on_fake):
             raise AssertionError("a failed build passed for a good one")
         m.transition(0, 1.0)
     """)
+
+
+@pytest.mark.parametrize("column", [0, -1])
+def test_bad_state_writes_nothing(on_fake, column):
+    """A leaf state that PhyloLik's columns refuse, in the first or in a later chunk of the
+    columns: no output has been written."""
+    on_fake("""
+    ctx = P.Context(0)
+    nl, ncols = 2000, 70000  # 512 MB a chunk: two
+    kids = [[0, 1]] + [[nl + i, i + 2] for i in range(nl - 2)]
+    kids = np.array(kids, np.int32)
+    Pm = np.zeros((2 * nl - 2, 4, 4))
+    prior = np.full(4, 0.25)
+    leaves = np.zeros((ncols, nl), np.int32)
+    z, post = np.full(ncols, -7.0), np.full((ncols, 4), -7.0)
+    dp, ip = C.POINTER(C.c_double), C.POINTER(C.c_int32)
+
+    def call():
+        return L.pcsf_lik_columns(ctx.h, 4, 2 * nl - 1, kids.ctypes.data_as(ip), Pm.ctypes.data_as(dp),
+                                  prior.ctypes.data_as(dp), leaves.ctypes.data_as(ip), ncols,
+                                  z.ctypes.data_as(dp), post.ctypes.data_as(dp))
+
+    leaves[%d, 3] = -2
+    assert call() == _lib.PCSF_EINVAL
+    assert (z == -7.0).all() and (post == -7.0).all()
+    leaves[:, 3] = 1
+    assert call() == 0 and (z == 1.0).all() and launches("lik_small") >= 2
+    """ % column)
