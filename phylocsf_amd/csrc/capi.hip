@@ -2586,6 +2586,20 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
   return PCSF_OK;
 }
 
+// Workgroups of lik_small_kernel over ncols columns (0: the column kernel takes
+// them).  Each holds the alpha of 64 columns, (n - nl) K 512 bytes of memory:
+// five per CU are as fast as more (66,000 columns of 120 leaves: 1.37 ms at k = 4
+// and 5.4 at k = 20; 2.1 and 15.8 with one per CU, the column kernel 9.4 and
+// 30.4), as many as 2 GiB hold on larger trees, and where those would leave CUs
+// idle (from some 700 leaves at k > 16) the column kernel's workspace is the
+// smaller one.
+int lik_small_grid(const pcsf_ctx* c, int k, int n, int64_t ncols) {
+  const size_t bytes = (size_t)(n - (n + 1) / 2) * lik_small_states(k) * 512;
+  const int64_t want = std::min<int64_t>((ncols + 63) / 64, 5 * c->num_cus);
+  const int64_t fit = (int64_t)(((size_t)2 << 30) / bytes);
+  return fit >= std::min<int64_t>(want, c->num_cus) ? (int)std::min(want, fit) : 0;
+}
+
 // Likelihoods and root posteriors for small alphabets (lik_small_kernel): one
 // upload of the states and one launch per chunk.  With bad_state the states are
 // still to be checked (*bad_state: one is below -1; nothing is written then):
@@ -2610,7 +2624,7 @@ hipError_t lik_small(pcsf_ctx* c, int k, int n, const std::vector<int32_t>& lc,
     *bad_state = vmin < -1;
     if (*bad_state) return hipSuccess;
   }
-  const int grid = (int)std::min<int64_t>((chunk + 63) / 64, 4096);
+  const int grid = lik_small_grid(c, k, n, chunk);
   int32_t *d_tree = nullptr, *d_leaves = nullptr, *d_bad = nullptr;
   double *d_P = nullptr, *d_dist = nullptr, *d_out = nullptr, *d_ws = nullptr;
   hipError_t e = hipSuccess;
@@ -2692,7 +2706,8 @@ int lik_impl(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P
     sib[a] = b;
     sib[b] = a;
   }
-  const bool small = lik_small_states(k) > 0 && !ecounts && post_mode != 2 && ncols > 0;
+  const bool small = lik_small_states(k) > 0 && !ecounts && post_mode != 2 && ncols > 0 &&
+                     lik_small_grid(c, k, n, ncols) > 0;
   double* root_post = post_mode == 1 ? post : nullptr;
   if (small && columns_entry) {  // its kernel checks the states
     HIP_TRY(c, hipSetDevice(c->device));

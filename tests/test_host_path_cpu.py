@@ -127,3 +127,27 @@ def test_bad_state_writes_nothing(on_fake, column):
     leaves[:, 3] = 1
     assert call() == 0 and (z == 1.0).all() and launches("lik_small") >= 2
     """ % column)
+
+
+@pytest.mark.parametrize("k,nl,ncols", [(20, 1000, 20000), (4, 5000, 30000), (20, 300, 100000),
+                                        (4, 300, 100000), (20, 4000, 300)])
+def test_small_alphabet_memory_is_bounded(on_fake, k, nl, ncols):
+    """PhyloLik's columns hold at most the 512 MB of a chunk, 2 GiB of workspace (or the
+    column kernel's 2,048 columns) and the tree's P, however large the tree."""
+    on_fake("""
+    k, nl, ncols = %d, %d, %d
+    ctx = P.Context(0)
+    kids = np.array([[0, 1]] + [[nl + i, i + 2] for i in range(nl - 2)], np.int32)
+    n = 2 * nl - 1
+    Pm, prior, z = np.zeros((n - 1, k, k)), np.full(k, 1.0 / k), np.zeros(ncols)
+    leaves = np.zeros((ncols, nl), np.int32)
+    dp, ip = C.POINTER(C.c_double), C.POINTER(C.c_int32)
+    before = fake.fake_used(0)
+    fake.fake_reset()
+    assert L.pcsf_lik_columns(ctx.h, k, n, kids.ctypes.data_as(ip), Pm.ctypes.data_as(dp),
+                              prior.ctypes.data_as(dp), leaves.ctypes.data_as(ip), ncols,
+                              z.ctypes.data_as(dp), None) == 0
+    assert launches("lik_small") + launches("lik_columns") > 0
+    bound = (512 << 20) + max(2 << 30, 2048 * 2 * n * k * 8) + 2 * Pm.nbytes
+    assert fake.fake_peak(0) - before <= 1.15 * bound, fake.fake_peak(0) - before
+    """ % (k, nl, ncols))
