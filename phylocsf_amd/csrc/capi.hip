@@ -2593,8 +2593,22 @@ int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
 // 30.4), as many as 2 GiB hold on larger trees, and where those would leave CUs
 // idle (from some 700 leaves at k > 16) the column kernel's workspace is the
 // smaller one.
+// A lane's chain over the nodes is longer than a wave's over one column, the more
+// so at large k, where P's scalar loads no longer fit: a few columns are faster
+// with a wave each.  us at 300 / 1000 / 2500 / 6000 columns, column kernel against
+// this one: 12 leaves, k = 20: 346 / 351 / 434 / 591 against 380 / 397 / 403 / 428;
+// 58 leaves, k = 20: 561 / 576 / 1301 / 1923 against 1631 / 1595 / 1567 / 1628, k = 16:
+// 482 / 508 / 838 / 1454 against 550 / 552 / 545 / 603; 120 leaves, k = 20: 855 / 1226 /
+// 2050 / 3440 against 3242 / 3165 / 3136 / 3203, k = 9: 597 / 634 / 1440 / 2082 against
+// 1030 / 1027 / 1028 / 1110, k = 5: 484 / 548 / 779 / 1252 against 556 / 552 / 544 / 608.
+// 12 leaves up to k = 16, 58 up to k = 8 and every tree at k <= 4 are faster here at
+// any size.
 int lik_small_grid(const pcsf_ctx* c, int k, int n, int64_t ncols) {
-  const size_t bytes = (size_t)(n - (n + 1) / 2) * lik_small_states(k) * 512;
+  const int inner = n - (n + 1) / 2, K = lik_small_states(k);
+  if ((K == 8 && inner > 64 && ncols < 1024) || (K == 16 && inner > 32 && ncols < 2048) ||
+      (K == 24 && ncols < std::min(6144, 2048 + 48 * inner)))
+    return 0;
+  const size_t bytes = (size_t)inner * K * 512;
   const int64_t want = std::min<int64_t>((ncols + 63) / 64, 5 * c->num_cus);
   const int64_t fit = (int64_t)(((size_t)2 << 30) / bytes);
   return fit >= std::min<int64_t>(want, c->num_cus) ? (int)std::min(want, fit) : 0;
