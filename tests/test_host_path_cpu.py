@@ -151,3 +151,21 @@ def test_small_alphabet_memory_is_bounded(on_fake, k, nl, ncols):
     bound = (512 << 20) + max(2 << 30, 2048 * 2 * n * k * 8) + 2 * Pm.nbytes
     assert fake.fake_peak(0) - before <= 1.15 * bound, fake.fake_peak(0) - before
     """ % (k, nl, ncols))
+
+
+@pytest.mark.parametrize("first,then", [("FP16S", "FP64M"), ("FP64M", "FP32"), ("FP64", "FP64M")])
+def test_set_budget_bounds_all_kinds_together(on_fake, first, then):
+    """A pass that adds a kind of transition matrix to sets that fill the budget goes through
+    in more chunks, not in twice the memory."""
+    on_fake("""
+    ctx = P.Context(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "12flies")
+    b = batch(m, 60, 3)
+    rho = np.full((60, 2), 1.5)
+    assert b.forward(rho, P.PCSF_%s, per_region=True)[0].shape == (60, 2)
+    assert launches("region_reduce_aligned") == 1
+    fake.fake_reset()
+    got = b.forward(rho, P.PCSF_%s, per_region=True)[0]
+    assert launches("region_reduce_aligned") == 2
+    assert (abs(got[:, 0] + 100 * (np.log(1.5) - 0.3) ** 2) < 1e-9).all()
+    """ % (first, then), env={"PHYLOCSF_SET_BUDGET_MB": "100"})
