@@ -412,14 +412,17 @@ int ensure_aligned(pcsf_batch* b) {
 // force many chunks, which the tests use).  2,000 regions on 100vertebrates take
 // the same time with 4, 8 and 24 GiB (mle in split FP16 296 / 295 / 302 ms, mle_grad
 // 211 / 209 / 211); with 12 the sets stay within the 16 GiB that the context's pool
-// keeps, so that calls of any size find their memory there.
-size_t set_budget() {
+// keeps, so that calls of any size find their memory there.  Sets with rate models
+// of their own have 24 GiB: in one chunk a pass starts their eigensystems from
+// those of the pass before or keeps them, in several it builds them all anew
+// (omega test of 700 regions on 58mammals: 635 ms in one chunk, 975 in two).
+size_t set_budget(bool own) {
   const char* e = std::getenv("PHYLOCSF_SET_BUDGET_MB");
   if (e && *e) {
     const long long mb = std::atoll(e);
     if (mb > 0) return (size_t)mb << 20;
   }
-  return (size_t)12 << 30;
+  return (size_t)(own ? 24 : 12) << 30;
 }
 
 // Bytes of one transition set on the device.
@@ -442,7 +445,7 @@ int ensure_region_sets(pcsf_batch* b, unsigned need, bool own) {
   PSets& rs = b->rs;
   const bool keep = rs.cap > 0 && own == (rs.d_eVT != nullptr);
   const unsigned all = need | (keep ? rs.outputs : 0);
-  int cap = (int)std::max<size_t>(m->nm, set_budget() / set_bytes(m, all, own) / m->nm * m->nm);
+  int cap = (int)std::max<size_t>(m->nm, set_budget(own) / set_bytes(m, all, own) / m->nm * m->nm);
   cap = std::min<int>(cap, std::max(m->nm, b->nreg * m->nm));
   if (rs.cap >= cap && keep && !(need & ~rs.outputs)) return PCSF_OK;
   b->eig_ok.clear();

@@ -169,3 +169,20 @@ def test_set_budget_bounds_all_kinds_together(on_fake, first, then):
     assert launches("region_reduce_aligned") == 2
     assert (abs(got[:, 0] + 100 * (np.log(1.5) - 0.3) ** 2) < 1e-9).all()
     """ % (first, then), env={"PHYLOCSF_SET_BUDGET_MB": "100"})
+
+
+def test_large_omega_call_goes_through_in_one_chunk(on_fake):
+    """3,000 regions of 58mammals, 24 GB of sets with rate models of their own, take as many
+    passes as ten regions: one chunk, in which a pass starts from the last one's
+    eigensystems."""
+    on_fake("""
+    ctx = P.Context(0)
+    tree = P.newick_tree(open(P.paramset_prefix("58mammals") + ".nh").read())
+    m = P.PhyloCSFModel.tree_only(ctx, tree)
+    passes = []
+    for regions in (10, 3000):
+        fake.fake_reset()
+        P.score_omega(batch(m, regions, 1), precision=P.PCSF_FP64M)
+        passes.append(launches("region_reduce_aligned"))
+    assert passes[0] == passes[1] > 20, passes
+    """)
