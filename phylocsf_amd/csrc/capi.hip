@@ -335,7 +335,7 @@ int ensure_transitions(pcsf_model* m, const double* rho, int fmt, unsigned need,
     const uint8_t all[8] = {1, 1, 1, 1, 1, 1, 1, 1};  // nm <= 8
     HIP_TRY(c, set_params(c, m->fixed, (size_t)m->nm, rho, all));
   }
-  if ((m->built & kBuildMfma) && m->fixed.fmt != fmt) m->built &= ~kBuildMfma;
+  if ((need & m->built & kBuildMfma) && m->fixed.fmt != fmt) m->built &= ~kBuildMfma;
   const bool tables = (need & kBuildMfma) && !m->cherries.empty() && !m->tables;
   if (tables) need |= kBuildP64M;  // the tables are products of the FP64 matrices
   const unsigned missing = need & ~m->built;

@@ -186,3 +186,26 @@ def test_large_omega_call_goes_through_in_one_chunk(on_fake):
         passes.append(launches("region_reduce_aligned"))
     assert passes[0] == passes[1] > 20, passes
     """)
+
+
+def test_alternating_precisions_keep_the_sets(on_fake):
+    """Forwards at one tree scale in FP64 and at an MFMA precision, and transition matrices in
+    between, build each kind once."""
+    on_fake("""
+    ctx = P.Context(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "12flies")
+    b = batch(m, 2, 70)
+
+    def turn():
+        b.forward(1.0, P.PCSF_FP16S)
+        b.forward(1.0, P.PCSF_FP64M)
+        m.transition(0, 1.0)
+        b.forward(1.0, P.PCSF_FP64)
+
+    turn()
+    fake.fake_reset()
+    turn()
+    assert launches("pbuild") == 0 and launches("cherry_table") == 0
+    b.forward(1.0, P.PCSF_FP32)  # another tile format: the tiles alone
+    assert launches("pbuild") == 1 and launches("cherry_table") == 0
+    """)
