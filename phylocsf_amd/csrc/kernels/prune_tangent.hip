@@ -38,13 +38,23 @@ hipError_t launch_prune_tangent_regions(const pcsf_model* m, const pcsf_batch* b
     const TreeProgram* t = static_cast<const TreeProgram*>(m->tree_p);
     if (t->tangent) return t->tangent(prm, PCSF_FP32, 0, m->ctx->num_cus, s);
   }
+  // The interpreter keeps every slot live through its dispatch: with two
+  // workgroups per CU it spills 20 registers at 2 slots, 78 at 3, 207 to 448 above,
+  // with one none up to 5 and 60 at 6.  us a launch with one / two, 60 regions of 800 columns: 23flies
+  // (2 slots) 858 / 689, 53birds (3) 2133 / 2120, 45 species of 58mammals (4) 1976 /
+  // 4162, 100 of 120mammals (5) 4340 / 9615; one region of 300: 117 / 117, 297 / 369, 272 /
+  // 511, 615 / 1202; 1,000 regions of 64: 53birds 2397 / 2904.  Two slots take two
+  // workgroups unless one finds a CU for every block (7yeast, 12 regions of 400: 40 / 42).
+  const int cus = m->ctx->num_cus;
   switch (m->slots) {
     case 1:
-    case 2: return launch_tangent_ns<2>(prm, m->ctx->num_cus, s);
-    case 3: return launch_tangent_ns<3>(prm, m->ctx->num_cus, s);
-    case 4: return launch_tangent_ns<4>(prm, m->ctx->num_cus, s);
-    case 5: return launch_tangent_ns<5>(prm, m->ctx->num_cus, s);
-    case 6: return launch_tangent_ns<6>(prm, m->ctx->num_cus, s);
+    case 2:
+      return prm.ngroups * prm.nm > cus ? launch_tangent_ns<2, 2>(prm, cus, s)
+                                        : launch_tangent_ns<2, 1>(prm, cus, s);
+    case 3: return launch_tangent_ns<3, 1>(prm, cus, s);
+    case 4: return launch_tangent_ns<4, 1>(prm, cus, s);
+    case 5: return launch_tangent_ns<5, 1>(prm, cus, s);
+    case 6: return launch_tangent_ns<6, 1>(prm, cus, s);
     default: return hipErrorInvalidValue;
   }
 }

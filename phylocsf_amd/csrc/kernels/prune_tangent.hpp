@@ -72,6 +72,8 @@ __device__ __forceinline__ f32x4 product_rule(const f32x4& t, const f32x4& m, co
   return r;
 }
 
+// AHEAD: an op's first leaf rows are loaded during the product before it
+template <bool AHEAD>
 struct TWalk {
   static constexpr int NT = 64 * kTWpg, GC = 16 * kTWpg;
   static constexpr int PER = 4096 / NT / 4;  // float4 per thread of a 4096-float tile
@@ -138,7 +140,7 @@ struct TWalk {
   }
   // the op's first leaf: loaded during the product before it (use_pf), or now
   __device__ __forceinline__ void first_leaf(TGathered& g, int leaf, bool use_pf) {
-    if (use_pf) {
+    if (AHEAD && use_pf) {
       g = pf;
       add_log(lpf);
     } else {
@@ -196,7 +198,7 @@ struct TWalk {
     const Rsrc rd = make_rsrc(p.Dfrag + (size_t)nset * p.nbr * 4096, p.nbr * 16384u);
     // (the code is read before the first copy starts: a read of the codes waits
     // for the copies in flight)
-    const bool ahead = pf_leaf != kNoBranch;
+    const bool ahead = AHEAD && pf_leaf != kNoBranch;
     const LeafAt leaf = leaf_at(pf, ahead ? pf_leaf : 0);
     if (ahead) lpf = leaf_log(leaf);
     __builtin_amdgcn_sched_barrier(0);
@@ -230,8 +232,7 @@ struct TWalk {
     // 11.0 -> 10.2 ms where each product had waited for the copies that it
     // started itself (Tbuf), 7.9 with the rows loaded ahead and, with fewer
     // loads counted wrongly and so fewer values held back in registers, two
-    // workgroups per CU (35 registers spilled; 593 before the diagonal's copy
-    // lost its branch).
+    // workgroups per CU.
     static_assert(PER == 4, "eight pieces per wave");
     f32x4 A[2][4];
     auto read = [&](int i) {
@@ -297,9 +298,12 @@ struct TWalk {
   }
 };
 
-template <int NS, class PROG>
-__global__ __launch_bounds__(64 * kTWpg, 2) void prune_tangent_kernel(MfmaParams p) {
-  constexpr int NT = TWalk::NT, GC = TWalk::GC, PER = TWalk::PER;
+// PERCU workgroups per CU: two in a generated program (100vertebrates: 35
+// registers spilled), what the interpreter takes by its slots in prune_tangent.hip.
+template <int NS, class PROG, int PERCU>
+__global__ __launch_bounds__(64 * kTWpg, PERCU) void prune_tangent_kernel(MfmaParams p) {
+  using W = TWalk<(NS < 6)>;  // (six slots leave no registers for a leaf's rows ahead)
+  constexpr int NT = W::NT, GC = W::GC, PER = W::PER;
   __shared__ __attribute__((aligned(16))) float Tbuf[2][kPairFloats];
   extern __shared__ __attribute__((aligned(16))) uint8_t codes_s[];  // nl x GC
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -329,8 +333,8 @@ __global__ __launch_bounds__(64 * kTWpg, 2) void prune_tangent_kernel(MfmaParams
       *reinterpret_cast<f32x4*>(&Tbuf[0][4096 + tid * 4]) =
           *reinterpret_cast<const f32x4*>(ps + 4096 + tid * 4);
   }
-  TWalk w{p, Tbuf, (TWalk::L3 (*)[kPairFloats])Tbuf, codes_s, tid, wave, lane, lane >> 4,
-          wave * 16 + (lane & 15)};
+  W w{p, Tbuf, (typename W::L3 (*)[kPairFloats])Tbuf, codes_s, tid, wave, lane, lane >> 4,
+      wave * 16 + (lane & 15)};
   for (;;) {
     Task nxt;
     int64_t jn = jc + 1;
@@ -361,9 +365,9 @@ __global__ __launch_bounds__(64 * kTWpg, 2) void prune_tangent_kernel(MfmaParams
   }
 }
 
-template <int NS, class PROG = Interp<NS>>
+template <int NS, int PERCU, class PROG = Interp<NS>>
 hipError_t launch_tangent_ns(const MfmaParams& prm, int num_cus, hipStream_t s) {
-  auto kern = prune_tangent_kernel<NS, PROG>;
+  auto kern = prune_tangent_kernel<NS, PROG, PERCU>;
   const size_t dyn = ((size_t)prm.nl * 16 * kTWpg + 15) / 16 * 16;
   int per_cu = 0;
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * kTWpg, dyn);
@@ -377,7 +381,7 @@ hipError_t launch_tangent_ns(const MfmaParams& prm, int num_cus, hipStream_t s) 
 // the forward's launcher signature; the tangent pass has one shape).
 template <class PROG>
 hipError_t launch_tangent_tree(const MfmaParams& prm, int, int, int cus, hipStream_t s) {
-  return launch_tangent_ns<PROG::NS, PROG>(prm, cus, s);
+  return launch_tangent_ns<PROG::NS, 2, PROG>(prm, cus, s);
 }
 
 }  // namespace pcsf_mfma
