@@ -32,12 +32,17 @@ hipError_t launch_forward_fp64m(const pcsf_model* m, const pcsf_batch* b, const 
   prm.off = b->d_offsets;
   if (prm.ngroups == 0) return hipSuccess;
   const int cus = m->ctx->num_cus;
-  // 64-column blocks of work.  Up to four per CU the row-split kernel is the
-  // faster one (58mammals: 251 against 285 us at 366 blocks, 529 against 556
-  // at 772), above it the generated program, which reads P once per 64
-  // columns (898 against 850 us at 1520 blocks, 3619 against 3207 at 6214).
+  // 64-column blocks of work.  While the row-split kernel finds a place for every
+  // 16 columns at once (two workgroups per CU: half a block per CU) it is the
+  // faster one; beyond, the generated program, which reads P once per 64 columns.
+  // us a forward at 64 / 128 / 160 / 256 / 512 / 1000 blocks on 256 CUs, row-split against
+  // generated: 12flies 39 / 47 / 57 / 60 / 91 / 164 against 51 / 53 / 53 / 55 / 78 / 139,
+  // 58mammals 82 / 122 / 182 / 193 / 349 / 663 against 154 / 161 / 163 / 173 / 292 / 562,
+  // 120mammals 142 / 217 / 409 / 423 / 800 / 1507 against 303 / 310 / 318 / 335 / 577 / 1100.
+  // With a set per region and many short regions, bound by the sets, the two are
+  // within 5% of each other from 100 blocks on.
   const int64_t blocks = ch.work > 0 ? ch.work : ch.nblocks * m->nm;
-  if (m->specialized && m->tree_p && blocks > 4 * (int64_t)cus) {
+  if (m->specialized && m->tree_p && blocks > cus / 2) {
     const auto* t = static_cast<const pcsf_mfma::TreeProgram*>(m->tree_p);
     if (t->fp64m) return t->fp64m(prm, 0, 0, cus, s);
   }

@@ -19,17 +19,16 @@
 // the loads hold the wave up until the memory pipeline has taken them (29
 // mammals, 14 blocks: 42 us in bursts, 33 us interleaved).  Live tiles below
 // the top of the program's stack wait in LDS, private to their lane, so the
-// depth needs no registers: 188 VGPRs and two workgroups per CU whatever the
-// tree, where the interpreter over prune_fp64m.hpp's layout kept every slot
+// depth needs no registers: 226 VGPRs (190 with two tiles) and two workgroups per
+// CU whatever the tree, where the interpreter over prune_fp64m.hpp's layout kept every slot
 // live through its dispatch (one workgroup per CU above three slots).
 //
 // Measured (us per forward over both models, against the column-per-wave
-// kernel): 29mammals, 37 columns 32 (74); 12flies, 100 columns 18 (34);
-// 58mammals, 366 blocks 251 (285), 772 blocks 529 (556), 1520 blocks 898
-// (850), 6214 blocks 3619 (3207), the last with the tree's generated program
-// on the other side; 53birds, which has none, 8182 blocks 4310 (5069).  What
-// bounds it at size is the traffic of P from L2 (32 KB per product for 16 CT
-// columns where the other kernel stages it once for 64).
+// kernel of the time): 29mammals, 37 columns 32 (74); 12flies, 100 columns 18 (34);
+// 53birds, which has no generated program, 8182 blocks 4310 (5069).  What bounds
+// it at size is the traffic of P from L2 (32 KB per product for 16 CT columns
+// where the other kernel stages it once for 64): a tree's generated program takes
+// over where these workgroups no longer all fit (prune_fp64m.hip has the figures).
 //
 // Every element is the same sum in the same order as in prune_fp64m.hpp
 // (K-steps ascending from zero, leaf factors and siblings multiplied in the
