@@ -2,20 +2,25 @@
 //
 // A batch lives for one call in the usual program (the command line scores
 // each alignment once), and hipMalloc / hipFree cost microseconds to hundreds
-// of milliseconds each (the driver clears what it hands out: a maximiser's
-// 20 GB of transition sets took 0.49 s of a 0.56 s call).  Freed blocks are
+// of milliseconds each, with the size and the state of the driver (a maximiser's
+// 20 GB of transition sets: under 10 ms on some machines, half a second on
+// others, where the driver clears what it hands out).  Freed blocks are
 // kept per context and handed out again to that context only: its work is
 // ordered on one stream, so a block's next user runs after its last one.  At
-// most kKeep bytes are kept; beyond it, at the context's end, and when the
-// device runs out of memory (any context's), blocks go back to the driver.
+// most kKeep bytes are kept, the latest freed; beyond it, at the context's end,
+// and when the device runs out of memory (any context's), blocks go back to the
+// driver.  No lock is held while the driver allocates or frees, which can wait
+// for the device.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
 #include <cstdint>
+#include <list>
 #include <map>
 #include <mutex>
 #include <unordered_map>
+#include <vector>
 
 namespace pcsf {
 
@@ -32,62 +37,111 @@ class DevPool {
   }
   // the context's stream has drained
   void close(uint64_t id) {
-    std::lock_guard<std::mutex> lock(mu_);
-    auto it = kept_.find(id);
-    if (it == kept_.end()) return;
-    give_back(it->second, 0);
-    kept_.erase(it);
+    std::vector<void*> out;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      auto it = kept_.find(id);
+      if (it == kept_.end()) return;
+      it->second.take_oldest(0, &out);
+      kept_.erase(it);
+    }
+    to_driver(out);
   }
   hipError_t alloc(uint64_t id, size_t bytes, void** out) {
-    const size_t size = rounded(bytes);
-    std::lock_guard<std::mutex> lock(mu_);
-    auto it = kept_.find(id);
-    if (it != kept_.end()) {
-      // the smallest kept block that fits without wasting half of itself
-      auto b = it->second.blocks.lower_bound(size);
-      if (b != it->second.blocks.end() && b->first <= 2 * size) {
-        *out = b->second;
-        live_[*out] = {b->first, id};
-        it->second.bytes -= b->first;
-        it->second.blocks.erase(b);
+    size_t size = rounded(bytes);
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      auto it = kept_.find(id);
+      if (it != kept_.end() && (*out = it->second.take_fitting(&size))) {
+        live_[*out] = {size, id};
         return hipSuccess;
       }
     }
     hipError_t e = hipMalloc(out, size);
     if (e == hipErrorOutOfMemory) {
+      // one thread at a time, so that none gives up while another gives back
+      std::lock_guard<std::mutex> lock_empty(empty_);
       (void)hipGetLastError();
-      for (auto& k : kept_) give_back(k.second, 0);
+      std::vector<void*> all;
+      {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (auto& k : kept_) k.second.take_oldest(0, &all);
+      }
+      to_driver(all);
       e = hipMalloc(out, size);
     }
-    if (e == hipSuccess) live_[*out] = {size, id};
+    if (e == hipSuccess) {
+      std::lock_guard<std::mutex> lock(mu_);
+      live_[*out] = {size, id};
+    }
     return e;
   }
   void free(void* p) {
-    std::lock_guard<std::mutex> lock(mu_);
-    auto l = live_.find(p);
-    if (l == live_.end()) return;
-    const Live was = l->second;
-    live_.erase(l);
-    auto it = kept_.find(was.id);
-    if (it == kept_.end() || was.bytes > kKeep) {
-      (void)hipFree(p);
-      return;
+    std::vector<void*> out;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      auto l = live_.find(p);
+      if (l == live_.end()) return;
+      const Live was = l->second;
+      live_.erase(l);
+      auto it = kept_.find(was.id);
+      if (it == kept_.end() || was.bytes > kKeep) {
+        out.push_back(p);
+      } else {
+        it->second.take_oldest(kKeep - was.bytes, &out);
+        it->second.put(was.bytes, p);
+      }
     }
-    give_back(it->second, kKeep - was.bytes);
-    it->second.blocks.emplace(was.bytes, p);
-    it->second.bytes += was.bytes;
+    to_driver(out);
   }
   // back to the driver, not kept: for memory whose address a caller may have
   // given to streams of their own (hipFree waits for the whole device)
   void release(void* p) {
-    std::lock_guard<std::mutex> lock(mu_);
-    if (live_.erase(p)) (void)hipFree(p);
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      if (!live_.erase(p)) return;
+    }
+    (void)hipFree(p);
   }
 
  private:
   struct Kept {
-    std::multimap<size_t, void*> blocks;
+    struct Block {
+      size_t bytes;
+      void* p;
+    };
+    std::list<Block> by_age;  // the oldest first
+    std::multimap<size_t, std::list<Block>::iterator> by_size;
     size_t bytes = 0;
+
+    void put(size_t n, void* p) {
+      by_age.push_back({n, p});
+      by_size.emplace(n, std::prev(by_age.end()));
+      bytes += n;
+    }
+    // the smallest block that fits without wasting half of itself (its size in
+    // *size), or nullptr
+    void* take_fitting(size_t* size) {
+      auto b = by_size.lower_bound(*size);
+      if (b == by_size.end() || b->first > 2 * *size) return nullptr;
+      void* p = b->second->p;
+      *size = b->first;
+      bytes -= b->first;
+      by_age.erase(b->second);
+      by_size.erase(b);
+      return p;
+    }
+    void take_oldest(size_t down_to, std::vector<void*>* out) {
+      while (bytes > down_to) {
+        const Block b = by_age.front();
+        auto r = by_size.equal_range(b.bytes);
+        while (r.first->second != by_age.begin()) ++r.first;
+        by_size.erase(r.first);
+        by_age.pop_front();
+        bytes -= b.bytes;
+        out->push_back(b.p);
+      }
+    }
   };
   struct Live {
     size_t bytes;
@@ -101,16 +155,11 @@ class DevPool {
     return (n + step - 1) / step * step;
   }
   // hipFree waits for the device, so a block still in use there is safe to give
-  static void give_back(Kept& k, size_t down_to) {
-    while (k.bytes > down_to) {
-      auto b = std::prev(k.blocks.end());
-      (void)hipFree(b->second);
-      k.bytes -= b->first;
-      k.blocks.erase(b);
-    }
+  static void to_driver(const std::vector<void*>& blocks) {
+    for (void* p : blocks) (void)hipFree(p);
   }
 
-  std::mutex mu_;
+  std::mutex mu_, empty_;
   uint64_t last_ = 0;
   std::unordered_map<uint64_t, Kept> kept_;
   std::unordered_map<void*, Live> live_;

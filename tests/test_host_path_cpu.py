@@ -209,3 +209,63 @@ def test_alternating_precisions_keep_the_sets(on_fake):
     b.forward(1.0, P.PCSF_FP32)  # another tile format: the tiles alone
     assert launches("pbuild") == 1 and launches("cherry_table") == 0
     """)
+
+
+def test_pool_keeps_the_latest_blocks(on_fake):
+    """Calls that repeat find their memory kept, also after larger or other ones: of more
+    than 16 GiB the blocks freed first go back to the driver."""
+    on_fake("""
+    ctx = P.Context(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "58mammals")
+
+    def call(regions):
+        b = batch(m, regions, 1)
+        for precision in (P.PCSF_FP16S, P.PCSF_FP64M):
+            b.forward(np.full((regions, 2), 1.5), precision, per_region=True)
+
+    base = fake.fake_used(0)
+    for regions in (150, 700, 290, 800):  # 2.3, 10.6, 4.4 and 12.2 GB of sets
+        for turn in range(4):
+            fake.fake_reset()
+            call(regions)
+            if turn > 1:
+                assert fake.fake_count(MALLOCS) == fake.fake_count(FREES) == 0, (regions, turn)
+        assert fake.fake_used(0) - base <= 16 << 30
+    ctx2 = P.Context(0)  # another context does not get this one's
+    m2 = P.PhyloCSFModel.from_paramset(ctx2, "12flies")
+    fake.fake_reset()
+    batch(m2, 1, 1).forward(1.0, P.PCSF_FP64M)
+    assert fake.fake_count(MALLOCS) > 0
+    """)
+
+
+def test_pool_gives_back_when_memory_runs_out(on_fake):
+    """An allocation that fails empties every context's kept memory and is tried again; a
+    context's end gives back what it kept."""
+    on_fake("""
+    ctx, ctx2 = P.Context(0), P.Context(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "58mammals")
+    m2 = P.PhyloCSFModel.from_paramset(ctx2, "58mammals")
+
+    def call(m, regions):
+        b = batch(m, regions, 1)
+        return b.forward(np.full((regions, 2), 1.5), P.PCSF_FP64M, per_region=True)
+
+    call(m, 1200)
+    fake.fake_capacity(fake.fake_used(0) + (1 << 30))
+    want = call(m2, 600)
+    assert fake.fake_used(0) < 8 << 30  # the first context's 9 GB went back
+    try:
+        call(m2, 1400)  # 10.6 GB do not fit: everything kept goes back, and it still fails
+        fake.fake_capacity(0)
+    except P.PcsfError as e:
+        assert e.code == _lib.PCSF_ENOMEM
+    fake.fake_capacity(288 << 30)
+    assert (call(m2, 600)[0] == want[0]).all()
+    L.pcsf_model_destroy(m2.h)
+    m2.h = None
+    before = fake.fake_used(0)
+    L.pcsf_ctx_destroy(ctx2.h)
+    ctx2.h = None
+    assert fake.fake_used(0) <= before - (4 << 30)
+    """)
