@@ -1067,8 +1067,7 @@ int pcsf_model_create(pcsf_ctx* c, int n, const int32_t* children, const double*
   HIP_TRY(c, dalloc(c, &m->d_lsl_t, std::max<size_t>(1, lsl_t.size())));
   HIP_TRY(c, dalloc(c, &m->d_perr, (size_t)1));
   if (!tree_only)
-    HIP_TRY(c, alloc_psets(c, m->fixed, nm, m->nbr,
-                           kBuildMfma | kBuildP64 | kBuildP64M | kBuildP64MT,
+    HIP_TRY(c, alloc_psets(c, m->fixed, nm, m->nbr, kBuildMfma | kBuildP64 | kBuildP64M,
                            (int)m->cherries.size() / 3));
   HIP_TRY(c, hipMemset(m->d_perr, 0xff, sizeof(unsigned long long)));
   std::vector<int32_t> lc32(m->lc.begin(), m->lc.end()), rc32(m->rc.begin(), m->rc.end());

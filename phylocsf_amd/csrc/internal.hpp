@@ -256,16 +256,13 @@ struct AdjointArgs {
   const double* P64F;        // sets: P per branch (PSets::d_P64F layout)
   const double* P64FT;       // sets: P^T per branch in A-fragment order; a leaf's Q P by columns
   const double* QT;          // per model: Q^T
-  const double* pi;          // per model, or per set with prior_per_set
-  const double* lnpi;        // its logarithm
-  int prior_per_set;
+  const double* pi;          // per model
   const double* branch;      // nbr
   const int32_t* block_region;
   const int64_t* astart;
   const int64_t* off;
   const uint8_t* active;
   int r0;
-  int shared_sets;           // 1: set q for every region (the model's fixed sets)
   double* logz;              // nm x ald
   double* coldrho;           // nm x ald: d ln z / d rho per column
   double* grad_branch;       // (region - r0) x nm x nbr, added to (may be null)

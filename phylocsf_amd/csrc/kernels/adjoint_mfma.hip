@@ -111,7 +111,7 @@ __global__ __launch_bounds__(kNT, 2) void adjoint_rows_kernel(AdjointArgs p) {
     if (r < 0) continue;  // padding block (uniform over the workgroup)
     const int64_t len = p.off[r + 1] - p.off[r];
     if (b0 - p.astart[r] >= len) continue;  // no column of the region in this tile
-    const int set = p.shared_sets ? q : (r - p.r0) * nm + q;
+    const int set = (r - p.r0) * nm + q;
     if (!p.active[set]) continue;
     const int64_t col = b0 + j;
     const bool valid = col - p.astart[r] < len;
@@ -128,10 +128,9 @@ __global__ __launch_bounds__(kNT, 2) void adjoint_rows_kernel(AdjointArgs p) {
 #pragma unroll
     for (int s = 0; s < 16; ++s)
       Qf[s] = p.QT[(size_t)q * 4096 + (16 * wave + j) * 64 + 4 * s + g];
-    const int pq = p.prior_per_set ? set : q;
     f64x4 prior;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) prior[v] = p.pi[pq * 64 + 16 * wave + 4 * v + g];
+    for (int v = 0; v < 4; ++v) prior[v] = p.pi[q * 64 + 16 * wave + 4 * v + g];
     __syncthreads();
     // the message of node c, a leaf's from P's columns (by pairs of lanes: own()
     // when it is used), an internal node's own rows from its slot (an absent one:
@@ -325,9 +324,7 @@ AdjointArgs make_args(const pcsf_model* m, const pcsf_batch* b, const RegionChun
   a.P64F = ch.sets->d_P64F;
   a.P64FT = ch.sets->d_P64FT;
   a.QT = m->d_QT;
-  a.prior_per_set = ch.sets->d_epi ? 1 : 0;
-  a.pi = a.prior_per_set ? ch.sets->d_epi : m->d_pi;
-  a.lnpi = a.prior_per_set ? ch.sets->d_elnpi : m->d_lnpi;
+  a.pi = m->d_pi;
   a.branch = m->d_branch;
   a.block_region = b->al.d_block_region;
   a.astart = b->al.d_astart;
@@ -338,7 +335,6 @@ AdjointArgs make_args(const pcsf_model* m, const pcsf_batch* b, const RegionChun
   a.coldrho = b->d_acolelpr;
   a.grad_branch = nullptr;
   a.scratch = scratch;
-  a.shared_sets = ch.sets == &m->fixed ? 1 : 0;
   return a;
 }
 
@@ -347,8 +343,8 @@ AdjointArgs make_args(const pcsf_model* m, const pcsf_batch* b, const RegionChun
 hipError_t launch_adjoint_mfma(const pcsf_model* m, const pcsf_batch* b, const RegionChunk& ch,
                                const AdjointPlan& plan, double* grad_branch, double* scratch,
                                hipStream_t s) {
+  if (ch.sets->d_epi) return hipErrorInvalidValue;  // Q is per model
   AdjointArgs a = make_args(m, b, ch, scratch);
-  if (a.prior_per_set) return hipErrorInvalidValue;  // Q is per model
   a.grad_branch = grad_branch;
   if (ch.nblocks <= 0 || m->nm <= 0) return hipSuccess;
   const size_t codes = (size_t)m->nl * 16;

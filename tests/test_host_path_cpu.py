@@ -269,3 +269,20 @@ def test_pool_gives_back_when_memory_runs_out(on_fake):
     ctx2.h = None
     assert fake.fake_used(0) <= before - (4 << 30)
     """)
+
+
+def test_model_memory(on_fake):
+    """A model holds of its fixed sets what forwards and pcsf_model_transition read (per
+    branch two tiles of FP32, two of FP64), no transposes for the outside pass, which
+    runs on a batch's sets."""
+    on_fake("""
+    ctx = P.Context(0)
+    before = fake.fake_used(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "100vertebrates")
+    nbr = m.tree.n - 1
+    sets = 2 * nbr * (65 * 64 * 4 + 4160 * 4 + 65 * 8 + 4096 * 8 + 65 * 64 * 8)
+    tables = 2 * 65 * 65 * (64 * 4 + 8)  # per cherry
+    kids = np.asarray(m.tree.children).reshape(-1, 2)
+    cherries = int((kids < m.tree.nl).all(axis=1).sum())
+    assert fake.fake_used(0) - before <= 1.07 * (sets + cherries * tables)
+    """)
