@@ -83,6 +83,17 @@ std::function<void()> emulate(const std::string& name, dim3 grid, void** a) {
           *perr = std::min(*perr, ((((unsigned long long)k * nbr) * 64 + 1) * 65 + 2) << 2 | 1);
     };
   }
+  if (is("transpose_codes_kernel")) {
+    auto src = arg<const uint8_t*>(a, 0);
+    auto ncols = arg<int64_t>(a, 1);
+    auto nl = arg<int>(a, 2);
+    auto dst = arg<uint8_t*>(a, 3);
+    auto ld = arg<int64_t>(a, 4);
+    return [=] {
+      for (int64_t c = 0; c < ncols; ++c)
+        for (int l = 0; l < nl; ++l) dst[(size_t)l * ld + c] = src[(size_t)c * nl + l];
+    };
+  }
   if (is("region_reduce_aligned_kernel")) {
     auto active = arg<const uint8_t*>(a, 4);
     auto r0 = arg<int>(a, 5), nm = arg<int>(a, 6);

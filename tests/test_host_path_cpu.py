@@ -286,3 +286,45 @@ def test_model_memory(on_fake):
     cherries = int((kids < m.tree.nl).all(axis=1).sum())
     assert fake.fake_used(0) - before <= 1.07 * (sets + cherries * tables)
     """)
+
+
+def test_pinned_ring_wraps(on_fake):
+    """Uploads that go round the context's 1 MB ring: what is still to be copied is not
+    overwritten (the fake's streams copy as late as they may)."""
+    on_fake("""
+    ctx = P.Context(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "58mammals")
+    nl = m.tree.nl
+    rng = np.random.default_rng(2)
+    made = []
+    fake.fake_reset()
+    for k in range(45):  # 0.9 KB to 64 KB each, 1.5 MB in all, some past the small size
+        codes = rng.integers(0, 64, (25 * k + 16, nl)).astype(np.uint8)
+        made.append((P.Batch(m, codes, np.array([0, 7, len(codes)])), codes))
+    assert 1 <= fake.fake_count(WAITS) <= 3
+    for b, codes in made:
+        assert (b.codes()[0] == codes).all()
+    """)
+
+
+def test_results_larger_than_the_ring(on_fake):
+    """Shared scales together (one wait) and one by one where their results do not fit the
+    ring, results and set parameters beyond it: the same values."""
+    on_fake("""
+    ctx = P.Context(0)
+    tree = P.newick_tree(open(P.paramset_prefix("12flies") + ".nh").read(), ["dmel", "dsim"])
+    prefix = P.paramset_prefix("12flies")
+    ecms = [P.import_parameters(prefix + "_%s.ECM" % w) for w in ("coding", "noncoding")]
+    m = P.PhyloCSFModel(ctx, tree, ecms)
+    want = [-100 * (np.log(1.5) - 0.3 - 0.01 * q) ** 2 for q in range(2)]
+    for strategy in ("mle", "mle_grad"):
+        small = P.score(batch(m, 3, 1), strategy, P.PCSF_FP64M)
+        large = P.score(batch(m, 12000, 1), strategy, P.PCSF_FP64M)  # 4 x 384 KB
+        for key in ("lpr", "rho", "elpr"):
+            assert (large[key] == small[key][0]).all(), key
+    b = batch(m, 70000, 1)  # 2.2 MB of results, 1.3 MB of scales and flags
+    assert np.allclose(b.forward(1.5, P.PCSF_FP64M)[0], want)
+    fake.fake_reset()
+    got = b.forward(np.full((70000, 2), 1.5), P.PCSF_FP64M, per_region=True)[0]
+    assert launches("region_reduce_aligned") == 1 and np.allclose(got, want)
+    """, env={"PHYLOCSF_SET_BUDGET_MB": "30000"})
