@@ -1323,13 +1323,14 @@ int pcsf_batch_codes(pcsf_batch* b, uint8_t* codes, int64_t* region_offsets) {
   if (region_offsets) std::copy(b->offsets.begin(), b->offsets.end(), region_offsets);
   if (!codes || b->ncols == 0) return PCSF_OK;
   HIP_TRY(c, hipSetDevice(c->device));
-  // leaf-major rows of ld bytes on the device -> n_cols x nl on the host
-  std::vector<uint8_t> rows((size_t)m->nl * b->ncols);
-  HIP_TRY(c, hipMemcpy2D(rows.data(), b->ncols, b->d_codes, b->ld, b->ncols, m->nl,
-                         hipMemcpyDeviceToHost));
+  // leaf-major rows of ld bytes on the device -> n_cols x nl on the host.  (In one
+  // piece: hipMemcpy2D has returned success without a byte copied in a process
+  // profiled by one release's tools while torch brought another's runtime.)
+  std::vector<uint8_t> rows((size_t)m->nl * b->ld);
+  HIP_TRY(c, hipMemcpy(rows.data(), b->d_codes, rows.size(), hipMemcpyDeviceToHost));
   for (int l = 0; l < m->nl; ++l)
     for (int64_t k = 0; k < b->ncols; ++k)
-      codes[(size_t)k * m->nl + l] = rows[(size_t)l * b->ncols + k];
+      codes[(size_t)k * m->nl + l] = rows[(size_t)l * b->ld + k];
   return PCSF_OK;
 }
 

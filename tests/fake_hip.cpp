@@ -239,11 +239,6 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
   return drain_all(), std::memcpy(d, s, n), hipSuccess;
 }
-hipError_t hipMemcpy2D(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, hipMemcpyKind) {
-  drain_all();
-  for (size_t k = 0; k < h; ++k) std::memcpy((char*)d + k * dp, (const char*)s + k * sp, w);
-  return hipSuccess;
-}
 hipError_t hipMemset(void* d, int v, size_t n) { return drain_all(), std::memset(d, v, n), hipSuccess; }
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t q) {
   of(q)->work.push_back([=] { std::memset(d, v, n); });
