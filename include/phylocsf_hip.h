@@ -249,8 +249,8 @@ int pcsf_score(pcsf_batch *b, int strategy, int precision, double *score, double
  * in [0.001, 10] (half-Cauchy prior, mode 1, scale 0.5) then over kappa in
  * [1, 10] (gamma(7, 0.25) prior on kappa - 1), with F3x4 codon frequencies
  * counted from the region (:102-134).  The codon model (:21-80) is rebuilt
- * and diagonalised per (region, hypothesis, kappa) on the host; every
- * likelihood is a batched per-region forward on the GPU.
+ * and diagonalised per (region, hypothesis, kappa), and every likelihood is a
+ * batched per-region forward, on the GPU.
  * The batch's model is a tree-only model (pcsf_model_create with n_models =
  * 0) or any two-model model (its rate models are not used).
  * score in decibans (n_regions; anc_comp is not defined for this test);
@@ -268,8 +268,9 @@ int pcsf_score_omega(pcsf_batch *b, double omega_h1, double sigma_h1, int precis
  * this batch at tree scale 1,
  * `reps` launches each, keeps the fastest on the batch's model for later
  * forwards at that precision and returns the per-shape milliseconds in
- * ms_out[PCSF_N_VARIANTS].  Until then a model uses shape 2 if its tree has
- * generated programs (see pcsf_model_specialized), else shape 1.  No
+ * ms_out[PCSF_N_VARIANTS].  Until then a model uses shape 2 (shape 5 at
+ * PCSF_FP32) if its tree has generated programs (see pcsf_model_specialized),
+ * else shape 1.  No
  * counterpart in the reference (a tuning step of this implementation). */
 #define PCSF_N_VARIANTS 7
 int pcsf_autotune(pcsf_batch *b, int precision, int reps, double *ms_out, int *chosen);
@@ -278,7 +279,7 @@ int pcsf_autotune(pcsf_batch *b, int precision, int reps, double *ms_out, int *c
 int pcsf_set_variant(pcsf_model *m, int precision, int variant);
 /* Tree-specialised kernels: the library carries straight-line op programs
  * generated at build time for the shipped trees; a model whose tree matches
- * one uses it (FP32 and split-FP16 GEMMs, launch shapes 1, 2, 4 and 6) instead
+ * one uses it (FP32 and split-FP16 GEMMs, launch shapes 1, 2, 4, 5 and 6) instead
  * of the op-program interpreter.  enable = 1 / 0 allows / forbids them
  * (-1 leaves the setting); *available (may be NULL) gets 1 if the plain
  * program is specialised, | 2 if the cherry-table program is.  No

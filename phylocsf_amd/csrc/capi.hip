@@ -667,9 +667,10 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
 }
 
 // Gradient pass at tree scales rho (nreg * nm) over the pairs in `active`
-// (optional): per-region lpr into d_gloglik, d lpr / d rho into d_grad and
-// the sum over columns of (d ln z / d rho)^2 into d_gsq
-// (the per-column buffers of the forward hold the column values).  tangent = false: the FP64
+// (optional): per region and model lpr, d lpr / d rho and the sum over columns
+// of (d ln z / d rho)^2, in the batch's d_gres and in loglik, grad and gsq (host,
+// may be null; the per-column buffers of the forward hold the column values).
+// tangent = false: the FP64
 // outside-pass adjoint, which also accumulates, if d_gbr is given, the
 // per-region sums of d ln z / d t_br (nreg * nm * nbr); tangent = true: the
 // FP32 MFMA tangent pass (d lpr / d rho only).
@@ -2411,14 +2412,6 @@ int pcsf_batch_last_timing(const pcsf_batch* b, double* prune_ms, double* reduce
 
 namespace {
 
-// PhyloLik.prepare + likelihood + node_posterior + add_branch_posteriors
-// (lib/CamlPaml/PhyloLik.ml:46-174) over n_cols columns: the host side of
-// kernels/lik.hip.  Columns go in chunks whose device buffers stay within
-// ~512 MB; post_mode 1 = the root's posterior, 2 = every node's.
-// The E-step for 64 states without `Distribution leaves on the FP64 matrix
-// cores (kernels/estep.hip): columns in chunks of up to 32,768, message and
-// beta of every (internal node, column) of a chunk in device memory, the counts
-// added per chunk.
 // The context's E-step buffers for chunks of `chunk` columns (grown, never
 // shrunk; a failed growth leaves them released).
 hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk) {
@@ -2474,6 +2467,10 @@ hipError_t estep_cache(pcsf_ctx* c, int n, int64_t ldu, int64_t chunk) {
   return hipSuccess;
 }
 
+// The E-step for 64 states without `Distribution leaves on the FP64 matrix
+// cores (kernels/estep.hip): columns in chunks of up to 32,768, message and
+// beta of every (internal node, column) of a chunk in device memory, the counts
+// added per chunk.
 int estep_mfma(pcsf_ctx* c, int n, const std::vector<int32_t>& lc,
                const std::vector<int32_t>& rc, const double* P, const double* prior,
                const int32_t* leaves, int64_t ncols, const double* weights, double* z,
@@ -2704,6 +2701,12 @@ hipError_t lik_small(pcsf_ctx* c, int k, int n, const std::vector<int32_t>& lc,
   return e;
 }
 
+// PhyloLik.prepare + likelihood + node_posterior + add_branch_posteriors
+// (lib/CamlPaml/PhyloLik.ml:46-174) over n_cols columns: the host side of
+// kernels/lik.hip and kernels/estep.hip.  Columns of kernels/lik.hip go in chunks
+// whose inputs and outputs on the device stay within ~512 MB, beside a workspace
+// of the kernel's; post_mode 1 = the root's posterior, 2 = every node's.
+// columns_entry: pcsf_lik_columns, which refuses states below -1.
 int lik_impl(pcsf_ctx* c, int k, int n, const int32_t* children, const double* P,
              const double* prior, const int32_t* leaves, const double* leaf_dist, int64_t ncols,
              const double* weights, double* z, int post_mode, double* post, double* ecounts,

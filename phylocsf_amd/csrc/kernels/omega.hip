@@ -68,9 +68,6 @@ __device__ __forceinline__ double exchangeability(const double* qs, int i, int j
   return kp * op;
 }
 
-// mode per set: kEigCold builds from scratch and stores U in ref (64 x 64
-// per set), kEigWarm starts from ref, kEigKeep leaves the outputs (unchanged
-// settings, or an inactive set)
 // (x, y) <- (c x - s y, s x + c y)
 __device__ __forceinline__ void rotate(double c, double s, double& x, double& y) {
   const double a = fma(c, x, -(s * y));
@@ -119,6 +116,9 @@ __device__ __forceinline__ void put(double* A, const f64x4 (&t)[2], int tid) {
   }
 }
 
+// mode per set: kEigCold builds from scratch and stores U in ref (64 x 64
+// per set), kEigWarm starts from ref, kEigKeep leaves the outputs (unchanged
+// settings, or an inactive set)
 __global__ __launch_bounds__(kNT, 4) void omega_eigen_kernel(
     const double* __restrict__ qs_all, const uint8_t* __restrict__ mode, double* __restrict__ ref,
     double* __restrict__ VT, double* __restrict__ Vinv, double* __restrict__ lam,
