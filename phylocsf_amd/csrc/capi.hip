@@ -109,6 +109,20 @@ unsigned set_outputs(int precision) {
   return precision == PCSF_FP64M ? kBuildP64M : precision == PCSF_FP64 ? kBuildP64 : kBuildMfma;
 }
 
+// The fused kernel's launch shape: the one chosen for this model, or else three
+// waves per SIMD for the straight-line programs (the fastest shape on every
+// shipped tree measured), two for the interpreter, whose switch needs more
+// registers; the straight-line programs in FP32 with the next leaf's rows loaded
+// ahead (1.03 to 1.14 times as fast over 12 to 120 leaves and 1 to 1000 regions; in
+// split FP16, bound by those gathers themselves, 0.97 to 1.05; in the interpreter,
+// which a shipped tree takes where its program is forbidden, 0.35 to 1.0: 114
+// registers spilled).
+int launch_shape(const pcsf_model* m, int precision) {
+  if (m->mfma_variant[precision] >= 0) return m->mfma_variant[precision];
+  if (!m->tree_p || !m->tree_t) return 1;
+  return precision == PCSF_FP32 && m->specialized ? 5 : 2;
+}
+
 constexpr const char* kTreeOnly =
     "a tree-only model (made with n_models = 0) serves the omega test only";
 
@@ -553,7 +567,7 @@ int forward_regions(pcsf_batch* b, const double* rho, const uint8_t* active, int
     b->eig_ok.clear();
     b->eig_ref_ok.clear();
   }
-  int variant = fp64 ? 0 : m->mfma_variant[precision];
+  int variant = fp64 ? 0 : launch_shape(m, precision);
   if (16 * kMfmaVariants[variant].wpg * kMfmaVariants[variant].g > kAlignCols) variant = 1;
   std::vector<uint8_t> act, eigmode;
   b->t_pbuild = b->t_prune = b->t_reduce = 0.f;
@@ -1017,16 +1031,6 @@ int pcsf_model_create(pcsf_ctx* c, int n, const int32_t* children, const double*
   m->n_gemm = pg.n_gemm;
   m->tree_p = find_tree_program(m->prog, false);
   m->tree_t = find_tree_program(m->prog_t, true);
-  // default launch shape until pcsf_autotune: three waves per SIMD for the
-  // straight-line programs (the fastest shape on every shipped tree measured),
-  // two for the interpreter, whose switch needs more registers; in FP32 with
-  // the next leaf's rows loaded ahead (1.03 to 1.14 times as fast over 12 to
-  // 120 leaves and 1 to 1000 regions; in split FP16, bound by those gathers
-  // themselves, 0.97 to 1.05)
-  if (m->tree_p && m->tree_t) {
-    for (int& v : m->mfma_variant) v = 2;
-    m->mfma_variant[PCSF_FP32] = 5;
-  }
   if (m->slots > kMaxSlots)
     return set_err(c, PCSF_EINVAL, "tree needs more than 6 live partial tiles");
   if (!c) {  // host-only model: simulation and model facts, no device work
@@ -1380,7 +1384,7 @@ int shared_pass(pcsf_batch* b, const double* r, int precision, bool later) {
     if (e == hipErrorInvalidValue)
       return set_err(c, PCSF_EINVAL, "FP64 kernel: tree workspace exceeds 64 KiB of LDS");
   } else if (frag_format(precision) >= 0) {
-    e = launch_prune_mfma(m, b, precision, m->mfma_variant[precision], c->stream);
+    e = launch_prune_mfma(m, b, precision, launch_shape(m, precision), c->stream);
   } else {
     return set_err(c, PCSF_EINVAL, "pcsf_forward: unknown precision");
   }
@@ -1533,7 +1537,7 @@ int pcsf_forward_noalloc(pcsf_model* m, const uint8_t* d_codes, int64_t n_cols,
     if (e == hipErrorInvalidValue)
       return set_err(c, PCSF_EINVAL, "FP64 kernel: tree workspace exceeds 64 KiB of LDS");
   } else {
-    e = launch_prune_mfma(m, &v, precision, m->mfma_variant[precision], c->stream);
+    e = launch_prune_mfma(m, &v, precision, launch_shape(m, precision), c->stream);
   }
   HIP_TRY(c, e);
   HIP_TRY(c, launch_region_reduce(&v, c->stream));
@@ -1558,7 +1562,7 @@ int pcsf_autotune(pcsf_batch* b, int precision, int reps, double* ms_out, int* c
   HIP_TRY(c, hipEventCreate(&e0));
   HIP_TRY(c, hipEventCreate(&e1));
   double best = 1e300;
-  int best_v = m->mfma_variant[precision];
+  int best_v = launch_shape(m, precision);
   hipError_t err = hipSuccess;
   for (int v = 0; v < kNumMfmaVariants && err == hipSuccess; ++v) {
     err = launch_prune_mfma(m, b, precision, v, c->stream);  // warm-up

@@ -117,8 +117,9 @@ struct pcsf_model {
   int32_t* d_cherries = nullptr;  // node, left leaf, right leaf per table
   int slots = 0;
   int n_gemm = 0;
-  int mfma_variant[5] = {1, 1, 1, 1, 1};  // launch shape per precision (pcsf_autotune;
-                                          // 2 for trees with generated programs)
+  // launch shape per precision that pcsf_autotune or pcsf_set_variant chose (-1:
+  // the default)
+  int mfma_variant[5] = {-1, -1, -1, -1, -1};
   // tree-specialised programs matching prog / prog_t (nullptr: none), and
   // whether launches may use them
   const void* tree_p = nullptr;

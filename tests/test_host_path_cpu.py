@@ -328,3 +328,27 @@ def test_results_larger_than_the_ring(on_fake):
     got = b.forward(np.full((70000, 2), 1.5), P.PCSF_FP64M, per_region=True)[0]
     assert launches("region_reduce_aligned") == 1 and np.allclose(got, want)
     """, env={"PHYLOCSF_SET_BUDGET_MB": "30000"})
+
+
+def test_interpreter_keeps_its_launch_shape(on_fake):
+    """FP32 on a shipped tree loads leaf rows ahead in the tree's own program; where that is
+    forbidden the interpreter runs without (<..., waves, per SIMD, ahead, ...>), unless a
+    shape was chosen."""
+    on_fake("""
+    ctx = P.Context(0)
+    m = P.PhyloCSFModel.from_paramset(ctx, "58mammals")
+    b = batch(m, 2, 70)
+    ahead, plain = "Li4ELi3ELb1E", "Li4ELi3ELb0E"
+
+    def shapes():
+        fake.fake_reset()
+        b.forward(1.0, P.PCSF_FP32)
+        b.forward(np.full((2, 2), 1.5), P.PCSF_FP32, per_region=True)
+        return launches(ahead), launches(plain)
+
+    assert shapes() == (2, 0)
+    m.specialized(False)
+    assert shapes() == (0, 2) and launches("Interp") == 2
+    m.set_variant(5, P.PCSF_FP32)
+    assert shapes() == (2, 0) and launches("Interp") == 2
+    """)
