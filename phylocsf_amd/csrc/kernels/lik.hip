@@ -126,7 +126,8 @@ __global__ __launch_bounds__(64) void lik_columns_kernel(
 // of leaf states are staged in LDS (ldsl; trees over 256 leaves read them from
 // memory); internal nodes' alpha lie in ws as [node][state][lane].  Bound by
 // those (66,000 columns of 58 leaves at k = 4: 85 us, 2.3 ms with a column per
-// wave).  With no leaf_dist a state below -1 sets *bad.
+// wave) and, from k = 17 on, where P's rows no longer fit the scalar registers, by
+// their reloads (calls of 66,000 columns at k = 20 3.0 ms, 14.8 with a column per wave).  With no leaf_dist a state below -1 sets *bad.
 template <int K>
 __global__ __launch_bounds__(64) void lik_small_kernel(
     int k, int n, const int32_t* __restrict__ lc, const int32_t* __restrict__ rc,
